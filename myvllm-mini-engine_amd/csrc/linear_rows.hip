@@ -6,15 +6,19 @@
 // attention output projection) that GEMM reads the 8 MB weight at a small
 // fraction of HBM bandwidth, because a library tile sized for large M leaves
 // most CUs idle.  Here the weight is the only large operand and is read
-// once.  Two kernels:
+// once.  Three kernels:
+// * streaming (K = 512, 1024, 1536 or 2048, more than 2048 features: the
+//   fused QKV projection, the vocabulary head): persistent work-groups that
+//   keep x in registers and stream 16-feature tiles of weight;
 // * staged (K a multiple of 512, N of 8, operands within 160 KB of LDS --
-//   the decode batch): one work-group per 8 output features, x and the
-//   weight slab copied global->LDS in whole 1 KiB segments;
+//   the decode batch's output projection): one work-group per 8 output
+//   features, x and the weight slab copied global->LDS in whole 1 KiB
+//   segments;
 // * register (any other shape): one work-group per 16 output features, each
 //   lane loading its operands straight into registers.
-// In both, the 16 waves split K, each wave computing D[n, m] = W[n, k-slice]
+// In all, the waves of a work-group split K, each wave computing D[n, m] = W[n, k-slice]
 // x[m, k-slice]^T for every 16-row block of x with v_mfma_f32_16x16x32 (fp32
-// accumulation), then the 16 partial tiles are summed through LDS and
+// accumulation), then their partial tiles are summed through LDS and
 // rounded once to the output type.  Measured over 28 layers' distinct
 // 2048 x 2048 bf16 weights at 32 rows: register kernel 7.8 us per call,
 // staged kernel 5.5 us (x re-read from L2 by every work-group dominated the
@@ -31,7 +35,8 @@ namespace {
 constexpr int kLinWaves = 16;
 constexpr int kLinThreads = kLinWaves * kWave;
 constexpr int kLinMaxRows = 64;
-constexpr int kLinMaxBlocks = kLinMaxRows / 16;
+constexpr int kLinCUs = 256;
+constexpr int kStreamMaxK = 2048;  // 16 waves of 128; x's operands for more would not fit the registers
 
 struct LinearArgs {
     void* out;
@@ -228,6 +233,135 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_staged_kernel(LinearA
     }
 }
 
+// Streaming variant for wide layers (the vocabulary head): persistent
+// work-groups of NW = K/128 waves, 16 waves per CU, each work-group over a
+// contiguous range of 16-feature tiles.  Wave w owns the k-slice [128 w,
+// 128 w + 128) and keeps x's operand for it in registers for the whole call
+// (16*MB VGPRs), so a tile costs its weight rows and nothing else: two tiles
+// of weight loads are in flight per wave (8 KiB, 128 KiB per CU).  The
+// waves' partial tiles meet in LDS, double-buffered, with one barrier per
+// tile, and MB of the waves (others for the next tile) sum and store it.
+// Bound by HBM: 32 rows of 2048 into 151,936 features (622 MB of bf16 weight)
+// 314 us with the staged kernel, whose 160 KB of LDS leave one work-group per
+// CU with nothing in flight while it multiplies, 105.6 us here (5.9 TB/s).
+//
+// A product wants 16 features in 16 consecutive lanes; loaded that way,
+// every quad of lanes touches four rows and the load unit spends a cycle per
+// lane.  Here load j of lane (4*a + p, lg) takes chunk 4*lg + p of feature
+// 4*a + j -- a quad reads 64 consecutive bytes -- and a 4x4 transpose inside
+// the quads (quad_transpose) turns the four loads into four operands: chunk
+// 4*lg + j of feature li.  Same call with operand-order loads 131.9 us.
+constexpr int kStreamSteps = 4;  // 32-wide k-steps per wave
+// Waves per CU: four per SIMD, three where 64 rows' operands and a work-group
+// below 16 waves would otherwise spill.
+template <int MB, int NW>
+constexpr int stream_waves() { return MB == 4 && NW < kLinWaves ? 12 : 16; }
+
+template <typename T, int MB, int NW>
+__global__ __launch_bounds__(NW * kWave, (stream_waves<MB, NW>() / 4)) void linear_rows_stream_kernel(LinearArgs a) {
+    __shared__ f32x4 sm_part[2][NW][MB][kWave];
+    constexpr int KS = kStreamSteps;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int li = lane & 15, lg = lane >> 4;
+    constexpr int K = NW * KS * 32;
+    const int tiles = a.out_features / 16;
+    const int t_begin = (int)((int64_t)blockIdx.x * tiles / gridDim.x);
+    const int t_end = (int)((int64_t)(blockIdx.x + 1) * tiles / gridDim.x);
+    if (t_begin >= t_end) return;
+    const uint16_t* wbase = static_cast<const uint16_t*>(a.weight) + (int64_t)(li & ~3) * K + wave * (KS * 32) +
+                            8 * (4 * lg + (li & 3));
+    auto load = [&](int t, u32x4 (&w)[KS]) __attribute__((always_inline)) {
+        const uint16_t* p = wbase + (int64_t)min(t, t_end - 1) * (16 * K);
+#pragma unroll
+        for (int j = 0; j < KS; ++j) w[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + j * K));
+    };
+    u32x4 wa[KS], wb[KS];
+    load(t_begin, wa);
+    // Rows of x past M read row 0 (in bounds); their products are dropped.
+    u32x4 xop[MB][KS];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        const int r = 16 * mb + li;
+        const uint16_t* xrow = static_cast<const uint16_t*>(a.x) + (int64_t)(r < a.rows ? r : 0) * a.x_stride +
+                               wave * (KS * 32) + 32 * lg;
+#pragma unroll
+        for (int j = 0; j < KS; ++j) xop[mb][j] = *reinterpret_cast<const u32x4*>(xrow + 8 * j);
+    }
+    load(t_begin + 1, wb);
+    auto tile = [&](int t, u32x4 (&w)[KS], int buf) __attribute__((always_inline)) {
+        f32x4 acc[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        quad_transpose(w);
+#pragma unroll
+        for (int j = 0; j < KS; ++j)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) acc[mb] = T::mfma16x16x32(w[j], xop[mb][j], acc[mb]);
+        load(t + 2, w);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) sm_part[buf][wave][mb][lane] = acc[mb];
+        // One barrier per tile: it publishes this tile's partials, and the
+        // sums of the tile before the last (this buffer's previous use) were
+        // read before their waves came to the previous barrier.
+        __syncthreads();
+        // Wave w sums row block mb when w = (t - t_begin) * MB + mb (mod NW).
+        const int first = (t - t_begin) * MB % NW;
+        const int mb = wave >= first ? wave - first : wave - first + NW;
+        if (mb >= MB) return;
+        f32x4 p[NW];
+#pragma unroll
+        for (int v = 0; v < NW; ++v) p[v] = sm_part[buf][v][mb][lane];
+#pragma unroll
+        for (int n = NW; n > 1; n = (n + 1) / 2)
+#pragma unroll
+            for (int v = 0; v < n / 2; ++v) p[v] += p[v + (n + 1) / 2];
+        const int row = 16 * mb + li;
+        if (row >= a.rows) return;
+        const int nb = 16 * t + 4 * lg;
+        float v[4] = {p[0][0], p[0][1], p[0][2], p[0][3]};
+        if (a.bias) {
+            const uint16_t* bias = static_cast<const uint16_t*>(a.bias) + nb;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] += T::lo((uint32_t)bias[i]);
+        }
+        const u32x2 packed = {T::pack(v[0], v[1]), T::pack(v[2], v[3])};
+        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (int64_t)row * a.out_features + nb) = packed;
+    };
+    // Pairs without a branch between the two tiles: with one, the compiler's
+    // wait for the first tile's weights also covers the second's.
+    int t = t_begin;
+    for (; t + 1 < t_end; t += 2) {
+        tile(t, wa, 0);
+        tile(t + 1, wb, 1);
+    }
+    if (t < t_end) tile(t, wa, 0);
+}
+
+template <typename T, int MB, int NW>
+void launch_stream(const LinearArgs& a, hipStream_t s) {
+    const int groups = min(a.out_features / 16, kLinCUs * (stream_waves<MB, NW>() / NW));
+    hipLaunchKernelGGL((linear_rows_stream_kernel<T, MB, NW>), dim3(groups), dim3(NW * kWave), 0, s, a);
+}
+
+template <typename T, int MB>
+void launch_stream_nw(const LinearArgs& a, hipStream_t s) {
+    switch (a.in_features / (32 * kStreamSteps)) {
+        case 4: launch_stream<T, MB, 4>(a, s); break;
+        case 8: launch_stream<T, MB, 8>(a, s); break;
+        case 12: launch_stream<T, MB, 12>(a, s); break;
+        default: launch_stream<T, MB, 16>(a, s); break;
+    }
+}
+
+template <typename T>
+void launch_linear_stream(const LinearArgs& a, int mb, hipStream_t s) {
+    if (mb == 1) launch_stream_nw<T, 1>(a, s);
+    else if (mb == 2) launch_stream_nw<T, 2>(a, s);
+    else if (mb == 3) launch_stream_nw<T, 3>(a, s);
+    else launch_stream_nw<T, 4>(a, s);
+}
+
 template <typename T, int MB>
 int launch_staged(const LinearArgs& a, hipStream_t s) {
     const size_t lds = staged_lds_bytes(MB, a.in_features);
@@ -294,6 +428,17 @@ extern "C" int mvme_linear_rows(void* out, const void* x, const void* weight, co
     a.x_stride = x_row_stride;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int mb = (int)((rows + 15) / 16);
+    // More features than one round of staged work-groups (8 each, one per CU)
+    // stream; at most that many fit the chip at once and start faster staged
+    // (no prologue that loads x into registers).  us per call, staged against
+    // streaming, K = 2048: N = 2048 4.3 / 5.3 at 16 rows, 5.7 / 6.9 at 32;
+    // N = 4096 8.3 / 6.3, 10.6 / 7.7, 13.2 / 11.9 at 64; N = 8192 14.3 / 11.0;
+    // K = 1024, N = 4096 4.4 / 4.2.
+    if (in_features % 512 == 0 && in_features <= kStreamMaxK && out_features > kLinCUs * kStagedFeat) {
+        if (dtype == MVME_FP16) launch_linear_stream<Half>(a, mb, s);
+        else launch_linear_stream<BFloat16>(a, mb, s);
+        return check_launch("linear rows");
+    }
     if (in_features % 512 == 0 && out_features % kStagedFeat == 0 &&
         staged_lds_bytes(mb, in_features) <= kStagedMaxLds) {
         const int rc = dtype == MVME_FP16 ? launch_linear_staged<Half>(a, mb, s) : launch_linear_staged<BFloat16>(a, mb, s);

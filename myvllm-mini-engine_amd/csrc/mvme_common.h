@@ -93,6 +93,38 @@ __device__ inline float shfl_xor(float v, int mask) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, __float_as_int(v)));
 }
 
+template <int CTRL>
+__device__ inline uint32_t quad_swap(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+}
+
+// 4x4 transpose between the register index and the lane inside each quad:
+// afterwards lane p holds in r[j] what lane j held in r[p].  Loads whose
+// quads read 64 consecutive bytes of one row become MFMA operands, whose
+// consecutive lanes are different rows.
+__device__ inline void quad_transpose(u32x4 (&r)[4]) {
+    const int lane = __lane_id();
+    const bool odd = lane & 1, high = lane & 2;
+    // (The exchanges stay outside the selects: they read every lane.)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+            const uint32_t x = r[j][d], y = r[j + 1][d];
+            const uint32_t sx = quad_swap<kDppQuadSwap1>(x), sy = quad_swap<kDppQuadSwap1>(y);
+            r[j][d] = odd ? sy : x;
+            r[j + 1][d] = odd ? y : sx;
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t x = r[j][d], y = r[j + 2][d];
+            const uint32_t sx = quad_swap<kDppQuadSwap2>(x), sy = quad_swap<kDppQuadSwap2>(y);
+            r[j][d] = high ? sy : x;
+            r[j + 2][d] = high ? y : sx;
+        }
+    }
+}
+
 // Sum over aligned groups of N consecutive lanes; every lane of a group
 // receives the group total.  N <= 16 stays inside one DPP row.
 template <int N>

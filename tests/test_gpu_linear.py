@@ -38,6 +38,18 @@ def test_linear_rows_matches_fp32_product(dtype, rows, k, n, bias):
     assert (actual == exact.to(dtype)).float().mean().item() >= 0.99
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,k,n,bias", [
+    (1, 512, 2064, False), (16, 1024, 4112, True), (17, 1536, 4096, False), (33, 2048, 2064, False),
+    (48, 1024, 8208, False), (64, 2048, 4112, True), (64, 512, 12304, False), (5, 2048, 20496, False),
+])
+def test_linear_rows_wide_layers(dtype, rows, k, n, bias):
+    """Layers of more than 2048 features (persistent work-groups over ranges
+    of 16-feature tiles): 4 to 16 waves, 1 to 4 row blocks, one tile per
+    work-group or a remainder over several."""
+    test_linear_rows_matches_fp32_product(dtype, rows, k, n, bias)
+
+
 def test_linear_rows_strided_input_rows():
     """x as a row slice of a wider buffer (row stride > in_features)."""
     gen = torch.Generator().manual_seed(3)
