@@ -80,7 +80,10 @@ struct BFloat16 {
 // DPP controls (gfx9 encoding): quad permutations and 16-lane row mirrors.
 constexpr int kDppQuadSwap1 = 0xB1;     // quad_perm [1,0,3,2]
 constexpr int kDppQuadSwap2 = 0x4E;     // quad_perm [2,3,0,1]
+constexpr int kDppQuadReverse = 0x1B;   // quad_perm [3,2,1,0]
 constexpr int kDppRowHalfMirror = 0x141; // lane i <- lane 7-i within 8
+constexpr int kDppRowRor4 = 0x124;       // lane i <- lane (i + 12) mod 16 within 16
+constexpr int kDppRowRor8 = 0x128;       // lane i <- lane i ^ 8 within 16
 constexpr int kDppRowMirror = 0x140;     // lane i <- lane 15-i within 16
 
 template <int CTRL>
@@ -136,6 +139,39 @@ __device__ inline float group_sum(float v) {
     if constexpr (N >= 32) v += shfl_xor(v, 16);
     if constexpr (N >= 64) v += shfl_xor(v, 32);
     return v;
+}
+
+// Max / sum over the four lanes {l, l^16, l^32, l^48} (the 4 MFMA k-groups
+// of one row or column) with gfx950 lane swaps -- no LDS round trip.
+__device__ inline float row4_max(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ inline float row4_sum(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// Max over the two lanes {l, l^32}.
+__device__ inline float pair32_max(float x) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+
+// One exchange of a reduction that halves what each lane holds: lanes 0..31
+// receive x + x(lane + 32), lanes 32..63 y + y(lane - 32).
+__device__ inline float swap32_add(float x, float y) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+// The same between the even and the odd row of each pair of 16-lane rows.
+__device__ inline float swap16_add(float x, float y) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
 }
 
 // Inclusive prefix sum over the 64 lanes of a wave, all in DPP (no LDS

@@ -23,6 +23,46 @@ constexpr int kMergeWindow = 2048;  // partition weights held in LDS at once
 template <int D>
 constexpr int merge_threads() { return (D + kWave - 1) / kWave * kWave; }
 
+// Merge of at most N partitions: every thread loads its dim's partials and all
+// (max, sum) pairs at once, without knowing yet how many partitions the
+// sequence has (rows past them hold nothing and are dropped), so the launch
+// is one memory round trip and no barrier (8 sequences of 512, bf16: the two
+// launches 9.4 -> 9.0 us, together with the attention kernel's early page
+// lookup).
+template <typename T, int D, int N>
+__device__ inline void merge_direct(const DecodeArgs& a, int64_t bh, int b) {
+    const int tid = threadIdx.x;
+    if (tid >= D) return;
+    const float* ml = a.ws_ml + bh * a.max_parts * 2;
+    const float* acc = a.ws_acc + bh * a.max_parts * D + tid;
+    float m[N], l[N], v[N];
+#pragma unroll
+    for (int p = 0; p < N; ++p) {
+        const int row = min(p, a.max_parts - 1);
+        m[p] = ml[2 * row];
+        l[p] = ml[2 * row + 1];
+        v[p] = acc[(int64_t)row * D];
+    }
+    const int len = seq_tokens(a.lens[b], a.capacity);
+    const int nparts = len > 0 ? (len + a.partition - 1) / a.partition : 1;
+    if (nparts == 1) return;  // written directly by the attention kernel
+    float mx = kNegInf;
+#pragma unroll
+    for (int p = 0; p < N; ++p) {
+        if (p >= nparts) m[p] = kNegInf;
+        mx = fmaxf(mx, m[p]);
+    }
+    const float ref = mx == kNegInf ? 0.f : mx;
+    float o = 0.f, sum = 0.f;
+#pragma unroll
+    for (int p = 0; p < N; ++p) {
+        const float w = fast_exp2(m[p] - ref);
+        sum += p < nparts ? l[p] * w : 0.f;
+        o += p < nparts ? v[p] * w : 0.f;
+    }
+    static_cast<uint16_t*>(a.out)[bh * D + tid] = T::from_float(sum > 0.f ? o / sum : 0.f);
+}
+
 template <typename T, int D>
 __global__ __launch_bounds__(256) void paged_decode_merge_kernel(DecodeArgs a) {
     static_assert(D <= 256, "one thread per output dim");
@@ -31,6 +71,18 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(DecodeArgs a) {
     __shared__ float sm_w[kMergeWindow];
     const int64_t bh = blockIdx.x;
     const int b = (int)(bh / a.q_heads);
+    if (a.max_parts <= 4) {
+        merge_direct<T, D, 4>(a, bh, b);
+        return;
+    }
+    if (a.max_parts <= 8) {
+        merge_direct<T, D, 8>(a, bh, b);
+        return;
+    }
+    if (a.max_parts <= 16) {
+        merge_direct<T, D, 16>(a, bh, b);
+        return;
+    }
     const int len = seq_tokens(a.lens[b], a.capacity);
     const int nparts = len > 0 ? (len + a.partition - 1) / a.partition : 1;
     if (nparts == 1) return;  // written directly by the attention kernel
@@ -120,7 +172,9 @@ __global__ __launch_bounds__(kLptMax) void paged_decode_flat_merge_kernel(Decode
     const int64_t p0 = dsc.p0;
     const int n = (int)(l - p0 + 1);
     const int kvh = dsc.r / a.gtiles;
-    const int h0 = kvh * a.group + (dsc.r - kvh * a.gtiles) * G;
+    const int tile0 = (dsc.r - kvh * a.gtiles) * a.tile_heads;
+    const int h0 = kvh * a.group + tile0;
+    const int heads = matrix_tile<D, G>() ? min(a.tile_heads, a.group - tile0) : G;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int64_t p = p0 + tid;
     const bool live = tid < n && flat_share_start(p, total) < flat_share_start(p + 1, total);
@@ -128,8 +182,8 @@ __global__ __launch_bounds__(kLptMax) void paged_decode_flat_merge_kernel(Decode
     float m[G], lsum[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-        m[g] = live ? a.ws_ml[(row + g) * 2] : kNegInf;
-        lsum[g] = live ? a.ws_ml[(row + g) * 2 + 1] : 0.f;
+        m[g] = live && g < heads ? a.ws_ml[(row + g) * 2] : kNegInf;
+        lsum[g] = live && g < heads ? a.ws_ml[(row + g) * 2 + 1] : 0.f;
         float v = m[g];
 #pragma unroll
         for (int off = kWave / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
@@ -152,40 +206,72 @@ __global__ __launch_bounds__(kLptMax) void paged_decode_flat_merge_kernel(Decode
         }
     }
     __syncthreads();
-    constexpr int kBatch = 16;
-    for (int idx = tid; idx < G * D; idx += kLptMax) {
-        const int g = idx / D;
-        const int d = idx - g * D;
-        float sum = 0.f, o = 0.f;
-        for (int t0 = 0; t0 < n; t0 += kBatch) {
-            float av[kBatch];
+    // Four output dims per thread; when that leaves threads over, kGroups of
+    // them share the pieces and meet in LDS.
+    constexpr int kVecs = G * D / 4;
+    constexpr int kGroups = kLptMax / kVecs;
+    static_assert(kGroups >= 1, "one thread per four output dims");
+    constexpr int kBatch = 8;
+    const int grp = tid / kVecs, idx = tid - grp * kVecs;
+    const int g = idx / (D / 4), d = 4 * (idx - g * (D / 4));
+    const bool active = grp < kGroups && g < heads;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    float sum = 0.f;
+    if (active) {
+        for (int t0 = grp; t0 < n; t0 += kBatch * kGroups) {
+            f32x4 av[kBatch];
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k)
+                av[k] = *reinterpret_cast<const f32x4*>(a.ws_acc + (sm_row[min(t0 + k * kGroups, n - 1)] + g) * D + d);
 #pragma unroll
             for (int k = 0; k < kBatch; ++k) {
-                av[k] = a.ws_acc[(sm_row[min(t0 + k, n - 1)] + g) * D + d];
-            }
-#pragma unroll
-            for (int k = 0; k < kBatch; ++k) {
-                const int t = min(t0 + k, n - 1);
-                const bool use = t0 + k < n && sm_w[g][t] != 0.f;
+                const int t = min(t0 + k * kGroups, n - 1);
+                const bool use = t0 + k * kGroups < n && sm_w[g][t] != 0.f;
+                const float w = use ? sm_w[g][t] : 0.f;
                 sum += use ? sm_lw[g][t] : 0.f;
-                o += use ? av[k] * sm_w[g][t] : 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] += use ? av[k][i] * w : 0.f;
             }
         }
-        static_cast<uint16_t*>(a.out)[((int64_t)dsc.b * a.q_heads + h0 + g) * D + d] =
-            T::from_float(sum > 0.f ? o / sum : 0.f);
     }
+    if constexpr (kGroups > 1) {
+        __shared__ f32x4 sm_o[kGroups * kVecs];
+        __shared__ float sm_sum[kGroups * kVecs];
+        if (grp < kGroups) {
+            sm_o[tid] = o;
+            sm_sum[tid] = sum;
+        }
+        __syncthreads();
+        if (grp > 0 || !active) return;
+        for (int q = 1; q < kGroups; ++q) {
+            o += sm_o[q * kVecs + idx];
+            sum += sm_sum[q * kVecs + idx];
+        }
+    } else if (!active) {
+        return;
+    }
+    uint16_t* out = static_cast<uint16_t*>(a.out) + ((int64_t)dsc.b * a.q_heads + h0 + g) * D + d;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = T::from_float(sum > 0.f ? o[i] / sum : 0.f);
 }
 
 struct DecodePlan {
     int partition;
     int max_parts;
     int gtile;  // G of the kernel instance
+    int gtiles; // query-head tiles per kv head
+    int tile_heads; // query heads per tile (at most gtile)
     int waves;  // waves per work-group (kSplitWaves or kWholeWaves; kFlatWaves in the walk)
     bool stream;  // non-temporal K/V loads
     int flat_groups;  // > 0: balanced walk with this many work-groups
 };
 
 
+// Query heads per kv head from which tiles run on the matrix cores.  A tile of
+// up to 4 heads costs them the same whatever the number; with 2 heads the
+// dot-product kernel is ahead (32 sequences of 2048, fp16: 44.6 us against
+// 46.3), with 4 the matrix cores are (48.4 -> 46.3).
+constexpr int64_t kMatrixGroup = 3;
 constexpr int64_t kStreamBytes = int64_t(64) << 20;  // K+V bytes within capacity above which loads stream
 
 int decode_tile_tokens(int64_t head_dim) {
@@ -203,6 +289,24 @@ int decode_tile_tokens(int64_t head_dim) {
 }
 
 constexpr int64_t kDeviceCUs = 256;  // MI355X compute units
+
+// Query-head tiles of a group: on the matrix cores the fewest tiles of at
+// most 8 heads, of equal size (a tile reads all K/V rows of its kv head, so
+// one tile of 7 beats seven of 1, and 9 heads are 5 + 4); otherwise tiles that
+// divide the group.
+void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim) {
+    if ((head_dim == 64 || head_dim == 128) && group >= kMatrixGroup) {
+        const int64_t tiles = (group + 7) / 8;
+        const int64_t heads = (group + tiles - 1) / tiles;
+        p.gtiles = (int)((group + heads - 1) / heads);
+        p.tile_heads = (int)heads;
+        p.gtile = heads <= 4 ? 4 : 8;
+        return;
+    }
+    p.gtile = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+    p.gtiles = (int)(group / p.gtile);
+    p.tile_heads = p.gtile;
+}
 
 // Host-side plan (lengths stay on the device, so it depends on the table
 // capacity only).  Long units (kLongUnitBytes of K+V capacity) numbering at
@@ -233,10 +337,10 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
                             int64_t block_size, int64_t table_width, int64_t requested) {
     DecodePlan p{};
     const int64_t group = q_heads / kv_heads;
-    p.gtile = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+    plan_tiles(p, group, head_dim);
     const int64_t tile = decode_tile_tokens(head_dim);
     const int64_t cap = table_width * block_size;
-    const int64_t units = batch * kv_heads * (group / p.gtile);
+    const int64_t units = batch * kv_heads * p.gtiles;
     const int64_t split_step = tile * kSplitWaves;
     const int64_t whole_step = tile * 16;  // the capacity unit the thresholds below were measured in
     int64_t part;
@@ -324,12 +428,18 @@ void launch_decode(const DecodeArgs& a, const DecodePlan& p, int units, bool pag
     if (a.flat_groups > 0)
         hipLaunchKernelGGL((paged_decode_flat_merge_kernel<T, D, G>), dim3(a.flat_groups), dim3(kLptMax), 0, s, a);
     else if (a.max_parts > 1)
-        hipLaunchKernelGGL((paged_decode_merge_kernel<T, D>), dim3(units / a.kv_heads / a.gtiles * a.q_heads),
+        hipLaunchKernelGGL((paged_decode_merge_kernel<T, D>), dim3(a.batch * a.q_heads),
                            dim3(merge_threads<D>()), 0, s, a);
 }
 
 template <typename T, int D>
 void launch_decode_g(const DecodeArgs& a, const DecodePlan& p, int units, bool page_uniform, hipStream_t s) {
+    if constexpr (max_gtile<D>() >= 8) {
+        if (p.gtile == 8) {
+            launch_decode<T, D, 8>(a, p, units, page_uniform, s);
+            return;
+        }
+    }
     if (p.gtile == 4) launch_decode<T, D, 4>(a, p, units, page_uniform, s);
     else if (p.gtile == 2) launch_decode<T, D, 2>(a, p, units, page_uniform, s);
     else launch_decode<T, D, 1>(a, p, units, page_uniform, s);
@@ -421,7 +531,7 @@ int launch_paged_attention(void* out, const void* query, const void* key_cache, 
     const DecodePlan p = make_decode_plan(batch, q_heads, kv_heads, head_dim, block_size, table_width,
                                           partition_tokens);
     const int64_t group = q_heads / kv_heads;
-    const int64_t units = batch * kv_heads * (group / p.gtile);
+    const int64_t units = batch * kv_heads * p.gtiles;
     if (units > 2147483647) return fail(MVME_EINVAL, "batch/head product too large");
     DecodeArgs a{};
     a.out = out;
@@ -445,7 +555,8 @@ int launch_paged_attention(void* out, const void* query, const void* key_cache, 
     a.q_heads = (int)q_heads;
     a.kv_heads = (int)kv_heads;
     a.group = (int)group;
-    a.gtiles = (int)(group / p.gtile);
+    a.gtiles = p.gtiles;
+    a.tile_heads = p.tile_heads;
     a.num_blocks = num_blocks;
     a.block_size = (int)block_size;
     a.block_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctzll((unsigned long long)block_size) : -1;

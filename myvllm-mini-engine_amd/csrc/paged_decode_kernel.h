@@ -29,6 +29,9 @@
 // that later reads that position (in every work-group whose token range
 // holds it: identical bytes from each G-tile), so no barrier is needed.
 //
+// Query groups of three or more heads at head_dim 64 and 128 run on the
+// matrix cores (see matrix_states); what follows describes the others.
+//
 // Scores: packed dot2 (fp16/bf16 products, fp32 accumulation) on the lane's
 // 8 elements, then a DPP reduction across the LPT lanes of the token.
 // Softmax: online, fp32, base-2 exponent with log2(e)/sqrt(D) folded into
@@ -68,7 +71,20 @@ struct DecodeShape {
                               : kChunks <= 8 ? 8 : kChunks <= 16 ? 16 : kChunks <= 32 ? 32 : 64;
     static constexpr int kTpl = kWave / kLpt;          // tokens per load
     static constexpr int kTpi = kTpl * kDecodeLoads;   // tokens per wave iteration
+    // Matrix-core path (see paged_decode_kernel): a score product covers the
+    // kTpl tokens of one load in 16 / kTpl parts of D * kTpl / 16 dims.
+    static constexpr bool kMatrix = D == 64 || D == 128;
+    static constexpr int kParts = 16 / kTpl;
+    static constexpr int kCols = 16 / kParts;  // query heads per score product
 };
+
+// Largest query-head tile: 8 heads where the matrix-core path serves the
+// head dim, else 4.
+template <int D>
+constexpr int max_gtile() { return DecodeShape<D>::kMatrix ? 8 : 4; }
+// The tile sizes computed on the matrix cores (the others use dot products).
+template <int D, int G>
+constexpr bool matrix_tile() { return DecodeShape<D>::kMatrix && G >= 4; }
 
 // Balanced walk: the merge duty of share l, written by the attention
 // kernel's work-group for that share on every call and read by the merge
@@ -96,7 +112,8 @@ struct DecodeArgs {
     int q_heads;
     int kv_heads;
     int group;      // q_heads / kv_heads
-    int gtiles;     // group / G
+    int gtiles;     // query-head tiles per kv head: ceil(group / tile_heads)
+    int tile_heads; // query heads per tile, at most G (a group's last tile may hold fewer)
     int64_t num_blocks;
     int block_size;
     int block_shift;  // log2(block_size) when it is a power of two, else -1
@@ -210,19 +227,60 @@ static_assert(kFlatGroups <= kLptMax, "one merge thread per piece");
 // First chunk of logical work-group l's share.
 __device__ inline int64_t flat_share_start(int64_t l, int64_t total) { return (l * total) >> kFlatShift; }
 
+constexpr float kRaise = 8.f;  // binary orders a score may exceed the running reference by (matrix tiles)
+
+// Value of lane i ^ 4 (the half-row mirror, then each quad reversed).
+__device__ inline float lane_xor4(float v) { return dpp<kDppQuadReverse>(dpp<kDppRowHalfMirror>(v)); }
+
+// Matrix-core tiles (D = 64 or 128, tiles of up to 4 or 8 query heads, G).
+// With dot products every head of a tile costs each K load 4 dot2 and a
+// cross-lane sum, and each V load 8 FMAs, so from about 4 heads on the vector
+// ALU, not memory, bounds the loop.  Here:
+// * Scores: one 16x16x32 product per K load of kTpl tokens.  K stays in the
+//   layout of a coalesced load: product row li = kParts * token + part holds
+//   the dims of chunks kParts * lg + part, and column kCols * part' + head
+//   the query's dims of chunks kParts * lg + part'.  Only the entries with
+//   part == part' are partial scores; adding a token's parts (DPP) gives the
+//   lane its V token's score for head li mod kCols.  (16 tokens as 16 rows
+//   would need no sum, but consecutive lanes then load 16 bytes of different
+//   rows, a cycle each in the load unit.)
+// * Output: v_mfma_f32_4x4x1 with fp32 operands, 16 blocks of 4 lanes: a lane
+//   supplies one V element (converted exactly) and the fp32 probability of
+//   head (lane mod 4) for its token, and receives that head's sums over the
+//   four chunks of its block.  Probabilities stay fp32.
+// At D = 128 a tile of 8 heads takes two score products per load (state t:
+// head 4 t + li mod 4); at D = 64 one product has 8 head columns, a lane's
+// state belongs to head li mod G and the second set of sums to head
+// (li mod 8) ^ 4, whose probabilities lane li ^ 4 holds.
+// Measured against tiles of 1, 2 or 4 heads on dot products (us per call):
+// 28/4 heads, 24 sequences U[1,4096] 121.5 -> 29.6 (seven 1-head tiles read
+// every row seven times); 32/4 heads, 16 of U[1,8192] 64.3 -> 40.6; 32/8
+// heads, 32 of 2048 48.4 -> 46.3, 8 of U[1,1024] 13.9 -> 10.3; 14/2 heads of
+// 64, 96 of U[1,1300] 39.8 -> 26.9.  With operand-order K loads the first two
+// were 39.2 and 51.3.
+template <int D, int G>
+constexpr int matrix_states() { return D == 128 ? G / 4 : 1; }
+
+// Waves per SIMD the register allocation has to leave room for (the walk runs
+// one work-group of 8 waves per CU).
+template <int D, int G, bool FLAT>
+constexpr int min_waves() { return !matrix_tile<D, G>() ? 1 : G == 4 && !FLAT ? 4 : 2; }
+
 // PRO: the kernel runs the fused prologue (a.prologue 1 or 2); without it
 // the prologue's code is not compiled in.  FLAT: the balanced walk (its
 // segment loop would cost the other modes about 20 VGPRs).
 template <typename T, int D, int G, bool PAGE_UNIFORM, int NW, bool STREAM, bool PRO, bool FLAT>
-__global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_decode_kernel(DecodeArgs a) {
     using S = DecodeShape<D>;
     constexpr int L = kDecodeLoads;
     constexpr int kStep = S::kTpi * NW;  // tokens per work-group iteration
+    constexpr bool MM = matrix_tile<D, G>();
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int tl = lane / S::kLpt;  // token slot inside one load
     const int c = lane % S::kLpt;   // 16-byte chunk of the token row
     const bool chunk_ok = c < S::kChunks;
+    const int li = lane & 15, lg = lane >> 4;  // matrix operand column / row and k-group
 
     const int unit = blockIdx.x;
     const int part = blockIdx.y;
@@ -236,6 +294,17 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
     __shared__ int fl_len[kLptMax];
     __shared__ int fl_pref[kLptMax + 1];
     __shared__ int fl_tot[kLptMax / kWave];
+    // First page of this wave's tokens when the segment's start does not depend
+    // on the lengths: looked up beside the length, not after it (entries past
+    // the context are read but not used).
+    typedef __attribute__((address_space(4))) const int64_t const_i64;
+    int64_t first_page = -1;
+    auto early_page = [&](int seq) __attribute__((always_inline)) {
+        const int t = __builtin_amdgcn_readfirstlane(part * a.partition + wave * S::kTpi);
+        if (PAGE_UNIFORM && t < a.capacity)
+            first_page = ((const const_i64*)(a.tables + (int64_t)seq * a.table_width))[a.block_shift >= 0 ? t >> a.block_shift
+                                                                                                     : t / a.block_size];
+    };
     int64_t fl_wc = 0, fl_pos = 0, fl_stop = 0, fl_row = 0, fl_row_later = 0;
     if constexpr (FLAT) {
         flat_prefix(a, S::kTpi, fl_len, fl_pref, fl_tot);
@@ -332,6 +401,7 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
             }
             len = __builtin_amdgcn_readlane(key, b) >> 6;
         } else {
+            early_page(b);
             len = seq_tokens(a.lens[b], a.capacity);
         }
         const int nparts = len > 0 ? (len + a.partition - 1) / a.partition : 1;
@@ -352,7 +422,10 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
             direct = fl_pos == first && last <= fl_stop;
         }
         const int kvh = r / a.gtiles;
-        const int h0 = kvh * a.group + (r - kvh * a.gtiles) * G;
+        const int tile0 = (r - kvh * a.gtiles) * a.tile_heads;  // first head of the tile inside the group
+        const int h0 = kvh * a.group + tile0;
+        // Heads of this tile.  Without matrix cores tiles are always full.
+        const int heads = MM ? min(a.tile_heads, a.group - tile0) : G;
 
         static_assert(!PRO || (S::kLpt == S::kChunks && S::kLpt >= 2), "prologue needs head_dim 16/32/64/128/256");
         // Fused prologue, with no barrier: the wave whose iterations hold the new
@@ -384,13 +457,13 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
                     *reinterpret_cast<u32x4*>(vdst) = vx;
                 }
             } else {
-                // Rows 0 .. G-1: the tile's query heads; row G (owner only): the new K.
+                // Rows 0 .. heads-1: the tile's query heads; row `heads` (owner only): the new K.
                 constexpr int kRowsPerWave = kWave / S::kLpt;
-                const int rows = G + (slot >= 0 ? 1 : 0);
+                const int rows = heads + (slot >= 0 ? 1 : 0);
                 for (int r0 = 0; r0 < rows; r0 += kRowsPerWave) {
                     const int row = r0 + tl;
                     const bool live = row < rows;
-                    const bool is_k = row == G;
+                    const bool is_k = row == heads;
                     // Lanes past the list compute on zeros and store nothing (the
                     // sum of squares and the rotation exchange read every lane).
                     const uint16_t* src = is_k ? kv_src
@@ -418,8 +491,26 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
             }
         }
 
-        // Query slice of this lane for every head of the tile (8 elements each).
-        uint32_t q[G][4];
+        // Query operands.  Matrix tiles: column li of the score product.
+        // Otherwise: this lane's 8 elements of every head of the tile.
+        constexpr int kStates = MM ? matrix_states<D, G>() : G;
+        u32x4 qop[MM ? kStates : 1];
+        uint32_t q[MM ? 1 : G][4];
+        if constexpr (MM) {
+#pragma unroll
+            for (int t = 0; t < kStates; ++t) {
+                const int head = (li % S::kCols) % G + 4 * t;
+                const int d = 8 * (S::kParts * lg + li / S::kCols);
+                u32x4 w = {0u, 0u, 0u, 0u};
+                if (PRO && a.prologue == 2) {
+                    if (head < heads) w = *reinterpret_cast<const u32x4*>(&sm_q[PRO ? wave : 0][PRO ? head : 0][PRO ? d : 0]);
+                } else if (head < heads) {
+                    w = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.query) +
+                                                        ((int64_t)b * a.q_heads + h0 + head) * D + d);
+                }
+                qop[t] = w;
+            }
+        } else {
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             u32x4 w = {0u, 0u, 0u, 0u};
@@ -431,14 +522,26 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
 #pragma unroll
             for (int i = 0; i < 4; ++i) q[g][i] = w[i];
         }
+        }
 
-        float m[G], l[G], acc[G][8];
+        // Running softmax state.  Matrix tiles: macc[t][e][i] is the sum of
+        // the head of sums t for dim 8 * (4 * (c / 4) + i) + e.
+        float m[kStates], l[kStates], acc[MM ? 1 : G][8];
+        f32x4 macc[MM ? G / 4 : 1][8];
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
+        for (int g = 0; g < kStates; ++g) {
             m[g] = kNegInf;
             l[g] = 0.f;
+            if constexpr (!MM) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
+                for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
+            }
+        }
+        if constexpr (MM) {
+#pragma unroll
+            for (int t = 0; t < G / 4; ++t)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) macc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
         const int64_t row_elems = (int64_t)a.kv_heads * D;
@@ -451,19 +554,165 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
         // id is a scalar load issued one iteration ahead (its latency hides
         // behind the current iteration); the loads are a scalar page base plus
         // 32-bit per-lane offsets, with no per-load branches.
-        typedef __attribute__((address_space(4))) const int64_t const_i64;
         const const_i64* ctable = (const const_i64*)table;
         const int row_bytes = (int)(row_elems * 2);
         uint32_t lane_off[L];
 #pragma unroll
         for (int u = 0; u < L; ++u) lane_off[u] = (uint32_t)((u * S::kTpl + tl) * row_bytes + (kvh * D + 8 * c) * 2);
+        // Matrix tiles: K load u of lane li brings chunk kParts * lg + part of
+        // token u * kTpl + key_tok.
+        const int key_tok = li / S::kParts;
+        const int key_dim = 8 * (S::kParts * lg + li % S::kParts);
+        const uint32_t key_off = (uint32_t)(key_tok * row_bytes + (kvh * D + key_dim) * 2);
         auto page_of = [&](int t) __attribute__((always_inline)) -> int64_t {
             if (t >= end) return -1;
             return ctable[a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size];
         };
         int it = __builtin_amdgcn_readfirstlane(start + wave * S::kTpi);
         int64_t page_next = 0;
-        if constexpr (PAGE_UNIFORM) page_next = page_of(it);
+        if constexpr (PAGE_UNIFORM) page_next = !FLAT && a.lpt_batch == 0 ? first_page : page_of(it);
+        if constexpr (MM) {
+            // The next iteration's rows are loaded into the registers as soon as
+            // the products have read them: K right after the score products,
+            // V load by load, so that their latency overlaps the softmax and
+            // the output products.  No load is skipped (a branch around one
+            // would make the compiler wait for all of them): past the segment
+            // or without a page the loads read page 0's first rows, and `lim`
+            // masks what they bring.
+            u32x4 kk[L], vv[L];
+            int lim = 0, next_lim = 0;  // page-uniform: rows of the iteration at or past it are absent
+            int64_t next_base = 0;
+            bool ok[L], next_ok[L];
+            auto row_of = [&](int t) __attribute__((always_inline)) -> int64_t {
+                int64_t page = -1;
+                if (t < end) page = table[t / a.block_size];
+                return page >= 0 && page < a.num_blocks ? page * page_elems + (int64_t)(t % a.block_size) * row_elems
+                                                        : (int64_t)-1;
+            };
+            auto fetch_k = [&](int t0) __attribute__((always_inline)) {
+                // The owner's store of the new row completes before the row is read.
+                if constexpr (PRO)
+                    if (owner && t0 <= pos && pos < t0 + S::kTpi) __builtin_amdgcn_s_waitcnt(0);
+                if constexpr (PAGE_UNIFORM) {
+                    const int64_t page = page_next;
+                    page_next = page_of(t0 + kStep);
+                    const bool page_ok = page >= 0 && page < a.num_blocks;
+                    const int in_page = a.block_shift >= 0 ? t0 & (a.block_size - 1) : t0 % a.block_size;
+                    next_base = page_ok ? (page * a.block_size + in_page) * (int64_t)row_bytes : 0;
+                    next_lim = page_ok ? end : 0;
+                    const uint8_t* kp = static_cast<const uint8_t*>(a.key_cache) + next_base;
+#pragma unroll
+                    for (int u = 0; u < L; ++u)
+                        kk[u] = kv_load<STREAM>(kp + (key_off + (uint32_t)(u * S::kTpl * row_bytes)));
+                } else {
+#pragma unroll
+                    for (int u = 0; u < L; ++u) {
+                        const int64_t row = row_of(t0 + u * S::kTpl + key_tok);
+                        kk[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
+                            static_cast<const uint16_t*>(a.key_cache) + (row >= 0 ? row : 0) + kvh * D + key_dim));
+                    }
+                }
+            };
+            auto fetch_v = [&](int t0, int u) __attribute__((always_inline)) {
+                if constexpr (PAGE_UNIFORM) {
+                    vv[u] = kv_load<STREAM>(static_cast<const uint8_t*>(a.value_cache) + next_base + lane_off[u]);
+                } else {
+                    const int64_t row = row_of(t0 + u * S::kTpl + tl);
+                    next_ok[u] = row >= 0;
+                    vv[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
+                        static_cast<const uint16_t*>(a.value_cache) + (row >= 0 ? row : 0) + kvh * D + 8 * c));
+                }
+            };
+            if (it < end) {
+                fetch_k(it);
+#pragma unroll
+                for (int u = 0; u < L; ++u) fetch_v(it, u);
+            }
+            for (; it < end; it += kStep) {
+                lim = next_lim;
+#pragma unroll
+                for (int u = 0; u < L; ++u) ok[u] = PAGE_UNIFORM ? it + u * S::kTpl + tl < lim : next_ok[u];
+                f32x4 sc[kStates][L];
+#pragma unroll
+                for (int u = 0; u < L; ++u)
+#pragma unroll
+                    for (int t = 0; t < kStates; ++t)
+                        sc[t][u] = T::mfma16x16x32(kk[u], qop[t], f32x4{0.f, 0.f, 0.f, 0.f});
+                fetch_k(it + kStep);
+                float p[kStates][L];
+#pragma unroll
+                for (int t = 0; t < kStates; ++t) {
+                    // Scores, unscaled (the scale is positive: the maximum
+                    // and the exponent apply it).
+                    float s[L];
+#pragma unroll
+                    for (int u = 0; u < L; ++u) {
+                        float d;
+                        if constexpr (S::kParts == 4) {
+                            // Lane li has the partial of part li / 4; its
+                            // token's other parts are in lanes li +- 4, 8.
+                            const float lo = (li & 4) ? sc[t][u][1] : sc[t][u][0], hi = (li & 4) ? sc[t][u][3] : sc[t][u][2];
+                            d = (li & 8) ? hi : lo;
+                            d += dpp<kDppRowRor4>(d);
+                            d += dpp<kDppRowRor8>(d);
+                        } else {
+                            // Rows 4 lg + 0, 1: token 2 lg's parts; + 2, 3:
+                            // token 2 lg + 1's.  Lanes 0..7 keep the first
+                            // token (part 0 their own), lanes 8..15 the second.
+                            const float keep = (li & 8) ? sc[t][u][3] : sc[t][u][0], send = (li & 8) ? sc[t][u][1] : sc[t][u][2];
+                            d = keep + dpp<kDppRowRor8>(send);
+                        }
+                        s[u] = ok[u] ? d : kNegInf;
+                    }
+                    const float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])) * a.scale_log2;
+                    // The reference is raised, and the sums rescaled, only
+                    // when a score exceeds it by kRaise binary orders (or
+                    // there is none yet): probabilities stay below 2^kRaise,
+                    // far inside fp32, and the final division does not depend
+                    // on the reference.
+                    if (__ballot(mx > m[t] + kRaise) != 0) {
+                        const float mn = fmaxf(m[t], mx);
+                        const float alpha = fast_exp2(m[t] - (mn == kNegInf ? 0.f : mn));
+                        m[t] = mn;
+                        l[t] *= alpha;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) macc[t][e] *= alpha;
+                        if constexpr (G == 8 && kStates == 1) {
+                            const float other = lane_xor4(alpha);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) macc[1][e] *= other;
+                        }
+                    }
+                    const float ref = m[t] == kNegInf ? 0.f : m[t];
+#pragma unroll
+                    for (int u = 0; u < L; ++u) p[t][u] = fast_exp2(fmaf(s[u], a.scale_log2, -ref));
+                    l[t] += (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
+                }
+                // 0 * (stale NaN) must not reach the sums.
+                if (!PAGE_UNIFORM || it + S::kTpi > lim) {
+#pragma unroll
+                    for (int u = 0; u < L; ++u)
+                        if (!ok[u]) vv[u] = u32x4{0u, 0u, 0u, 0u};
+                }
+#pragma unroll
+                for (int u = 0; u < L; ++u) {
+                    float pu[G / 4];
+                    pu[0] = p[0][u];
+                    if constexpr (G == 8) pu[1] = kStates == 2 ? p[kStates - 1][u] : lane_xor4(p[0][u]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float v0 = T::lo(vv[u][i]), v1 = T::hi(vv[u][i]);
+#pragma unroll
+                        for (int t = 0; t < G / 4; ++t) {
+                            macc[t][2 * i] = __builtin_amdgcn_mfma_f32_4x4x1f32(v0, pu[t], macc[t][2 * i], 0, 0, 0);
+                            macc[t][2 * i + 1] =
+                                __builtin_amdgcn_mfma_f32_4x4x1f32(v1, pu[t], macc[t][2 * i + 1], 0, 0, 0);
+                        }
+                    }
+                    fetch_v(it + kStep, u);
+                }
+            }
+        } else {
         for (; it < end; it += kStep) {
             u32x4 kk[L], vv[L];
             bool ok[L];
@@ -554,36 +803,107 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
             }
         }
 
-        // Merge the token groups of this wave (lanes with equal chunk index).
-#pragma unroll
-        for (int mask = S::kLpt; mask < kWave; mask <<= 1) {
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const float mo = shfl_xor(m[g], mask);
-                const float lo = shfl_xor(l[g], mask);
-                const float mn = fmaxf(m[g], mo);
-                const float ref = mn == kNegInf ? 0.f : mn;
-                const float a1 = fast_exp2(m[g] - ref);
-                const float a2 = fast_exp2(mo - ref);
-                l[g] = l[g] * a1 + lo * a2;
-                m[g] = mn;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float ao = shfl_xor(acc[g][i], mask);
-                    acc[g][i] = acc[g][i] * a1 + ao * a2;
-                }
-            }
         }
 
+        // (Exchanging every sum with every partner lane through ds_bpermute,
+        // as it was, took 128 of them per wave for a tile of 8 heads.)
+        if constexpr (MM) {
+            // Merge the token slots of this wave: the states' maxima and sums
+            // across lanes 16 and 32 apart (and 8 apart at D = 64), the
+            // running sums scaled to the common reference and added, each
+            // exchange halving what a lane holds: lanes of the upper half
+            // keep dims 4..7 of each chunk, odd 16-lane rows the odd chunks.
+            float f[G / 4];
+#pragma unroll
+            for (int g = 0; g < kStates; ++g) {
+                float mn = row4_max(m[g]);
+                if constexpr (S::kLpt == 8) mn = fmaxf(mn, dpp<kDppRowRor8>(mn));
+                f[g] = fast_exp2(m[g] - (mn == kNegInf ? 0.f : mn));
+                m[g] = mn;
+                l[g] = row4_sum(l[g] * f[g]);
+                if constexpr (S::kLpt == 8) l[g] += dpp<kDppRowRor8>(l[g]);
+            }
+            if constexpr (G == 8 && kStates == 1) f[G / 4 - 1] = lane_xor4(f[0]);
+#pragma unroll
+            for (int t = 0; t < G / 4; ++t) {
+                float half[4][4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        half[e][i] = swap32_add(macc[t][e][i] * f[t], macc[t][e + 4][i] * f[t]);
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float v = swap16_add(half[e][2 * k], half[e][2 * k + 1]);
+                        if constexpr (S::kLpt == 8) v += dpp<kDppRowRor8>(v);
+                        macc[t][k][e] = v;
+                    }
+            }
+        } else {
+        // The same for the dot-product tiles: token slots 2, 4 and 8 lanes
+        // apart are added in place, those 16 and 32 apart by exchanges, after
+        // which a lane keeps kKeep of its chunk's 8 dims, from keep0 on.
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            float mn = m[g];
+            if constexpr (S::kLpt <= 2) mn = fmaxf(mn, dpp<kDppQuadSwap2>(mn));
+            if constexpr (S::kLpt <= 4) mn = fmaxf(mn, lane_xor4(mn));
+            if constexpr (S::kLpt <= 8) mn = fmaxf(mn, dpp<kDppRowRor8>(mn));
+            if constexpr (S::kLpt <= 16) mn = row4_max(mn);
+            else if constexpr (S::kLpt == 32) mn = pair32_max(mn);
+            const float f = fast_exp2(m[g] - (mn == kNegInf ? 0.f : mn));
+            m[g] = mn;
+            auto within = [](float v) __attribute__((always_inline)) -> float {
+                if constexpr (S::kLpt <= 2) v += dpp<kDppQuadSwap2>(v);
+                if constexpr (S::kLpt <= 4) v += lane_xor4(v);
+                if constexpr (S::kLpt <= 8) v += dpp<kDppRowRor8>(v);
+                return v;
+            };
+            l[g] = within(l[g] * f);
+            if constexpr (S::kLpt <= 16) l[g] = row4_sum(l[g]);
+            else if constexpr (S::kLpt == 32) l[g] = swap32_add(l[g], l[g]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[g][i] = within(acc[g][i] * f);
+            if constexpr (S::kLpt <= 32)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[g][i] = swap32_add(acc[g][i], acc[g][i + 4]);
+            if constexpr (S::kLpt <= 16)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc[g][i] = swap16_add(acc[g][i], acc[g][i + 2]);
+        }
+        }
+        constexpr int kKeep = S::kLpt <= 16 ? 2 : S::kLpt == 32 ? 4 : 8;
+        const int keep0 = S::kLpt <= 16 ? 4 * (lane >> 5) + 2 * (lg & 1) : S::kLpt == 32 ? 4 * (lane >> 5) : 0;
+
         // Merge the waves through LDS.
-        __shared__ float sm_acc[NW][G][D];
+        __shared__ __attribute__((aligned(16))) float sm_acc[NW][G][D];
         __shared__ float sm_ml[NW][G][2];
-        if (tl == 0 && chunk_ok) {
+        if constexpr (MM) {
+            if (li < S::kLpt) {
+#pragma unroll
+                for (int t = 0; t < G / 4; ++t) {
+                    const int g = kStates == 1 ? (c % G) ^ (4 * t) : c % 4 + 4 * t;
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        const int chunk = 4 * (c >> 2) + 2 * k + (lg & 1);
+                        *reinterpret_cast<f32x4*>(&sm_acc[wave][g][8 * chunk + 4 * (lg >> 1)]) = macc[t][k];
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < kStates; ++t)
+                    if (lane < G / kStates) {
+                        sm_ml[wave][lane + 4 * t][0] = m[t];
+                        sm_ml[wave][lane + 4 * t][1] = l[t];
+                    }
+            }
+        } else if ((lane & (S::kLpt <= 16 ? 15 : 63) & ~(S::kLpt == 32 ? 32 : 0)) < S::kLpt && chunk_ok) {
 #pragma unroll
             for (int g = 0; g < G; ++g) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) sm_acc[wave][g][8 * c + i] = acc[g][i];
-                if (c == 0) {
+                for (int i = 0; i < kKeep; ++i) sm_acc[wave][g][8 * c + keep0 + i] = acc[g][i];
+                if (lane == 0) {
                     sm_ml[wave][g][0] = m[g];
                     sm_ml[wave][g][1] = l[g];
                 }
@@ -591,7 +911,7 @@ __global__ __launch_bounds__(NW * kWave) void paged_decode_kernel(DecodeArgs a) 
         }
         __syncthreads();
 
-        for (int idx = threadIdx.x; idx < G * D; idx += NW * kWave) {
+        for (int idx = threadIdx.x; idx < heads * D; idx += NW * kWave) {
             const int g = idx / D;
             const int d = idx - g * D;
             float mx = sm_ml[0][g][0];

@@ -340,21 +340,6 @@ __device__ inline void landed_barrier() {
     asm volatile("s_barrier" : : : "memory");
 }
 
-// Max / sum over the four lanes {l, l^16, l^32, l^48} (the 4 MFMA k-groups
-// holding one query row) with gfx950 lane swaps -- no LDS round trip.
-__device__ inline float row4_max(float x) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ inline float row4_sum(float x) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // Direct global -> LDS copy from a wave-uniform base plus a per-lane 32-bit
 // byte offset (the SGPR-base form of global_load_lds_dwordx4: no 64-bit
 // per-lane address arithmetic).  M0 (the LDS destination) is declared

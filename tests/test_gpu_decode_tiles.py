@@ -1,0 +1,96 @@
+"""GPU parity of decode attention for query groups on the matrix cores.
+
+Groups of three or more query heads per kv head at head_dim 64 and 128 run in
+tiles of up to 4 or 8 heads (several tiles above 8, the last one partly
+filled).  Cases sit at the tiles' edges: group sizes around 4 and 8, contexts
+around one wave iteration (16 or 32 tokens) and one page, pages that do and
+do not hold whole iterations, whole sequences, split-K and the balanced walk.
+Tolerance: the decode gate against the fp32 oracle."""
+
+import pytest
+import torch
+
+from gpu_cases import decode_inputs
+from mini_engine_hip.kernels.paged import paged_attention
+from oracle import paged_oracle
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+GATE = {torch.float16: 2e-3, torch.bfloat16: 1.6e-2}
+
+
+def oracle(args):
+    return paged_oracle.fp32_oracle(dict(zip(paged_oracle.TENSOR_NAMES, args[:5])), args[5])
+
+
+def check(args, dtype, partition):
+    dev = [a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args]
+    actual = paged_attention(*dev, partition_tokens=partition).float().cpu()
+    assert (actual - oracle(args)).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("group", [3, 4, 5, 7, 8, 9, 12, 16, 17])
+def test_group_sizes_around_the_tiles(dtype, dim, group):
+    lengths = (1, 15, 16, 17, 33, 130, 257, 700)
+    args = decode_inputs(dtype, head_dim=dim, lengths=lengths, heads=2 * group, kv_heads=2, seed=100 * dim + group)
+    for partition in (0, 64, 192, -1):
+        check(args, dtype, partition)
+
+
+@pytest.mark.parametrize("block,lengths,partition", [
+    (7, (50, 13, 1), 0), (24, (500, 24, 25), 128), (5, (333, 40), -1),     # per-token page lookups
+    (16, (4097,), 0), (256, (2048, 1, 700), 0), (256, (5000, 4100), 0),    # plan's walk and split-K
+    (16, tuple([200] * 40), 0), (16, tuple(range(1, 161, 4)), 0),           # whole sequences
+])
+@pytest.mark.parametrize("dim,group", [(64, 7), (128, 4), (128, 7)])
+def test_pages_and_modes(block, lengths, partition, dim, group):
+    dtype = torch.bfloat16
+    args = decode_inputs(dtype, head_dim=dim, block_size=block, lengths=lengths, heads=4 * group, kv_heads=4,
+                         seed=block + len(lengths))
+    check(args, dtype, partition)
+
+
+@pytest.mark.parametrize("dim,group", [(64, 8), (128, 4), (128, 8)])
+def test_scores_that_keep_rising_and_stale_rows(dim, group):
+    """Scores rise by several binary orders along the context, so that the
+    running reference is raised again and again (and late keys carry nearly
+    all of the weight); rows past a context's end hold NaN and infinities."""
+    dtype = torch.float16
+    args = list(decode_inputs(dtype, head_dim=dim, lengths=(601, 250), heads=2 * group, kv_heads=2, seed=dim))
+    q, key, value, table, lens, block = args
+    q.fill_(0.5)
+    for b in range(2):
+        for i, page in enumerate(table[b].tolist()):
+            key[page] = 0.02 * key[page] + 0.004 * i * (128 / dim)
+    last = table[1, 250 // block]
+    key[last, 250 % block:] = float("nan")
+    value[last, 250 % block:] = float("inf")
+    dev = [a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args]
+    clean = [a.clone() if isinstance(a, torch.Tensor) else a for a in args]
+    clean[1][last, 250 % block:] = 0
+    clean[2][last, 250 % block:] = 0
+    for partition in (0, 64, -1):
+        actual = paged_attention(*dev, partition_tokens=partition, validate=False).float().cpu()
+        assert (actual - oracle(clean)).abs().max().item() <= GATE[dtype]
+
+
+def test_absent_pages_and_lengths_count_as_nothing():
+    """Trusted calls with pages and lengths out of range: those tokens are
+    absent, a sequence without any gives zeros."""
+    args = list(decode_inputs(torch.bfloat16, lengths=(300, 90, 64), heads=28, kv_heads=4))
+    q, key, value, table, lens, block = [a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args]
+    table = table.clone()
+    table[0, 3] = 1 << 40
+    table[1, :] = -1
+    lens = torch.tensor([300, 90, 1 << 40], device=DEV)
+    keep = [t for t in range(300) if t // block != 3]
+    flat_k = key[table[0].clamp(0, key.shape[0] - 1)].flatten(0, 1)[keep].float()
+    flat_v = value[table[0].clamp(0, key.shape[0] - 1)].flatten(0, 1)[keep].float()
+    score = torch.stack([flat_k[:, h // 7] @ q[0, h].float() for h in range(28)]) * 128 ** -0.5
+    want = torch.stack([score[h].softmax(0) @ flat_v[:, h // 7] for h in range(28)])
+    for partition in (0, 64, -1):
+        out = paged_attention(q, key, value, table, lens, block, validate=False, partition_tokens=partition).float()
+        assert (out[0] - want).abs().max().item() <= GATE[torch.bfloat16]
+        assert out[1].abs().max().item() == 0 and out[2].abs().max().item() == 0
