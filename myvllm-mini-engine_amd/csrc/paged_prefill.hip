@@ -302,6 +302,70 @@ __device__ inline bool find_item(const PrefillArgs& a, int chunk_len, int item, 
     return found;
 }
 
+// Query blocks of a sequence that need more than `t` keys (t >= -1).  A block's
+// key end grows with its index, so these are the last ones.
+__device__ inline int blocks_above(const PrefillArgs& a, const SeqMeta& m, int blocks, int64_t t) {
+    if (t < 0) return blocks;
+    const int64_t cap = (int64_t)a.table_width * a.block_size;
+    if (min(m.ctx, cap) <= t || m.start + m.n <= t) return 0;
+    // Blocks b with start + (b + 1) * qb <= t need at most t keys.
+    const int64_t below = t - m.start;
+    if (below < a.qb) return blocks;
+    // floor(below / qb): the float quotient's ceiling, one less when it is no exact multiple.
+    const uint32_t up = ceil_div_u32((uint32_t)below, (uint32_t)a.qb);
+    const int full = (int)(up * (uint32_t)a.qb == (uint32_t)below ? up : up - 1);
+    return max(blocks - full, 0);
+}
+
+// Item `item` of a call without a key split (every query block is one item)
+// and at most 64 sequences, enumerated by falling key end: blocks of all
+// sequences in buckets of kOrderKeys keys, the longest bucket first, so that
+// the work-groups dispatched last are short whichever sequence they belong
+// to.  In sequence order a long block of a late sequence starts when the
+// others are nearly done: 16 sequences of 56..900 new tokens after 0..700
+// cached ones (fp16, pages of 16) 91 -> 86 us, 4 prompts of 4096 273.5 ->
+// 265.1.  Buckets, not single lengths, so that the blocks of one sequence
+// stay together and share its K/V in L2.  Lane s holds sequence s; the bucket
+// is found by bisection on the number of blocks above a key count.
+constexpr int kOrderKeys = 256;
+template <bool DENSE>
+__device__ inline bool find_item_longest(const PrefillArgs& a, int item, PrefillItem& it) {
+    const int lane = __lane_id();
+    const SeqMeta m = load_meta<DENSE>(a, lane);
+    const int blocks = query_blocks(a, m.n);
+    auto count_above = [&](int64_t t) __attribute__((always_inline)) -> int {
+        return lane_value(wave_incl_scan(blocks_above(a, m, blocks, t)), kWave - 1);
+    };
+    if (item >= count_above(-1)) return false;
+    // Largest bucket [lo * kOrderKeys, (lo + 1) * kOrderKeys) with more than `item` blocks above its
+    // lower end; lo = -1 stands for the blocks that need no key.
+    int lo = -1, hi = (int)(((int64_t)a.table_width * a.block_size + kOrderKeys - 1) / kOrderKeys);
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (count_above((int64_t)mid * kOrderKeys) > item) lo = mid;
+        else hi = mid;
+    }
+    const int above = blocks_above(a, m, blocks, (int64_t)hi * kOrderKeys);  // blocks of longer buckets
+    const int mine = blocks_above(a, m, blocks, lo < 0 ? -1 : (int64_t)lo * kOrderKeys) - above;
+    const int before = lane_value(wave_incl_scan(above), kWave - 1);
+    const int incl = wave_incl_scan(mine);
+    const uint64_t hit = __ballot(before + incl > item);
+    const int sel = __builtin_ctzll(hit);
+    const int rank = item - before - (lane_value(incl, sel) - lane_value(mine, sel));
+    const int block = lane_value(blocks, sel) - 1 - lane_value(above, sel) - rank;
+    it.seq = sel;
+    it.q0 = block * a.qb;
+    it.chunk = 0;
+    it.nchunks = 1;
+    it.chunk_len = a.chunk;
+    it.row0 = lane_value(m.row0, sel);
+    it.qlen = lane_value(m.n, sel);
+    it.start = lane_value(m.start, sel);
+    it.ctx = lane_value(m.ctx, sel);
+    it.kv_end = block_kv_end(a, it.start, it.ctx, it.qlen, it.q0);
+    return true;
+}
+
 // Direct global -> LDS copy of 16 bytes per lane: lane i's bytes land at LDS
 // address `lds_base + 16*i` (lds_base is wave-uniform, passed through M0).
 // Issued as inline assembly so that the compiler does not serialise it
@@ -369,6 +433,7 @@ __device__ inline uint32_t wave_min_u32(uint32_t x) {
 constexpr int kPagesPerLane = 0;
 constexpr int kPagesPerRows = 1;
 constexpr int kPagesPerTile = 2;
+constexpr int kPagesPerWave = 3;
 
 // How page ids are found (PAGES):
 //   kPagesPerTile: block_size is a power of two >= 64, so a 64-key tile lies
@@ -376,6 +441,10 @@ constexpr int kPagesPerTile = 2;
 //     are a scalar base plus precomputed per-lane offsets -- a few scalar
 //     instructions per tile, which matters because the scalar unit is shared
 //     by all waves of the CU.
+//   kPagesPerWave: block_size is 8, 16 or 32 (the 128 shape): the 8 key rows
+//     of a tile that one wave copies lie in one page, so a whole tile's copies
+//     are again a scalar base (each wave its own page's) plus the same
+//     per-lane offsets.
 //   kPagesPerRows: see below; the fallback for partial tiles as well.
 // SCALAR_PAGES: block_size is a multiple of 4, so the 4 key rows one copy
 // instruction covers sit in one page and the page id is wave-uniform (a
@@ -510,8 +579,16 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                                                             PrefillLds& lds) {
     using SH = PfShape<HD>;
     constexpr bool SCALAR_PAGES = PAGES != kPagesPerLane;
-    // The software-pipelined loop serves whole-tile pages of the 128 shape.
-    constexpr bool PIPE = PAGES == kPagesPerTile && !NARROW && HD == 128 && !DENSE;
+    // The software-pipelined loop serves pages of the 128 shape that hold
+    // each wave's copy rows of a tile.
+    constexpr bool WAVE_PAGES = PAGES == kPagesPerWave;
+    constexpr bool PIPE = (PAGES == kPagesPerTile || WAVE_PAGES) && !NARROW && HD == 128;
+    // Queries scaled once by scale*log2(e) (one more rounding of q) instead
+    // of every score in fp32.  The modes that joined the pipelined loop later
+    // (small pages 127.9 -> 111.2 us for 16 sequences of 56..900 tokens with
+    // their norm, rotation and write; a dense 8192-token prompt 255.3 -> 239.4)
+    // scale in fp32, which they did before: their error stays what it was.
+    constexpr bool PRESCALE = PAGES == kPagesPerTile && !DENSE;
     const int hd = NARROW ? a.head_dim : SH::kD;  // elements per K/V/Q/output row in memory
     const int dchunks = hd / 8;                 // 16-byte chunks per row
     auto& sm_k = lds.k;
@@ -784,39 +861,70 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
         // ahead of the V copies, both in 4-stage rings (tile i: K and V
         // stage i mod 4, i counted from t_begin).
         //
-        // The queries are pre-scaled by scale*log2(e) and each score product
-        // starts from the row's -reference (the MFMA's C input), so a
-        // probability is one exp2 of the product.
+        // With PRESCALE (pages of at least a tile) the queries are pre-scaled
+        // by scale*log2(e) and each score product starts from the row's
+        // -reference (the MFMA's C input), so a probability is one exp2 of the
+        // product; otherwise an fp32 multiply-add scales the score.
         const u32x4 ones = {T::pack(1.f, 1.f), T::pack(1.f, 1.f), T::pack(1.f, 1.f), T::pack(1.f, 1.f)};
         const int ntiles = t_end - t_begin;
         f32x4 sc[SH::kHalves][SH::kNb][2];
         u32x4 pops[SH::kHalves][SH::kNb];
         // Per lane j: byte offset (from the kv head's base) of tile
-        // tile_base + j's first key row when the tile is whole (present page,
-        // all of its keys in the chunk), else -1.
+        // tile_base + j's first key row when the tile is whole (present
+        // pages, all of its keys in the chunk), else -1.  With pages per
+        // wave: where that row would lie if the page of this wave's rows
+        // went back that far (a wave adds only its own rows' offsets), plus
+        // wave_bias so that no whole tile's value is negative.
+        constexpr int kCopyRows = SH::kKeys / kPfWaves;  // key rows of a tile one wave copies
+        const int64_t wave_bias = WAVE_PAGES ? (int64_t)SH::kKeys * row_bytes_g : 0;
         int64_t tile_offs = -1;
         auto window_offsets = [&](int64_t raw, int base) -> int64_t {
             const int key0 = (base + lane) * SH::kKeys;
             const bool whole = raw >= 0 && raw < a.num_blocks && key0 + SH::kKeys <= chunk_end;
             return whole ? raw * page_bytes_g + (int64_t)(key0 & (a.block_size - 1)) * row_bytes_g : (int64_t)-1;
         };
+        // Pages per wave: the window's tiles need every page of a tile (it
+        // is whole, for all waves, only if all are present).
+        auto window_small = [&](int base) -> int64_t {
+            const int key0 = (base + lane) * SH::kKeys;
+            bool whole = key0 + SH::kKeys <= chunk_end;
+            int64_t mine = 0;
+            if (whole) {
+                const int per_tile = SH::kKeys >> bs_shift;
+                const int own = (kCopyRows * wave) >> bs_shift;
+                for (int j = 0; j < per_tile; ++j) {
+                    const int64_t page = table[(key0 >> bs_shift) + j];
+                    whole = whole && page >= 0 && page < a.num_blocks;
+                    if (j == own) mine = page;
+                }
+            }
+            const int in_page = (kCopyRows * wave) & (a.block_size - 1);
+            return whole ? mine * page_bytes_g + (int64_t)(in_page - kCopyRows * wave) * row_bytes_g + wave_bias
+                         : (int64_t)-1;
+        };
         // Moves to the next window (loaded a window ago, retired by a landed
         // barrier's full wait since) and loads the one after it.  Called at
         // one place per issue phase: two consecutive tiles never both cross
         // a window boundary, and a second call site would read the load the
-        // first one just issued.
+        // first one just issued.  (Pages per wave: loaded here, once per 64
+        // tiles.)
         auto next_window = [&]() {
-            tile_pages = next_pages;
             tile_base += kWave;
-            tile_offs = window_offsets(tile_pages, tile_base);
-            if (tile_base + kWave < t_end) next_pages = window_pages(tile_base + kWave);
+            if constexpr (WAVE_PAGES) {
+                tile_offs = window_small(tile_base);
+            } else {
+                tile_pages = next_pages;
+                tile_offs = window_offsets(tile_pages, tile_base);
+                if (tile_base + kWave < t_end) next_pages = window_pages(tile_base + kWave);
+            }
         };
         // Row-by-row copies of a tile that is not whole: absent rows load
         // zeros (finite in both rings) and, for K, get a -inf bias.
         auto issue_rows = [&](int tile, int st, bool is_k) {
             const int key0 = tile * SH::kKeys;
-            const int64_t page = ctable[(key0 < cap ? key0 : cap - 1) >> bs_shift];
-            const bool pg_ok = key0 < chunk_end && page >= 0 && page < a.num_blocks;
+            const int first = key0 + (WAVE_PAGES ? kCopyRows * wave : 0);
+            const int64_t page = ident ? seq : ctable[(first < cap ? first : cap - 1) >> bs_shift];
+            const bool pg_ok = first < chunk_end && page >= 0 && page < a.num_blocks;
             const int64_t base = pg_ok ? page * page_bytes_g : 0;
             const uint8_t* cache = is_k ? kcache : vcache;
             const uint32_t lds0 = lds_addr(is_k ? &sm_k[st][0] : &sm_v[st][0]);
@@ -838,7 +946,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                 full_stages |= 1u << st;
                 const uint32_t lk = lds_addr(&sm_k[st][0]);
 #pragma unroll
-                for (int i = 0; i < SH::kIpw; ++i) lds_dma16_s(kcache + off, tile_off[i], lk + 1024 * (SH::kIpw * wave + i));
+                for (int i = 0; i < SH::kIpw; ++i) lds_dma16_s(kcache + (off - wave_bias), tile_off[i], lk + 1024 * (SH::kIpw * wave + i));
             } else {
                 full_stages &= ~(1u << st);
                 issue_rows(tile, st, true);
@@ -849,12 +957,12 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                 const uint32_t lv = lds_addr(&sm_v[st][0]);
 #pragma unroll
                 for (int i = 0; i < SH::kIpw; ++i)
-                    lds_dma16_s(vcache + off, tile_off_v[i], lv + 1024 * (SH::kIpw * wave + i));
+                    lds_dma16_s(vcache + (off - wave_bias), tile_off_v[i], lv + 1024 * (SH::kIpw * wave + i));
             } else {
                 issue_rows(tile, st, false);
             }
         };
-        // S^T of a tile (K stage st), starting from -reference.
+        // S^T of a tile (K stage st), starting from -reference (PRESCALE).
         auto s_product = [&](int st) __attribute__((always_inline)) {
             const uint8_t* smk = &sm_k[st][0];
             __builtin_amdgcn_s_setprio(1);
@@ -870,7 +978,8 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                 for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
                     for (int nb = 0; nb < SH::kNb; ++nb) {
-                        f32x4 c = {nref[nb], nref[nb], nref[nb], nref[nb]};
+                        const float c0 = PRESCALE ? nref[nb] : 0.f;
+                        f32x4 c = {c0, c0, c0, c0};
 #pragma unroll
                         for (int dc = 0; dc < SH::kDc; ++dc) c = T::mfma16x16x32(kop[kk][dc], qop[nb][dc], c);
                         sc[h][nb][kk] = c;
@@ -960,7 +1069,9 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
 #pragma unroll
                     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) p[4 * kk + j] = fast_exp2(sc[h][nb][kk][j]);
+                        for (int j = 0; j < 4; ++j)
+                            p[4 * kk + j] = fast_exp2(PRESCALE ? sc[h][nb][kk][j]
+                                                               : fmaf(sc[h][nb][kk][j], a.scale_log2, nref[nb]));
                     pops[h][nb] = u32x4{T::pack(p[0], p[1]), T::pack(p[2], p[3]), T::pack(p[4], p[5]), T::pack(p[6], p[7])};
                     {
                         typedef unsigned short us2 __attribute__((ext_vector_type(2)));
@@ -981,7 +1092,8 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
 #pragma unroll
                         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) r = fmaxf(r, sc[h][nb][kk][j] - nref[nb]);
+                            for (int j = 0; j < 4; ++j) r = fmaxf(r, PRESCALE ? sc[h][nb][kk][j] - nref[nb] : sc[h][nb][kk][j]);
+                    if constexpr (!PRESCALE) r *= a.scale_log2;
                     const float mn = fmaxf(m_run[nb], row4_max(r));
                     const float alpha = (m_run[nb] == kNegInf || mn == kNegInf) ? 1.f : fast_exp2(m_run[nb] - mn);
                     const float shift = mn == kNegInf ? 0.f : nref[nb] + mn;
@@ -998,7 +1110,9 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
 #pragma unroll
                         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) p[4 * kk + j] = fast_exp2(sc[h][nb][kk][j] - shift);
+                            for (int j = 0; j < 4; ++j)
+                                p[4 * kk + j] = fast_exp2(PRESCALE ? sc[h][nb][kk][j] - shift
+                                                                   : fmaf(sc[h][nb][kk][j], a.scale_log2, nref[nb]));
                         pops[h][nb] =
                             u32x4{T::pack(p[0], p[1]), T::pack(p[2], p[3]), T::pack(p[4], p[5]), T::pack(p[6], p[7])};
                     }
@@ -1050,16 +1164,22 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
             // with the queries; tile 0 is then computed whole while K of
             // tiles 1, 2 and V of tile 1 are in flight.
             const int key0 = t_begin * SH::kKeys;
-            const int64_t page0 = ctable[key0 >> bs_shift];
-            const bool whole0 = key0 + SH::kKeys <= chunk_end && page0 >= 0 && page0 < a.num_blocks;
-            const int64_t off0 =
-                whole0 ? page0 * page_bytes_g + (int64_t)(key0 & (a.block_size - 1)) * row_bytes_g : (int64_t)-1;
+            int64_t off0;
+            if constexpr (WAVE_PAGES) {
+                tile_offs = window_small(tile_base);
+                off0 = lane_value(tile_offs, 0);
+            } else {
+                const int64_t page0 = ident ? seq : ctable[key0 >> bs_shift];
+                const bool whole0 = key0 + SH::kKeys <= chunk_end && page0 >= 0 && page0 < a.num_blocks;
+                off0 = whole0 ? page0 * page_bytes_g + (int64_t)(key0 & (a.block_size - 1)) * row_bytes_g : (int64_t)-1;
+            }
             issue_k(t_begin, 0, off0);
             issue_v(t_begin, 0, off0);
-            if (t_begin + kWave < t_end) next_pages = window_pages(t_begin + kWave);
+            if constexpr (!WAVE_PAGES)
+                if (t_begin + kWave < t_end) next_pages = window_pages(t_begin + kWave);
             if (threadIdx.x == 0) lds.arrive = 0;  // no wave counts before the next barrier
             landed_barrier();
-            tile_offs = window_offsets(tile_pages, tile_base);
+            if constexpr (!WAVE_PAGES) tile_offs = window_offsets(tile_pages, tile_base);
             int64_t pend = -1;  // offset of the last K tile issued, whose V is still to come
             if (ntiles > 1) {  // tiles 1 and 2 lie in the first window
                 const int64_t off1 = lane_value(tile_offs, 1);
@@ -1072,7 +1192,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
             }
             // Queries scaled by scale*log2(e) (they landed at the barrier).
 #pragma unroll
-            for (int nb = 0; nb < SH::kNb; ++nb)
+            for (int nb = 0; nb < (PRESCALE ? SH::kNb : 0); ++nb)
 #pragma unroll
                 for (int dc = 0; dc < SH::kDc; ++dc)
 #pragma unroll
@@ -1567,7 +1687,10 @@ __global__ __launch_bounds__(kPfThreads, 1) void paged_prefill_mfma_kernel(Prefi
     }
     if constexpr (!WALK) {
         PrefillItem item;
-        if (!find_item<DENSE>(a, a.chunk, blockIdx.x / a.kv_heads, item)) return;
+        const int index = blockIdx.x / a.kv_heads;
+        const bool found = a.max_chunks == 1 && a.num_seqs <= kWave ? find_item_longest<DENSE>(a, index, item)
+                                                                    : find_item<DENSE>(a, a.chunk, index, item);
+        if (!found) return;
         prefill_item<T, PAGES, NARROW, HD, DENSE>(a, item, lds);
     } else {
         // The first lookup also counts the items, so that the walk ends
@@ -2001,7 +2124,11 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
         const int64_t block_size = a.block_size;
         const bool dense = a.tables == nullptr;
         if (dense && !tile_pages) return fail(MVME_EINVAL, "prefill key/value token stride too large");
-        int pages = tile_pages ? kPagesPerTile : (block_size % 4 == 0 ? kPagesPerRows : kPagesPerLane);
+        // Pages per wave: a wave copies 8 consecutive key rows of a tile, so
+        // power-of-two blocks of 8, 16 or 32 tokens keep them in one page.
+        const bool wave_pages = a.block_shift >= 3 && p.hd == 128 && !p.narrow &&
+                                a.kv_row_bytes * p.keys < (int64_t(1) << 31);
+        int pages = tile_pages ? kPagesPerTile : wave_pages ? kPagesPerWave : (block_size % 4 == 0 ? kPagesPerRows : kPagesPerLane);
         if (p.narrow && pages == kPagesPerRows) pages = kPagesPerLane;  // no narrow instantiation of that mode
         const dim3 grid((unsigned)groups), block(kPfThreads);
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
@@ -2052,6 +2179,9 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
             } else if (pages == kPagesPerTile) {
                 launch_walk(paged_prefill_mfma_kernel<T, kPagesPerTile, false, false, 128, false>,
                             paged_prefill_mfma_kernel<T, kPagesPerTile, true, false, 128, false>);
+            } else if (pages == kPagesPerWave) {
+                launch_walk(paged_prefill_mfma_kernel<T, kPagesPerWave, false, false, 128, false>,
+                            paged_prefill_mfma_kernel<T, kPagesPerWave, true, false, 128, false>);
             } else if (pages == kPagesPerRows) {
                 launch_walk(paged_prefill_mfma_kernel<T, kPagesPerRows, false, false, 128, false>,
                             paged_prefill_mfma_kernel<T, kPagesPerRows, true, false, 128, false>);

@@ -1,0 +1,94 @@
+"""GPU parity of the pipelined prefill loop over pages smaller than a key
+tile (8, 16 and 32 tokens) and in dense mode, and of the order of query
+blocks across sequences."""
+
+import pytest
+import torch
+
+from mini_engine_hip.kernels.prefill import paged_prefill_attention, prefill_attention
+from oracle import paged_oracle
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+GATE = {torch.float16: 2e-3, torch.bfloat16: 1.6e-2}
+
+
+def paged_case(new, prior, block, heads, kv_heads, dtype, seed):
+    gen = torch.Generator().manual_seed(seed)
+    cu = torch.tensor([0] + torch.tensor(new).cumsum(0).tolist())
+    starts = torch.tensor(prior)
+    lens = starts + torch.tensor(new)
+    width = max(1, -(-int(lens.max()) // block))
+    pages = len(new) * width + 3
+    kc = torch.randn(pages, block, kv_heads, 128, generator=gen).to(dtype)
+    vc = torch.randn(pages, block, kv_heads, 128, generator=gen).to(dtype)
+    tables = torch.randperm(pages, generator=gen)[:len(new) * width].view(len(new), width)
+    q = torch.randn(int(cu[-1]), heads, 128, generator=gen).to(dtype)
+    return [q, kc, vc, cu, starts, tables, lens]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block", [8, 16, 32])
+@pytest.mark.parametrize("new,prior,chunk", [
+    ([64, 1, 130], [0, 63, 64], 0),          # whole tiles, one key past a tile, one before
+    ([40], [4400], 0), ([40], [4400], 8192),  # more than a window of 64 tiles, split and not
+    ([300, 77], [1200, 41], 256),            # walks over key chunks
+])
+def test_small_pages_match_the_oracle(dtype, block, new, prior, chunk):
+    args = paged_case(new, prior, block, 8, 4, dtype, seed=block + sum(new))
+    actual = paged_prefill_attention(*[a.to(DEV) for a in args], block, chunk_tokens=chunk).float().cpu()
+    expected = paged_oracle.paged_prefill_attention(*args, block, cast=False)
+    assert (actual - expected).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("block", [8, 16, 32, 64])
+def test_absent_pages_inside_a_tile(block):
+    """Trusted calls: a page out of range in the middle of a whole tile; its
+    keys are absent for every wave, the tile's other keys are not."""
+    dtype = torch.bfloat16
+    args = paged_case([50, 200], [400, 0], block, 8, 4, dtype, seed=block)
+    q, kc, vc, cu, starts, tables, lens = args
+    hole = 192 // block  # keys 192 .. 192 + block of sequence 0
+    tables[0, hole] = kc.shape[0] + 5
+    out = paged_prefill_attention(*[a.to(DEV) for a in args], block, validate=False).float().cpu()
+    keep = [k for k in range(450) if k // block != hole]
+    key = kc[tables[0].clamp(max=kc.shape[0] - 1)].flatten(0, 1).float()
+    value = vc[tables[0].clamp(max=kc.shape[0] - 1)].flatten(0, 1).float()
+    for row in (0, 49):
+        seen = [k for k in keep if k <= 400 + row]
+        for h in (0, 7):
+            p = (key[seen, h // 2] @ q[row, h].float() * 128 ** -0.5).softmax(0)
+            assert (out[row, h] - p @ value[seen, h // 2]).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("seqs,heads,kv_heads", [(40, 16, 8), (64, 8, 8), (65, 8, 8)])
+def test_query_blocks_of_many_sequences(seqs, heads, kv_heads):
+    """Enough ragged sequences that keys are not split: the work-groups take
+    the query blocks by falling key end across sequences (up to 64 of them;
+    65 keep the order of the batch), empty sequences among them.  Every
+    block has to be computed exactly once: the outputs start as NaN where a
+    block is missed, and every row is compared."""
+    dtype, block = torch.bfloat16, 16
+    gen = torch.Generator().manual_seed(seqs)
+    new = torch.randint(0, 400, (seqs,), generator=gen).tolist()
+    new[3] = 0
+    prior = torch.randint(0, 900, (seqs,), generator=gen).tolist()
+    prior[5] = 0
+    args = paged_case(new, prior, block, heads, kv_heads, dtype, seed=seqs)
+    dev = [a.to(DEV) for a in args]
+    torch.full_like(dev[0], float("nan"))  # freed at once: the output's storage
+    actual = paged_prefill_attention(*dev, block, validate=False).float().cpu()
+    expected = paged_oracle.paged_prefill_attention(*args, block, cast=False)
+    assert (actual - expected).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens,start", [(64, 0), (65, 0), (1, 128), (130, 4300), (700, 33)])
+def test_dense_tiles_and_windows(dtype, tokens, start):
+    gen = torch.Generator().manual_seed(tokens + start)
+    q = torch.randn(1, 8, tokens, 128, generator=gen).to(dtype)
+    k = torch.randn(1, 4, start + tokens + 9, 128, generator=gen).to(dtype)
+    v = torch.randn(1, 4, start + tokens + 9, 128, generator=gen).to(dtype)
+    actual = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), query_start=start).float().cpu()
+    expected = paged_oracle.prefill_attention(q, k, v, query_start=start, cast=False)
+    assert (actual - expected).abs().max().item() <= GATE[dtype]
