@@ -1,4 +1,5 @@
-"""Build step of the HIP library: hipcc for gfx950 -> libmvme_paged.so (in-tree).
+"""Build step of the HIP library: hipcc for gfx950 -> libmvme_paged.so (in-tree),
+and of the Python entry points' native call path: g++ -> mvme_host.so.
 
 The reference JIT-builds its CUDA extension on first use
 (mini_engine/kernels/cuda_extension.py:14-66).  This package instead builds
@@ -24,6 +25,7 @@ SOURCE_DIR = PACKAGE_DIR.parent / "csrc"
 INCLUDE_DIR = PACKAGE_DIR.parents[1] / "include"
 LIB_DIR = PACKAGE_DIR / "_lib"
 LIB_NAME = "libmvme_paged.so"
+HOST_NAME = "mvme_host.so"
 ARCH = "gfx950"
 
 # Packed-FP32 VALU forms are disabled for every HIP translation unit; hipcc's
@@ -38,6 +40,25 @@ def library_path() -> Path:
     return LIB_DIR / LIB_NAME
 
 
+def host_path() -> Path:
+    return LIB_DIR / HOST_NAME
+
+
+def host_command(target: Path) -> list[str]:
+    """The compiler call for csrc/host_calls.cpp: a CPython module on torch's C++ API (host code only)."""
+    import sysconfig
+
+    import torch
+
+    torch_dir = Path(torch.__file__).resolve().parent
+    lib = torch_dir / "lib"
+    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f"-I{INCLUDE_DIR}", f"-I{torch_dir / 'include'}", f"-I{torch_dir / 'include/torch/csrc/api/include'}",
+            f"-I{sysconfig.get_paths()['include']}", str(SOURCE_DIR / "host_calls.cpp"), "-o", str(target),
+            f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{lib}"]
+
+
 def digest_path() -> Path:
     return LIB_DIR / "SOURCE_DIGEST"
 
@@ -48,7 +69,8 @@ def sources() -> list[Path]:
 
 def source_digest() -> str:
     digest = hashlib.sha256()
-    for path in sorted([*SOURCE_DIR.glob("*.hip"), *SOURCE_DIR.glob("*.h"), *INCLUDE_DIR.glob("*.h")]):
+    for path in sorted([*SOURCE_DIR.glob("*.hip"), *SOURCE_DIR.glob("*.cpp"), *SOURCE_DIR.glob("*.h"),
+                        *INCLUDE_DIR.glob("*.h")]):
         digest.update(path.name.encode())
         digest.update(path.read_bytes())
     return digest.hexdigest()
@@ -72,7 +94,7 @@ def _run(cmd: list[str]) -> None:
 
 
 def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
-    """Compile every csrc/*.hip for gfx950 and link libmvme_paged.so.
+    """Compile every csrc/*.hip for gfx950 and link libmvme_paged.so; build mvme_host.so beside it.
 
     Always recompiles (the build check must exercise the compiler).  The
     source digest is written next to the library; the loader refuses a
@@ -88,6 +110,8 @@ def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
         obj = build_dir / (src.stem + ".o")
         objects.append(obj)
         commands.append([hipcc, *HIP_FLAGS, f"-I{INCLUDE_DIR}", "-c", str(src), "-o", str(obj)])
+    host_tmp = host_path().with_suffix(".so.tmp")
+    commands.append(host_command(host_tmp))
     workers = jobs or min(len(commands), max(1, min(8, os.cpu_count() or 1)))
     with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as pool:
         for cmd, _ in zip(commands, pool.map(_run, commands)):
@@ -97,6 +121,7 @@ def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
     tmp = target.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objects)])
     os.replace(tmp, target)
+    os.replace(host_tmp, host_path())
     digest_path().write_text(source_digest() + "\n")
     return target
 

@@ -123,6 +123,8 @@ def write_kv_cache_slots(key_cache, value_cache, slot_mapping, key, value,
     may be strided views whose per-token [kv_heads, head_dim] rows are dense.
     """
     _backend(backend)
+    if not validate and ext.native_calls().write_slots(key_cache, value_cache, slot_mapping, key, value):
+        return
     if (key_cache.ndim != 4 or value_cache.shape != key_cache.shape
             or any(size <= 0 for size in key_cache.shape)
             or not key_cache.is_contiguous() or not value_cache.is_contiguous()):

@@ -20,6 +20,10 @@ MAX_ROWS = 64
 
 def linear_rows(x, weight, bias=None, *, out=None):
     """out[m] = x[m] @ weight.T (+ bias) for a 2-D ``x`` of at most 64 rows."""
+    if out is None:
+        result = ext.native_calls().linear(x, weight, bias)
+        if result is not None:
+            return result
     if not x.is_cuda or not weight.is_cuda:
         raise ValueError("HipLinear requires CUDA input and weights")
     if x.ndim != 2 or weight.ndim != 2 or x.shape[1] != weight.shape[1]:
@@ -61,6 +65,9 @@ class HipLinear(nn.Linear):
     backend = "hip"
 
     def forward(self, x):
+        result = ext.native_calls().linear(x, self.weight, self.bias)
+        if result is not None:
+            return result
         if not x.is_cuda or not self.weight.is_cuda:
             raise ValueError("HipLinear requires CUDA input and weights")
         original_shape = x.shape

@@ -81,6 +81,11 @@ def paged_attention(query, key_cache, value_cache, block_tables, context_lens, b
     """
     if backend != "hip":
         raise ValueError("decode backend must be hip")
+    if not validate and out is None and workspace is None:
+        result = ext.native_calls().decode(query, key_cache, value_cache, block_tables, context_lens, block_size,
+                                           partition_tokens)
+        if result is not None:
+            return result
     if query.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError("HIP paged attention supports FP16/BF16")
     _native_checks(query, key_cache, value_cache, block_tables, context_lens, block_size, validate)
@@ -134,11 +139,17 @@ def paged_attention_decode_write(query, key_cache, value_cache, block_tables, co
     shapes run the two launches above.  Returns the attention output
     ``[B, Hq, D]``.
     """
+    if backend != "hip":
+        raise ValueError("decode backend must be hip")
+    if not validate and out is None and workspace is None and q_out is None:
+        result = ext.native_calls().decode_write(query, key_cache, value_cache, block_tables, context_lens, block_size,
+                                                 new_key, new_value, q_weight, k_weight, cos, sin, eps,
+                                                 partition_tokens)
+        if result is not None:
+            return result
     from .data import _row_stride, write_kv_cache_batch
     from .rope import qk_norm_rope_write_kv
 
-    if backend != "hip":
-        raise ValueError("decode backend must be hip")
     if query.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError("HIP paged attention supports FP16/BF16")
     rope = q_weight is not None

@@ -46,6 +46,11 @@ def paged_prefill_attention(q, key_cache, value_cache, cu_seqlens_q, query_start
     """
     if backend != "hip":
         raise ValueError("paged prefill backend must be hip")
+    if not validate and workspace is None:
+        result = ext.native_calls().prefill(q, key_cache, value_cache, cu_seqlens_q, query_starts, block_tables,
+                                            context_lens, block_size, chunk_tokens)
+        if result is not None:
+            return result
     if (type(block_size) is not int or block_size <= 0 or key_cache.ndim != 4
             or value_cache.shape != key_cache.shape or key_cache.shape[1] != block_size
             or any(size <= 0 for size in key_cache.shape)
@@ -168,6 +173,10 @@ def prefill_attention(q, k, v, backend="hip", *, query_start=0, out=None, worksp
     """
     if backend != "hip":
         raise ValueError("unknown prefill backend")
+    if out is None and workspace is None:
+        result = ext.native_calls().dense(q, k, v, query_start)
+        if result is not None:
+            return result
     if (q.ndim != 4 or k.ndim != 4 or k.shape != v.shape or k.shape[1] == 0
             or q.shape[1] % k.shape[1]):
         raise ValueError("prefill expects [batch, heads, tokens, dim] and divisible GQA heads")

@@ -1,0 +1,141 @@
+"""The entry points' native call path against the Python path: every form it
+takes gives the same bits as the same call with caller-supplied buffers (which
+it leaves to the Python code), and it declines everything else."""
+
+import pytest
+import torch
+
+from mini_engine_hip.kernels import hip_extension as ext
+from mini_engine_hip.kernels.data import write_kv_cache_slots
+from mini_engine_hip.kernels.linear import linear_rows
+from mini_engine_hip.kernels.paged import paged_attention, paged_attention_decode_write
+from mini_engine_hip.kernels.prefill import paged_prefill_attention, prefill_attention
+from mini_engine_hip.kernels.rope import qk_norm_rope_write_kv
+
+DEV = "cuda"
+
+
+class Subclass(torch.Tensor):
+    pass
+
+
+def decode_args(device, dtype=torch.bfloat16, batch=3, heads=4, kv=2, dim=64, block=16, width=9):
+    gen = torch.Generator().manual_seed(7)
+    key, value = (torch.randn(batch * width + 2, block, kv, dim, generator=gen).to(dtype) for _ in range(2))
+    table = torch.randperm(batch * width + 2, generator=gen)[:batch * width].view(batch, width)
+    lens = torch.tensor([1 + 40 * i for i in range(batch)])
+    q = torch.randn(batch, heads, dim, generator=gen).to(dtype)
+    return [t.to(device) for t in (q, key, value, table, lens)] + [block]
+
+
+def test_declines_what_is_not_plain():
+    """CPU tensors, subclasses, wrong argument types: None, and no error."""
+    native = ext.native_calls()
+    args = decode_args("cpu")
+    assert native.decode(*args, 0) is None
+    assert native.decode(*args[:5], 16.0, 0) is None
+    assert native.decode(args[0].as_subclass(Subclass), *args[1:], 0) is None
+    assert native.decode(None, *args[1:], 0) is None
+    assert native.decode() is None
+    q, k, v = (torch.zeros(1, 2, 4, 64) for _ in range(3))
+    assert native.dense(q, k, v, 0) is None
+    assert native.linear(torch.zeros(2, 64), torch.zeros(32, 64), None) is None
+    with pytest.raises(RuntimeError, match="must be CUDA"):
+        paged_attention(*args, validate=False)
+
+
+def test_bind_refuses_a_wrong_library():
+    with pytest.raises(ValueError):
+        ext.native_calls().bind(len, (1, 2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim", [64, 80, 128])
+@pytest.mark.parametrize("partition", [0, 64, -1])
+def test_decode_equals_the_python_path(dtype, dim, partition):
+    args = decode_args(DEV, dtype, dim=dim)
+    assert ext.native_calls().decode(*args, partition) is not None
+    out = torch.empty_like(args[0])
+    paged_attention(*args, validate=False, partition_tokens=partition, out=out)
+    assert torch.equal(paged_attention(*args, validate=False, partition_tokens=partition), out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("layout", ["split", "dense", "misaligned"])
+def test_decode_write_equals_the_python_path(rope, layout):
+    dtype, heads, kv, dim = torch.bfloat16, 4, 2, 64
+    base, key, value, table, lens, block = decode_args(DEV, dtype)
+    gen = torch.Generator().manual_seed(3)
+    qkv = torch.randn(3, heads + 2 * kv, dim, generator=gen).to(dtype).to(DEV)
+    q, nk, nv = qkv.split([heads, kv, kv], dim=1)
+    if layout != "split" or not rope:
+        q = q.contiguous()
+    if layout != "split":
+        nk, nv = nk.contiguous(), nv.contiguous()
+    if layout == "misaligned":  # 2-byte offset: the two launches of the Python path
+        nk = torch.cat([nk.flatten()[:1], nk.flatten()])[1:].view(nk.shape)
+        assert nk.data_ptr() % 16 != 0
+    cos, sin = torch.rand(3, dim // 2, generator=gen).to(dtype).to(DEV), torch.rand(3, dim // 2, generator=gen).to(dtype).to(DEV)
+    weight = torch.rand(dim, generator=gen).to(dtype).to(DEV)
+    extra = dict(q_weight=weight, k_weight=weight, cos=cos, sin=sin) if rope else {}
+    k1, v1, k2, v2 = key.clone(), value.clone(), key.clone(), value.clone()
+    out = torch.empty(3, heads, dim, dtype=dtype, device=DEV)
+    paged_attention_decode_write(q, k1, v1, table, lens, block, nk, nv, validate=False, out=out, **extra)
+    got = paged_attention_decode_write(q, k2, v2, table, lens, block, nk, nv, validate=False, **extra)
+    assert torch.equal(got, out) and torch.equal(k1, k2) and torch.equal(v1, v2)
+    values = [extra.get(n) for n in ("q_weight", "k_weight", "cos", "sin")]
+    taken = ext.native_calls().decode_write(q, k2, v2, table, lens, block, nk, nv, *values, 1e-6, 0) is not None
+    assert taken == (layout != "misaligned")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("new", [[5, 40], [300, 1]])
+def test_prefill_write_and_rope_equal_the_python_path(new):
+    dtype, heads, kv, dim, block = torch.float16, 4, 2, 128, 16
+    gen = torch.Generator().manual_seed(new[0])
+    tokens, starts = sum(new), torch.tensor([100, 0])
+    lens = starts + torch.tensor(new)
+    width = -(-int(lens.max()) // block)
+    key, value = (torch.randn(2 * width, block, kv, dim, generator=gen).to(dtype).to(DEV) for _ in range(2))
+    table = torch.randperm(2 * width, generator=gen).view(2, width)
+    slots = torch.cat([table[i, p // block] * block + p % block
+                       for i in range(2) for p in [torch.arange(starts[i], lens[i])]]).to(DEV)
+    cu = torch.tensor([0, new[0], tokens]).to(DEV)
+    table, starts, lens = table.to(DEV), starts.to(DEV), lens.to(DEV)
+    q, k, v = torch.randn(tokens, heads + 2 * kv, dim, generator=gen).to(dtype).to(DEV).split([heads, kv, kv], dim=1)
+    cos, sin = torch.rand(2, tokens, dim // 2, generator=gen).to(dtype).to(DEV)
+    weight = torch.rand(dim, generator=gen).to(dtype).to(DEV)
+    caches = [[key.clone(), value.clone()] for _ in range(2)]
+    out = torch.empty(tokens, heads, dim, dtype=dtype, device=DEV)
+    rope = lambda c, **kw: qk_norm_rope_write_kv(q, k, v, weight, weight, cos, sin, *c, slot_mapping=slots,  # noqa: E731
+                                                 validate=False, **kw)
+    assert torch.equal(rope(caches[0]), rope(caches[1], out=out))
+    write_kv_cache_slots(*caches[0], slots, k, v, validate=False)
+    write_kv_cache_slots(*caches[1], slots, k, v)
+    assert all(torch.equal(a, b) for a, b in zip(*caches))
+    args = (out, *caches[0], cu, starts, table, lens, block)
+    workspace = torch.empty(1 << 24, dtype=torch.uint8, device=DEV)
+    assert torch.equal(paged_prefill_attention(*args, validate=False),
+                       paged_prefill_attention(*args, validate=False, workspace=workspace))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,view", [(128, True), (128, False), (64, True), (100, False)])
+def test_dense_and_linear_equal_the_python_path(dim, view):
+    gen = torch.Generator().manual_seed(dim)
+    make = lambda n, h: (torch.randn(n, h, dim, generator=gen).bfloat16().to(DEV).transpose(0, 1).unsqueeze(0))  # noqa: E731
+    q, k, v = make(70, 4), make(90, 2), make(90, 2)
+    if not view:
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    out = torch.empty(1, 4, 70, dim, dtype=q.dtype, device=DEV)
+    result = prefill_attention(q, k, v, query_start=20)
+    assert torch.equal(result, prefill_attention(q, k, v, query_start=20, out=out))
+    assert result.stride() == (70 * 4 * dim, dim, 4 * dim, 1)
+    x, weight = torch.randn(7, 512, generator=gen).bfloat16().to(DEV), torch.randn(64, 512, generator=gen).bfloat16().to(DEV)
+    bias = torch.randn(64, generator=gen).bfloat16().to(DEV)
+    for b in (None, bias):
+        buffer = torch.empty(7, 64, dtype=x.dtype, device=DEV)
+        assert torch.equal(linear_rows(x, weight, b), linear_rows(x, weight, b, out=buffer))
+    assert torch.equal(linear_rows(x[:, ::1][:3], weight), linear_rows(x, weight)[:3])
