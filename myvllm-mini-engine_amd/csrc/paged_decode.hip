@@ -1,6 +1,7 @@
 // GQA paged decode attention for gfx950: launch plan, split-K merge and
 // the C entry points.  The attention kernel and its design notes are in
 // paged_decode_kernel.h.
+#include <algorithm>
 #include <mutex>
 
 #include "paged_decode_kernel.h"
@@ -255,6 +256,83 @@ __global__ __launch_bounds__(kLptMax) void paged_decode_flat_merge_kernel(Decode
     for (int i = 0; i < 4; ++i) out[i] = T::from_float(sum > 0.f ? o[i] / sum : 0.f);
 }
 
+// Merge of even parts: one work-group per (sequence, query head).  The
+// partition length is recomputed from the lengths as the attention kernel
+// did; a sequence's rows lie one slot (a.kv_heads * a.gtiles work-groups of G
+// rows) apart.  kThreads / D groups of threads take every kGroups-th
+// partition, kBatch at a time with a running reference, and meet in LDS.
+template <typename T, int D, int G>
+__global__ __launch_bounds__(256) void paged_decode_even_merge_kernel(DecodeArgs a) {
+    constexpr int kGroups = 256 / D, kBatch = 8;
+    __shared__ float sm[kGroups > 1 ? kGroups : 1][3][D];
+    const int b = blockIdx.x / a.q_heads, h = blockIdx.x - b * a.q_heads;
+    const EvenParts e = even_parts(a, DecodeShape<D>::kTpi * kSplitWaves);
+    const int n = lane_value(e.count, b);
+    if (n == 1) return;  // written directly by the attention kernel
+    const int slot0 = lane_value(e.incl, b) - n;
+    const int kvh = h / a.group, hg = h - kvh * a.group;
+    const int tile = hg / a.tile_heads;
+    const int cols = a.kv_heads * a.gtiles;
+    const int64_t row0 = ((int64_t)slot0 * cols + kvh * a.gtiles + tile) * G + (hg - tile * a.tile_heads);
+    const int64_t stride = (int64_t)cols * G;
+    const int grp = threadIdx.x / D, d = threadIdx.x - grp * D;
+    float mx = kNegInf, sum = 0.f, o = 0.f;
+    if (grp < kGroups) {
+        for (int p0 = grp; p0 < n; p0 += kBatch * kGroups) {
+            float m[kBatch], l[kBatch], v[kBatch];
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const int64_t row = row0 + min(p0 + k * kGroups, n - 1) * stride;
+                m[k] = a.ws_ml[2 * row];
+                l[k] = a.ws_ml[2 * row + 1];
+                v[k] = a.ws_acc[row * D + d];
+            }
+            float bm = mx;
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                if (p0 + k * kGroups >= n) m[k] = kNegInf;
+                bm = fmaxf(bm, m[k]);
+            }
+            const float ref = bm == kNegInf ? 0.f : bm;
+            const float old = fast_exp2(mx - ref);
+            sum *= old;
+            o *= old;
+            mx = bm;
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const float w = p0 + k * kGroups < n ? fast_exp2(m[k] - ref) : 0.f;
+                sum += p0 + k * kGroups < n ? l[k] * w : 0.f;
+                o += p0 + k * kGroups < n ? v[k] * w : 0.f;
+            }
+        }
+    }
+    if constexpr (kGroups > 1) {
+        if (grp < kGroups) {
+            sm[grp][0][d] = mx;
+            sm[grp][1][d] = sum;
+            sm[grp][2][d] = o;
+        }
+        __syncthreads();
+        if (grp > 0) return;
+        float all = mx;
+#pragma unroll
+        for (int g = 1; g < kGroups; ++g) all = fmaxf(all, sm[g][0][d]);
+        const float ref = all == kNegInf ? 0.f : all;
+        const float own = fast_exp2(mx - ref);
+        sum *= own;
+        o *= own;
+#pragma unroll
+        for (int g = 1; g < kGroups; ++g) {
+            const float w = fast_exp2(sm[g][0][d] - ref);
+            sum += sm[g][1][d] * w;
+            o += sm[g][2][d] * w;
+        }
+    } else if (grp > 0) {
+        return;
+    }
+    static_cast<uint16_t*>(a.out)[(int64_t)blockIdx.x * D + d] = T::from_float(sum > 0.f ? o / sum : 0.f);
+}
+
 struct DecodePlan {
     int partition;
     int max_parts;
@@ -264,6 +342,8 @@ struct DecodePlan {
     int waves;  // waves per work-group (kSplitWaves or kWholeWaves; kFlatWaves in the walk)
     bool stream;  // non-temporal K/V loads
     int flat_groups;  // > 0: balanced walk with this many work-groups
+    int even_slots;   // > 0: even parts, work-groups per column
+    int even_min;     // shortest part
 };
 
 
@@ -306,6 +386,30 @@ void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim) {
     p.gtile = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
     p.gtiles = (int)(group / p.gtile);
     p.tile_heads = p.gtile;
+}
+
+constexpr int64_t kEvenCapacity = 2048;
+
+// Partition length of a split over tiles of 2 to 4 heads of 128: the number of
+// partitions n that minimises the iterations the busiest CU runs, half at full
+// tables and half at tables filled a little over half (ragged batches), plus
+// a share per partition for its start, its end and the merge.  A target of two
+// work-groups per CU alone leaves some CUs with three and others with two: 24
+// sequences of 2048, 8 kv heads (192 units): 3 partitions 42.9 us (26.7 for
+// U[1,2048]), 4 partitions -- three per CU -- 36.5 (22.1).
+int64_t split_partition(int64_t cap, int64_t units, int64_t step) {
+    const int64_t steps = (cap + step - 1) / step;
+    int64_t best = 1;
+    double best_cost = 1e300;
+    for (int64_t n = 2; n <= 32 && n <= steps; ++n) {
+        const int64_t iterations = (steps + n - 1) / n;
+        const double groups = (double)(units * n);
+        const double full = (double)((units * n + kDeviceCUs - 1) / kDeviceCUs);
+        const double ragged = std::max(1.0, 0.55 * groups / (double)kDeviceCUs);
+        const double cost = 0.5 * (full + ragged) * (double)iterations + 0.15 * (double)n;
+        if (cost < best_cost) best_cost = cost, best = n;
+    }
+    return (steps + best - 1) / best * step;
 }
 
 // Host-side plan (lengths stay on the device, so it depends on the table
@@ -359,9 +463,13 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
         p.waves = kSplitWaves;
         if (requested > 0) {
             part = requested;
+        } else if (group >= 2 && group <= 4 && head_dim == 128) {
+            part = split_partition(cap, units, split_step);
         } else {
-            constexpr int64_t kTargetGroups = 2 * kDeviceCUs;
-            part = (cap * units + kTargetGroups - 1) / kTargetGroups;
+            // Wide tiles of 64 dims gain from more and shorter partitions: 14/2 heads, 60 sequences
+            // U[1,1300] 22.2 -> 16.5 at 128 keys, 20 of U[1,4000] 22.6 -> 17.6.
+            const int64_t target = head_dim == 64 && p.gtile == 8 ? 5 * kDeviceCUs : 2 * kDeviceCUs;
+            part = (cap * units + target - 1) / target;
         }
         part = (part + split_step - 1) / split_step * split_step;
         const int64_t cap_steps = (cap + split_step - 1) / split_step * split_step;
@@ -386,12 +494,30 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
     // (64 sequences U[1,4096] sharing a 1024-token prefix, bf16, block 16:
     // 88.1 -> 90.5 µs; 128 sequences U[1,4096]: 166.4 -> 169.2).
     const bool long_units = (double)cap * (double)head_dim * 4.0 >= (double)kLongUnitBytes;
-    const bool flat = batch <= kLptMax &&
+    // Even parts: 8-head tiles over tables of 2048 tokens and more.
+    const bool even = requested <= 0 && requested != -1 && !whole && p.gtile == 8 && head_dim == 128 && batch <= kWave &&
+                      cap >= kEvenCapacity;
+    if (even) {
+        p.even_slots = (int)(kEvenGroups / (kv_heads * p.gtiles));
+        p.even_min = (int)(4 * split_step);
+        p.max_parts = 1;
+    }
+    const bool flat = !even && batch <= kLptMax &&
                       (requested == -1 || (requested <= 0 && long_units && units <= kDeviceCUs));
     if (flat) {
         p.flat_groups = kFlatGroups;
         p.waves = kFlatWaves;
         p.max_parts = 1;
+    }
+    // Pairs of heads: the matrix cores' loop, which keeps loads in flight,
+    // where several work-groups share a CU (16/8 heads, pages of 16: 64 sequences U[1,4096] 94.5 -> 91.5 us, 16 of
+    // U[1,1024] 13.2 -> 12.5, 8 of 512 8.9 -> 8.6; one 8-wave work-group per CU
+    // or the walk has no use for it: 32 of 2048 44.6 -> 45.8, walk of 32 of
+    // U[1,4096] 51.7 -> 54.0.)
+    if (group == 2 && (head_dim == 64 || head_dim == 128) && !flat &&
+        (p.max_parts > 1 || (p.waves == kWholeWaves && units > kDeviceCUs))) {
+        p.gtile = 4;
+        p.tile_heads = 2;
     }
     // In floating point: the size query runs before any shape check, where the
     // integer product could overflow.  The walk's kernels always load with the
@@ -413,7 +539,10 @@ void launch_decode_kernel_pro(const DecodeArgs& a, dim3 grid, bool page_uniform,
 
 template <typename T, int D, int G, int NW>
 void launch_decode_nw(const DecodeArgs& a, int units, bool page_uniform, bool stream, hipStream_t s) {
-    const dim3 grid(a.flat_groups > 0 ? a.flat_groups : units, a.max_parts);
+    const dim3 grid(a.flat_groups > 0  ? a.flat_groups
+                    : a.even_slots > 0 ? a.even_slots * a.kv_heads * a.gtiles
+                                       : units,
+                    a.max_parts);
     if (stream) {
         launch_decode_kernel_pro<T, D, G, NW, true>(a, grid, page_uniform, s);
         return;
@@ -425,6 +554,12 @@ template <typename T, int D, int G>
 void launch_decode(const DecodeArgs& a, const DecodePlan& p, int units, bool page_uniform, hipStream_t s) {
     if (p.waves == kWholeWaves) launch_decode_nw<T, D, G, kWholeWaves>(a, units, page_uniform, p.stream, s);
     else launch_decode_nw<T, D, G, kSplitWaves>(a, units, page_uniform, p.stream, s);
+    if constexpr (even_tile<D, G>()) {
+        if (a.even_slots > 0) {
+            hipLaunchKernelGGL((paged_decode_even_merge_kernel<T, D, G>), dim3(a.batch * a.q_heads), dim3(256), 0, s, a);
+            return;
+        }
+    }
     if (a.flat_groups > 0)
         hipLaunchKernelGGL((paged_decode_flat_merge_kernel<T, D, G>), dim3(a.flat_groups), dim3(kLptMax), 0, s, a);
     else if (a.max_parts > 1)
@@ -501,6 +636,8 @@ extern "C" size_t mvme_paged_attention_workspace_size(int64_t batch, int64_t q_h
     if (p.flat_groups > 0)
         return (size_t)p.flat_groups * 2 * p.gtile * (head_dim + 2) * sizeof(float) +
                (size_t)p.flat_groups * sizeof(FlatMergeDesc);
+    if (p.even_slots > 0)
+        return (size_t)p.even_slots * kv_heads * p.gtiles * p.gtile * (head_dim + 2) * sizeof(float);
     if (p.max_parts <= 1) return 0;
     return (size_t)batch * q_heads * p.max_parts * (head_dim + 2) * sizeof(float);
 }
@@ -542,7 +679,8 @@ int launch_paged_attention(void* out, const void* query, const void* key_cache, 
     a.lens = context_lens;
     if (need > 0) {
         a.ws_acc = static_cast<float*>(workspace);
-        a.ws_ml = a.ws_acc + (p.flat_groups > 0 ? (int64_t)p.flat_groups * 2 * p.gtile
+        a.ws_ml = a.ws_acc + (p.flat_groups > 0  ? (int64_t)p.flat_groups * 2 * p.gtile
+                              : p.even_slots > 0 ? (int64_t)p.even_slots * kv_heads * p.gtiles * p.gtile
                                                  : batch * q_heads * p.max_parts) * head_dim;
         // After the partial rows (a multiple of 16 bytes: 256 shares x 2 x G
         // x (D + 2) floats).
@@ -564,7 +702,9 @@ int launch_paged_attention(void* out, const void* query, const void* key_cache, 
     a.capacity = (int)(table_width * block_size);
     a.partition = p.partition;
     a.max_parts = p.max_parts;
-    a.lpt_batch = p.flat_groups == 0 && p.max_parts == 1 && batch >= 2 && batch <= kLptMax ? (int)batch : 0;
+    a.even_slots = p.even_slots;
+    a.even_min = p.even_min;
+    a.lpt_batch = p.flat_groups == 0 && p.even_slots == 0 && p.max_parts == 1 && batch >= 2 && batch <= kLptMax ? (int)batch : 0;
     // Two 8-wave work-groups per CU hold every unit at once (units in
     // (CUs, 2 CUs]): pair long sequences with short ones.  Longest first
     // alone put the k-th and the (k + batch/2)-th longest on one CU: 64

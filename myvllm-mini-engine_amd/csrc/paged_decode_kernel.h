@@ -131,6 +131,11 @@ struct DecodeArgs {
     // token chunks.
     int flat_groups;
     int batch;
+    // Even parts (even_slots > 0, batch <= 64): split-K whose partition length
+    // the lengths decide; even_slots work-groups per column, even_min tokens
+    // at least.
+    int even_slots;
+    int even_min;
     float scale_log2;
     // Fused prologue: 0 none; 1 write new_k / new_v rows at position len - 1;
     // 2 RMSNorm + RoPE of the query heads (query = raw rows, q_stride apart)
@@ -227,6 +232,43 @@ static_assert(kFlatGroups <= kLptMax, "one merge thread per piece");
 // First chunk of logical work-group l's share.
 __device__ inline int64_t flat_share_start(int64_t l, int64_t total) { return (l * total) >> kFlatShift; }
 
+// Even parts: the split of a ragged batch, decided on the device.  A partition
+// length sized by the tables' capacity leaves most of a ragged batch's
+// partitions empty or short and the CUs with unequal work.  Here a column (a
+// kv head's query tile, across the sequences) has `even_slots` work-groups, and
+// the length is the smallest with which its partitions fit them whatever
+// their remainders: T / (slots - batch) tokens, T the column's tokens.  Slot j
+// of a column takes the j-th partition, sequence by sequence.  One wave holds
+// the batch, a sequence per lane: a scan and a ballot, no barrier.
+//
+// us per call, capacity-sized split or walk -> even parts (bf16, pages of 16):
+// 32/4 heads, 16 sequences U[1,8192] 40.7 -> 34.2, all 8192 53.6 -> 52.9, 12
+// of U[1,2048] 15.1 -> 13.8; 28/4 heads, 24 of U[1,4096] 30.1 -> 25.1, all
+// 4096 46.3 -> 43.3, 1 of 8192 21.7 -> 13.8.  The scan costs about 0.7 us per
+// launch: tables below 2048 tokens keep the split (40/8 heads, 12 of
+// U[1,1200] 15.6 against 16.9), and so do narrower tiles, whose work-groups
+// are not bound by how many fit a CU (32/8 heads, 8 of 2048 16.2 against 17.9;
+// 16/8, 16 of U[1,1024] 12.6 against 13.8).
+template <int D, int G>
+constexpr bool even_tile() { return D == 128 && G == 8; }
+constexpr int kEvenGroups = 512;  // work-groups: two of 4 waves per CU, what the 8-head tile's registers hold
+struct EvenParts {
+    int len, count, incl, part;  // lane b: its sequence's tokens, partitions, inclusive prefix; uniform length
+};
+__device__ inline EvenParts even_parts(const DecodeArgs& a, int step) {
+    const int lane = __lane_id();
+    EvenParts e;
+    e.len = lane < a.batch ? seq_tokens(a.lens[lane], a.capacity) : 0;
+    // At most 64 sequences of 2^20 tokens: the sum fits 32 bits.
+    const int total = lane_value(wave_incl_scan(e.len), kWave - 1);
+    const int room = a.even_slots - a.batch;
+    const int want = max((total + room - 1) / room, a.even_min);
+    e.part = (want + step - 1) / step * step;
+    e.count = lane < a.batch ? max((e.len + e.part - 1) / e.part, 1) : 0;
+    e.incl = wave_incl_scan(e.count);
+    return e;
+}
+
 constexpr float kRaise = 8.f;  // binary orders a score may exceed the running reference by (matrix tiles)
 
 // Value of lane i ^ 4 (the half-row mirror, then each quad reversed).
@@ -275,6 +317,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
     constexpr int L = kDecodeLoads;
     constexpr int kStep = S::kTpi * NW;  // tokens per work-group iteration
     constexpr bool MM = matrix_tile<D, G>();
+    constexpr bool EVEN = even_tile<D, G>() && NW == kSplitWaves && !FLAT;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int tl = lane / S::kLpt;  // token slot inside one load
@@ -283,7 +326,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
     const int li = lane & 15, lg = lane >> 4;  // matrix operand column / row and k-group
 
     const int unit = blockIdx.x;
-    const int part = blockIdx.y;
+    int part = blockIdx.y;
     const int per_seq = a.kv_heads * a.gtiles;
     // The segment this work-group computes: tokens [start, end) of the unit
     // (sequence b, column r = kv head * gtiles + query-head tile); `direct`
@@ -349,7 +392,17 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
     } else {
         b = unit / per_seq;
         r = unit - b * per_seq;
-        if (a.lpt_batch > kWave) {
+        int partition = a.partition;
+        if (EVEN && a.even_slots > 0) {
+            const EvenParts e = even_parts(a, kStep);
+            // b: slot of the column.
+            if (b >= lane_value(e.incl, kWave - 1)) return;
+            const int slot = b;
+            b = __builtin_ctzll(__ballot(e.incl > slot));
+            part = slot - (lane_value(e.incl, b) - lane_value(e.count, b));
+            len = lane_value(e.len, b);
+            partition = e.part;
+        } else if (a.lpt_batch > kWave) {
             // As below for 64 < batch <= kLptMax: thread s keeps sequence s's key
             // in LDS and counts the larger keys with broadcast reads.
             __shared__ int lpt_keys[kLptMax];
@@ -404,10 +457,10 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             early_page(b);
             len = seq_tokens(a.lens[b], a.capacity);
         }
-        const int nparts = len > 0 ? (len + a.partition - 1) / a.partition : 1;
+        const int nparts = len > 0 ? (len + partition - 1) / partition : 1;
         if (part >= nparts) return;
-        start = part * a.partition;
-        end = min(start + a.partition, len);
+        start = part * partition;
+        end = min(start + partition, len);
         direct = nparts == 1;
     }
 
@@ -426,6 +479,97 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         const int h0 = kvh * a.group + tile0;
         // Heads of this tile.  Without matrix cores tiles are always full.
         const int heads = MM ? min(a.tile_heads, a.group - tile0) : G;
+
+        const int64_t row_elems = (int64_t)a.kv_heads * D;
+        const int64_t page_elems = (int64_t)a.block_size * row_elems;
+        const uint16_t* kbase = static_cast<const uint16_t*>(a.key_cache) + kvh * D + 8 * c;
+        const uint16_t* vbase = static_cast<const uint16_t*>(a.value_cache) + kvh * D + 8 * c;
+        const int64_t* table = a.tables + (int64_t)b * a.table_width;
+
+        // Page-uniform iterations: the iteration's tokens lie in one page, whose
+        // id is a scalar load issued one iteration ahead (its latency hides
+        // behind the current iteration); the loads are a scalar page base plus
+        // 32-bit per-lane offsets, with no per-load branches.
+        const const_i64* ctable = (const const_i64*)table;
+        const int row_bytes = (int)(row_elems * 2);
+        uint32_t lane_off[L];
+#pragma unroll
+        for (int u = 0; u < L; ++u) lane_off[u] = (uint32_t)((u * S::kTpl + tl) * row_bytes + (kvh * D + 8 * c) * 2);
+        // Matrix tiles: K load u of lane li brings chunk kParts * lg + part of
+        // token u * kTpl + key_tok.
+        const int key_tok = li / S::kParts;
+        const int key_dim = 8 * (S::kParts * lg + li % S::kParts);
+        const uint32_t key_off = (uint32_t)(key_tok * row_bytes + (kvh * D + key_dim) * 2);
+        auto page_of = [&](int t) __attribute__((always_inline)) -> int64_t {
+            if (t >= end) return -1;
+            return ctable[a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size];
+        };
+        int it = __builtin_amdgcn_readfirstlane(start + wave * S::kTpi);
+        int64_t page_next = 0;
+        if constexpr (PAGE_UNIFORM) page_next = !FLAT && a.lpt_batch == 0 && !(EVEN && a.even_slots > 0) ? first_page : page_of(it);
+        // The next iteration's rows are loaded into the registers as soon as
+        // the products have read them: K right after the score products,
+        // V load by load, so that their latency overlaps the softmax and
+        // the output products.  No load is skipped (a branch around one
+        // would make the compiler wait for all of them): past the segment
+        // or without a page the loads read page 0's first rows, and `lim`
+        // masks what they bring.
+        u32x4 mk[MM ? L : 1], mv[MM ? L : 1];
+        int next_lim = 0;  // page-uniform: rows of the iteration at or past it are absent
+        int64_t next_base = 0;
+        bool next_ok[L];
+        auto row_of = [&](int t) __attribute__((always_inline)) -> int64_t {
+            int64_t page = -1;
+            if (t < end) page = table[t / a.block_size];
+            return page >= 0 && page < a.num_blocks ? page * page_elems + (int64_t)(t % a.block_size) * row_elems
+                                                    : (int64_t)-1;
+        };
+        auto fetch_page = [&](int t0) __attribute__((always_inline)) {
+            if constexpr (PAGE_UNIFORM) {
+                const int64_t page = page_next;
+                page_next = page_of(t0 + kStep);
+                const bool page_ok = page >= 0 && page < a.num_blocks;
+                const int in_page = a.block_shift >= 0 ? t0 & (a.block_size - 1) : t0 % a.block_size;
+                next_base = page_ok ? (page * a.block_size + in_page) * (int64_t)row_bytes : 0;
+                next_lim = page_ok ? end : 0;
+            }
+        };
+        auto fetch_k = [&](int t0) __attribute__((always_inline)) {
+            if constexpr (PAGE_UNIFORM) {
+                const uint8_t* kp = static_cast<const uint8_t*>(a.key_cache) + next_base;
+#pragma unroll
+                for (int u = 0; u < L; ++u)
+                    mk[MM ? u : 0] = kv_load<STREAM>(kp + (key_off + (uint32_t)(u * S::kTpl * row_bytes)));
+            } else {
+#pragma unroll
+                for (int u = 0; u < L; ++u) {
+                    const int64_t row = row_of(t0 + u * S::kTpl + key_tok);
+                    mk[MM ? u : 0] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
+                        static_cast<const uint16_t*>(a.key_cache) + (row >= 0 ? row : 0) + kvh * D + key_dim));
+                }
+            }
+        };
+        auto fetch_v = [&](int t0, int u) __attribute__((always_inline)) {
+            if constexpr (PAGE_UNIFORM) {
+                mv[MM ? u : 0] = kv_load<STREAM>(static_cast<const uint8_t*>(a.value_cache) + next_base + lane_off[u]);
+            } else {
+                const int64_t row = row_of(t0 + u * S::kTpl + tl);
+                next_ok[u] = row >= 0;
+                mv[MM ? u : 0] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
+                    static_cast<const uint16_t*>(a.value_cache) + (row >= 0 ? row : 0) + kvh * D + 8 * c));
+            }
+        };
+        // The first iteration's loads go out before the prologue and the
+        // query's: their latency overlaps the norm and the rotation (16/8
+        // heads: a 28-layer step of 16 sequences 849 -> 822 us, a step of 8
+        // of 512 10.1 -> 9.6).
+        if constexpr (MM)
+            if (it < end) {
+                fetch_page(it);
+                fetch_k(it);
+#pragma unroll
+                for (int u = 0; u < L; ++u) fetch_v(it, u);
+            }
 
         static_assert(!PRO || (S::kLpt == S::kChunks && S::kLpt >= 2), "prologue needs head_dim 16/32/64/128/256");
         // Fused prologue, with no barrier: the wave whose iterations hold the new
@@ -491,6 +635,16 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             }
         }
 
+        // The first iteration holds the new row: load it again once the owner's
+        // store has completed.
+        if constexpr (PRO && MM)
+            if (owner && it <= pos && pos < it + S::kTpi) {
+                __builtin_amdgcn_s_waitcnt(0);
+                fetch_k(it);
+#pragma unroll
+                for (int u = 0; u < L; ++u) fetch_v(it, u);
+            }
+
         // Query operands.  Matrix tiles: column li of the score product.
         // Otherwise: this lane's 8 elements of every head of the tile.
         constexpr int kStates = MM ? matrix_states<D, G>() : G;
@@ -544,92 +698,10 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 for (int e = 0; e < 8; ++e) macc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
-        const int64_t row_elems = (int64_t)a.kv_heads * D;
-        const int64_t page_elems = (int64_t)a.block_size * row_elems;
-        const uint16_t* kbase = static_cast<const uint16_t*>(a.key_cache) + kvh * D + 8 * c;
-        const uint16_t* vbase = static_cast<const uint16_t*>(a.value_cache) + kvh * D + 8 * c;
-        const int64_t* table = a.tables + (int64_t)b * a.table_width;
-
-        // Page-uniform iterations: the iteration's tokens lie in one page, whose
-        // id is a scalar load issued one iteration ahead (its latency hides
-        // behind the current iteration); the loads are a scalar page base plus
-        // 32-bit per-lane offsets, with no per-load branches.
-        const const_i64* ctable = (const const_i64*)table;
-        const int row_bytes = (int)(row_elems * 2);
-        uint32_t lane_off[L];
-#pragma unroll
-        for (int u = 0; u < L; ++u) lane_off[u] = (uint32_t)((u * S::kTpl + tl) * row_bytes + (kvh * D + 8 * c) * 2);
-        // Matrix tiles: K load u of lane li brings chunk kParts * lg + part of
-        // token u * kTpl + key_tok.
-        const int key_tok = li / S::kParts;
-        const int key_dim = 8 * (S::kParts * lg + li % S::kParts);
-        const uint32_t key_off = (uint32_t)(key_tok * row_bytes + (kvh * D + key_dim) * 2);
-        auto page_of = [&](int t) __attribute__((always_inline)) -> int64_t {
-            if (t >= end) return -1;
-            return ctable[a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size];
-        };
-        int it = __builtin_amdgcn_readfirstlane(start + wave * S::kTpi);
-        int64_t page_next = 0;
-        if constexpr (PAGE_UNIFORM) page_next = !FLAT && a.lpt_batch == 0 ? first_page : page_of(it);
         if constexpr (MM) {
-            // The next iteration's rows are loaded into the registers as soon as
-            // the products have read them: K right after the score products,
-            // V load by load, so that their latency overlaps the softmax and
-            // the output products.  No load is skipped (a branch around one
-            // would make the compiler wait for all of them): past the segment
-            // or without a page the loads read page 0's first rows, and `lim`
-            // masks what they bring.
-            u32x4 kk[L], vv[L];
-            int lim = 0, next_lim = 0;  // page-uniform: rows of the iteration at or past it are absent
-            int64_t next_base = 0;
-            bool ok[L], next_ok[L];
-            auto row_of = [&](int t) __attribute__((always_inline)) -> int64_t {
-                int64_t page = -1;
-                if (t < end) page = table[t / a.block_size];
-                return page >= 0 && page < a.num_blocks ? page * page_elems + (int64_t)(t % a.block_size) * row_elems
-                                                        : (int64_t)-1;
-            };
-            auto fetch_k = [&](int t0) __attribute__((always_inline)) {
-                // The owner's store of the new row completes before the row is read.
-                if constexpr (PRO)
-                    if (owner && t0 <= pos && pos < t0 + S::kTpi) __builtin_amdgcn_s_waitcnt(0);
-                if constexpr (PAGE_UNIFORM) {
-                    const int64_t page = page_next;
-                    page_next = page_of(t0 + kStep);
-                    const bool page_ok = page >= 0 && page < a.num_blocks;
-                    const int in_page = a.block_shift >= 0 ? t0 & (a.block_size - 1) : t0 % a.block_size;
-                    next_base = page_ok ? (page * a.block_size + in_page) * (int64_t)row_bytes : 0;
-                    next_lim = page_ok ? end : 0;
-                    const uint8_t* kp = static_cast<const uint8_t*>(a.key_cache) + next_base;
-#pragma unroll
-                    for (int u = 0; u < L; ++u)
-                        kk[u] = kv_load<STREAM>(kp + (key_off + (uint32_t)(u * S::kTpl * row_bytes)));
-                } else {
-#pragma unroll
-                    for (int u = 0; u < L; ++u) {
-                        const int64_t row = row_of(t0 + u * S::kTpl + key_tok);
-                        kk[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
-                            static_cast<const uint16_t*>(a.key_cache) + (row >= 0 ? row : 0) + kvh * D + key_dim));
-                    }
-                }
-            };
-            auto fetch_v = [&](int t0, int u) __attribute__((always_inline)) {
-                if constexpr (PAGE_UNIFORM) {
-                    vv[u] = kv_load<STREAM>(static_cast<const uint8_t*>(a.value_cache) + next_base + lane_off[u]);
-                } else {
-                    const int64_t row = row_of(t0 + u * S::kTpl + tl);
-                    next_ok[u] = row >= 0;
-                    vv[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
-                        static_cast<const uint16_t*>(a.value_cache) + (row >= 0 ? row : 0) + kvh * D + 8 * c));
-                }
-            };
-            if (it < end) {
-                fetch_k(it);
-#pragma unroll
-                for (int u = 0; u < L; ++u) fetch_v(it, u);
-            }
             for (; it < end; it += kStep) {
-                lim = next_lim;
+                const int lim = next_lim;  // page-uniform: rows of the iteration at or past it are absent
+                bool ok[L];
 #pragma unroll
                 for (int u = 0; u < L; ++u) ok[u] = PAGE_UNIFORM ? it + u * S::kTpl + tl < lim : next_ok[u];
                 f32x4 sc[kStates][L];
@@ -637,7 +709,11 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 for (int u = 0; u < L; ++u)
 #pragma unroll
                     for (int t = 0; t < kStates; ++t)
-                        sc[t][u] = T::mfma16x16x32(kk[u], qop[t], f32x4{0.f, 0.f, 0.f, 0.f});
+                        sc[t][u] = T::mfma16x16x32(mk[u], qop[t], f32x4{0.f, 0.f, 0.f, 0.f});
+                // The owner's store of the new row completes before the row is read.
+                if constexpr (PRO)
+                    if (owner && it + kStep <= pos && pos < it + kStep + S::kTpi) __builtin_amdgcn_s_waitcnt(0);
+                fetch_page(it + kStep);
                 fetch_k(it + kStep);
                 float p[kStates][L];
 #pragma unroll
@@ -692,7 +768,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 if (!PAGE_UNIFORM || it + S::kTpi > lim) {
 #pragma unroll
                     for (int u = 0; u < L; ++u)
-                        if (!ok[u]) vv[u] = u32x4{0u, 0u, 0u, 0u};
+                        if (!ok[u]) mv[u] = u32x4{0u, 0u, 0u, 0u};
                 }
 #pragma unroll
                 for (int u = 0; u < L; ++u) {
@@ -701,7 +777,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                     if constexpr (G == 8) pu[1] = kStates == 2 ? p[kStates - 1][u] : lane_xor4(p[0][u]);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const float v0 = T::lo(vv[u][i]), v1 = T::hi(vv[u][i]);
+                        const float v0 = T::lo(mv[u][i]), v1 = T::hi(mv[u][i]);
 #pragma unroll
                         for (int t = 0; t < G / 4; ++t) {
                             macc[t][2 * i] = __builtin_amdgcn_mfma_f32_4x4x1f32(v0, pu[t], macc[t][2 * i], 0, 0, 0);
@@ -929,7 +1005,9 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             if (direct) {
                 static_cast<uint16_t*>(a.out)[bh * D + d] = T::from_float(sum > 0.f ? o / sum : 0.f);
             } else {
-                const int64_t row = FLAT ? fl_row + g : bh * a.max_parts + part;
+                const int64_t row = FLAT ? fl_row + g
+                                    : EVEN && a.even_slots > 0 ? (int64_t)unit * G + g
+                                                               : bh * a.max_parts + part;
                 a.ws_acc[row * D + d] = o;
                 if (d == 0) {
                     a.ws_ml[row * 2] = mx;

@@ -11,7 +11,8 @@ import pytest
 import torch
 
 from gpu_cases import decode_inputs
-from mini_engine_hip.kernels.paged import paged_attention
+from mini_engine_hip.kernels.data import write_kv_cache_batch
+from mini_engine_hip.kernels.paged import paged_attention, paged_attention_decode_write
 from oracle import paged_oracle
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +95,33 @@ def test_absent_pages_and_lengths_count_as_nothing():
         out = paged_attention(q, key, value, table, lens, block, validate=False, partition_tokens=partition).float()
         assert (out[0] - want).abs().max().item() <= GATE[torch.bfloat16]
         assert out[1].abs().max().item() == 0 and out[2].abs().max().item() == 0
+
+
+@pytest.mark.parametrize("lengths,kv_heads", [
+    ((2048,), 1), ((3000,), 4), ((1, 2500, 64, 65, 129, 2), 4), (tuple([2300] * 20), 4),
+    (tuple(1 + 37 * i for i in range(64)), 3), (tuple(2600 - 40 * i for i in range(59)), 4),
+])
+@pytest.mark.parametrize("group", [7, 8, 12])
+def test_partitions_decided_by_the_lengths(lengths, kv_heads, group):
+    """8-head tiles over tables of 2048 tokens and more: the partition length
+    follows from the lengths (one sequence, 64 of them, equal, one token,
+    two tiles per group), also when they change under the same tables, with
+    an empty sequence, and with the step's row written by the launch."""
+    dtype = torch.bfloat16
+    args = decode_inputs(dtype, lengths=lengths, heads=group * kv_heads, kv_heads=kv_heads, seed=len(lengths))
+    check(args, dtype, 0)
+    q, key, value, table, lens, block = [a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args]
+    shorter = torch.clamp(lens // 3, min=1)
+    got = paged_attention(q, key, value, table, shorter, block, validate=False).float().cpu()
+    want = oracle(list(args[:4]) + [shorter.cpu(), block])
+    assert (got - want).abs().max().item() <= GATE[dtype]
+    empty = lens.clone()
+    empty[0] = 0
+    out = paged_attention(q, key, value, table, empty, block, validate=False)
+    assert out[0].abs().max().item() == 0
+    new_k, new_v = (torch.randn(len(lengths), kv_heads, 128, device=DEV).to(dtype) for _ in range(2))
+    k2, v2 = key.clone(), value.clone()
+    fused = paged_attention_decode_write(q, key, value, table, lens, block, new_k, new_v, validate=False)
+    write_kv_cache_batch(k2, v2, table, lens - 1, new_k, new_v, block, validate=False)
+    assert torch.equal(key, k2) and torch.equal(value, v2)
+    assert torch.equal(fused, paged_attention(q, k2, v2, table, lens, block, validate=False))
