@@ -15,7 +15,8 @@
 //   features, x and the weight slab copied global->LDS in whole 1 KiB
 //   segments;
 // * register (any other shape): one work-group per 16 output features, each
-//   lane loading its operands straight into registers.
+//   lane loading its operands straight into registers (by quads where K is a
+//   multiple of 128).
 // In all, the waves of a work-group split K, each wave computing D[n, m] = W[n, k-slice]
 // x[m, k-slice]^T for every 16-row block of x with v_mfma_f32_16x16x32 (fp32
 // accumulation), then their partial tiles are summed through LDS and
@@ -48,6 +49,30 @@ struct LinearArgs {
     int out_features;  // N, a multiple of 16
     int64_t x_stride;  // elements between rows of x
 };
+
+// Sum of NW waves' partials of one (row block, lane) slot of a 16-feature tile,
+// every partial read before any is added, and the store of its 4 features.
+template <typename T, int NW, typename F>
+__device__ inline void sum_and_store(const LinearArgs& a, int n0, int mb, int l, F part) {
+    f32x4 p[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) p[w] = part(w);
+#pragma unroll
+    for (int n = NW; n > 1; n = (n + 1) / 2)
+#pragma unroll
+        for (int w = 0; w < n / 2; ++w) p[w] += p[w + (n + 1) / 2];
+    const int row = 16 * mb + (l & 15);
+    if (row >= a.rows) return;
+    const int nb = n0 + 4 * (l >> 4);
+    float v[4] = {p[0][0], p[0][1], p[0][2], p[0][3]};
+    if (a.bias) {
+        const uint16_t* bias = static_cast<const uint16_t*>(a.bias) + nb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += T::lo((uint32_t)bias[i]);
+    }
+    const u32x2 packed = {T::pack(v[0], v[1]), T::pack(v[2], v[3])};
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (int64_t)row * a.out_features + nb) = packed;
+}
 
 // A operand: W rows n0 + (lane % 16), k = k0 + 8 * (lane / 16) .. +8.
 // B operand: x rows 16 * mb + (lane % 16), same k.  D: lane holds output
@@ -126,6 +151,69 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(LinearArgs a) 
         const u32x2 packed = {T::pack(v[0], v[1]), T::pack(v[2], v[3])};
         *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (int64_t)row * a.out_features + nb) = packed;
     }
+}
+
+// Register kernel for K a multiple of 128: as above, but with a wave's k-slices
+// 128 wide and both operands loaded by quads and transposed (see
+// quad_transpose), two slices in flight.  us per call into 2048 features,
+// operand-order loads -> quads: K = 4096 10.8 -> 7.8 at 16 rows, 14.7 -> 9.5 at
+// 32, 22.7 -> 15.1 at 64; K = 896, 16 rows 5.9 -> 4.1.
+template <typename T, int MB>
+__global__ __launch_bounds__(kLinThreads) void linear_rows_quads_kernel(LinearArgs a) {
+    __shared__ f32x4 sm_part[kLinWaves][MB][kWave];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int n0 = blockIdx.x * 16;
+    const int li = lane & 15, lg = lane >> 4;
+    const int slices = a.in_features / 128;
+    const int quad = li & ~3, chunk = 8 * (4 * lg + (li & 3));
+    const uint16_t* wrow = static_cast<const uint16_t*>(a.weight) + (int64_t)(n0 + quad) * a.in_features + chunk;
+    const uint16_t* xbase = static_cast<const uint16_t*>(a.x) + chunk;
+    f32x4 acc[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int kInFlight = MB <= 2 ? 2 : 1;
+    for (int s0 = wave; s0 < slices; s0 += kLinWaves * kInFlight) {
+        u32x4 wv[kInFlight][4], xv[kInFlight][MB][4];
+#pragma unroll
+        for (int f = 0; f < kInFlight; ++f) {
+            const int s = min(s0 + f * kLinWaves, slices - 1);  // past the end: re-read the last, unused
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                wv[f][j] = *reinterpret_cast<const u32x4*>(wrow + (int64_t)j * a.in_features + 128 * s);
+            // Rows of x past M read row 0 (in bounds); their products are dropped.
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int r = 16 * mb + quad + j;
+                    xv[f][mb][j] = *reinterpret_cast<const u32x4*>(xbase + (int64_t)(r < a.rows ? r : 0) * a.x_stride + 128 * s);
+                }
+        }
+#pragma unroll
+        for (int f = 0; f < kInFlight; ++f) {
+            const bool live = s0 + f * kLinWaves < slices;
+            quad_transpose(wv[f]);
+            if (!live)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) wv[f][j] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                quad_transpose(xv[f][mb]);
+                if (!live)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) xv[f][mb][j] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[mb] = T::mfma16x16x32(wv[f][j], xv[f][mb][j], acc[mb]);
+            }
+        }
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) sm_part[wave][mb][lane] = acc[mb];
+    __syncthreads();
+    for (int slot = threadIdx.x; slot < MB * kWave; slot += kLinThreads)
+        sum_and_store<T, kLinWaves>(a, n0, slot / kWave, slot % kWave,
+                                    [&](int w) { return sm_part[w][slot / kWave][slot % kWave]; });
 }
 
 // Staged variant for the decode batch (K a multiple of 512, N of 8, x and an
@@ -278,17 +366,22 @@ __global__ __launch_bounds__(NW * kWave, (stream_waves<MB, NW>() / 4)) void line
     };
     u32x4 wa[KS], wb[KS];
     load(t_begin, wa);
-    // Rows of x past M read row 0 (in bounds); their products are dropped.
+    // x's operands, loaded and transposed like the weight's (64 rows into 4096
+    // features 11.9 -> 9.4 us, 32 rows 7.8 -> 7.0).  Rows past M read row 0 (in
+    // bounds); their products are dropped.
     u32x4 xop[MB][KS];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-        const int r = 16 * mb + li;
-        const uint16_t* xrow = static_cast<const uint16_t*>(a.x) + (int64_t)(r < a.rows ? r : 0) * a.x_stride +
-                               wave * (KS * 32) + 32 * lg;
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int j = 0; j < KS; ++j) xop[mb][j] = *reinterpret_cast<const u32x4*>(xrow + 8 * j);
-    }
+        for (int j = 0; j < KS; ++j) {
+            const int r = 16 * mb + (li & ~3) + j;
+            xop[mb][j] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.x) +
+                                                         (int64_t)(r < a.rows ? r : 0) * a.x_stride +
+                                                         wave * (KS * 32) + 8 * (4 * lg + (li & 3)));
+        }
     load(t_begin + 1, wb);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) quad_transpose(xop[mb]);
     auto tile = [&](int t, u32x4 (&w)[KS], int buf) __attribute__((always_inline)) {
         f32x4 acc[MB];
 #pragma unroll
@@ -309,24 +402,7 @@ __global__ __launch_bounds__(NW * kWave, (stream_waves<MB, NW>() / 4)) void line
         const int first = (t - t_begin) * MB % NW;
         const int mb = wave >= first ? wave - first : wave - first + NW;
         if (mb >= MB) return;
-        f32x4 p[NW];
-#pragma unroll
-        for (int v = 0; v < NW; ++v) p[v] = sm_part[buf][v][mb][lane];
-#pragma unroll
-        for (int n = NW; n > 1; n = (n + 1) / 2)
-#pragma unroll
-            for (int v = 0; v < n / 2; ++v) p[v] += p[v + (n + 1) / 2];
-        const int row = 16 * mb + li;
-        if (row >= a.rows) return;
-        const int nb = 16 * t + 4 * lg;
-        float v[4] = {p[0][0], p[0][1], p[0][2], p[0][3]};
-        if (a.bias) {
-            const uint16_t* bias = static_cast<const uint16_t*>(a.bias) + nb;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] += T::lo((uint32_t)bias[i]);
-        }
-        const u32x2 packed = {T::pack(v[0], v[1]), T::pack(v[2], v[3])};
-        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + (int64_t)row * a.out_features + nb) = packed;
+        sum_and_store<T, NW>(a, 16 * t, mb, lane, [&](int w) { return sm_part[buf][w][mb][lane]; });
     };
     // Pairs without a branch between the two tiles: with one, the compiler's
     // wait for the first tile's weights also covers the second's.
@@ -390,6 +466,13 @@ template <typename T>
 void launch_linear_rows(const LinearArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)(a.out_features / 16)), block(kLinThreads);
     const int mb = (a.rows + 15) / 16;
+    if (a.in_features % 128 == 0) {
+        if (mb == 1) hipLaunchKernelGGL((linear_rows_quads_kernel<T, 1>), grid, block, 0, s, a);
+        else if (mb == 2) hipLaunchKernelGGL((linear_rows_quads_kernel<T, 2>), grid, block, 0, s, a);
+        else if (mb == 3) hipLaunchKernelGGL((linear_rows_quads_kernel<T, 3>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((linear_rows_quads_kernel<T, 4>), grid, block, 0, s, a);
+        return;
+    }
     if (mb == 1) hipLaunchKernelGGL((linear_rows_kernel<T, 1>), grid, block, 0, s, a);
     else if (mb == 2) hipLaunchKernelGGL((linear_rows_kernel<T, 2>), grid, block, 0, s, a);
     else if (mb == 3) hipLaunchKernelGGL((linear_rows_kernel<T, 3>), grid, block, 0, s, a);
@@ -432,7 +515,7 @@ extern "C" int mvme_linear_rows(void* out, const void* x, const void* weight, co
     // stream; at most that many fit the chip at once and start faster staged
     // (no prologue that loads x into registers).  us per call, staged against
     // streaming, K = 2048: N = 2048 4.3 / 5.3 at 16 rows, 5.7 / 6.9 at 32;
-    // N = 4096 8.3 / 6.3, 10.6 / 7.7, 13.2 / 11.9 at 64; N = 8192 14.3 / 11.0;
+    // N = 4096 8.3 / 6.1, 10.6 / 7.0, 13.2 / 9.4 at 64; N = 8192 14.3 / 11.0;
     // K = 1024, N = 4096 4.4 / 4.2.
     if (in_features % 512 == 0 && in_features <= kStreamMaxK && out_features > kLinCUs * kStagedFeat) {
         if (dtype == MVME_FP16) launch_linear_stream<Half>(a, mb, s);

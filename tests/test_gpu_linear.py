@@ -50,6 +50,17 @@ def test_linear_rows_wide_layers(dtype, rows, k, n, bias):
     test_linear_rows_matches_fp32_product(dtype, rows, k, n, bias)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,k,n,bias", [
+    (1, 128, 16, False), (16, 640, 48, True), (32, 896, 2048, False), (33, 3584, 80, False),
+    (64, 4096, 2048, True), (48, 384, 32, False), (17, 2176, 64, False),
+])
+def test_linear_rows_quad_slices(dtype, rows, k, n, bias):
+    """K a multiple of 128 outside the staged and the streaming kernel: fewer
+    slices than waves, one round of them, a remainder of a second and third."""
+    test_linear_rows_matches_fp32_product(dtype, rows, k, n, bias)
+
+
 def test_linear_rows_strided_input_rows():
     """x as a row slice of a wider buffer (row stride > in_features)."""
     gen = torch.Generator().manual_seed(3)
