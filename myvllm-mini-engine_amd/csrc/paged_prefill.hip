@@ -73,17 +73,19 @@ constexpr int kArriveSpinLimit = 1 << 18; // polls (each with a 64-cycle sleep) 
 constexpr int kTileBytes = 16384;         // one K (or V) tile in LDS, every tile shape
 constexpr int kPfMaxKeys = 64;            // keys per tile, largest tile shape
 
-// Tile shape of the MFMA kernel by padded head dim: 128 (head_dim 128 and
-// narrower multiples of 8) or 256.  Every tile is 16 KiB of K (and of V) in
-// LDS; at 256 a wave holds one 16-row block (the accumulators of 256 dims
-// fill the registers two blocks used) and a tile has 32 keys.
+// Tile shape of the MFMA kernel by padded head dim: 64 (head_dim 64 on
+// power-of-two pages), 128 (head_dim 128 and other narrower multiples of 8)
+// or 256.  A tile is 16 KiB of K (and of V) in LDS, 8 at 64; at 256 a wave
+// holds one 16-row block (the accumulators of 256 dims fill the registers two
+// blocks used) and a tile has 32 keys.
 template <int HD>
 struct PfShape {
-    static_assert(HD == 128 || HD == 256, "padded head dim 128 or 256");
+    static_assert(HD == 64 || HD == 128 || HD == 256, "padded head dim 64, 128 or 256");
     static constexpr int kD = HD;
-    static constexpr int kNb = HD == 128 ? 2 : 1;      // 16-row MFMA column blocks per wave
+    static constexpr int kPart = HD <= 128 ? 128 : HD;  // elements between partial rows
+    static constexpr int kNb = HD <= 128 ? 2 : 1;      // 16-row MFMA column blocks per wave
     static constexpr int kRows = kPfWaves * kNb * 16;  // query rows per work-group
-    static constexpr int kKeys = HD == 128 ? 64 : 32;  // keys per LDS tile
+    static constexpr int kKeys = HD <= 128 ? 64 : 32;  // keys per LDS tile
     static constexpr int kHalves = kKeys / 32;         // 32-key halves per tile
     static constexpr int kRowBytes = HD * 2;           // bytes per K/V row in LDS
     static constexpr int kChunks = HD / 8;             // 16-byte chunks per row
@@ -91,7 +93,12 @@ struct PfShape {
     static constexpr int kIpw = kKeys * kRowBytes / 1024 / kPfWaves;  // copy instructions per wave per tile
     static constexpr int kDc = HD / 32;  // 32-dim slices of a score product
     static constexpr int kDt = HD / 16;  // 16-dim output blocks
-    static_assert(kKeys * kRowBytes == kTileBytes, "one tile = 16 KiB");
+    static_assert(kKeys * kRowBytes <= kTileBytes, "a tile fits its stage");
+    // Slot of a row's 16-byte chunk c in LDS: c ^ k_swizzle(row) for K, c ^
+    // v_swizzle(row) for V.  With 64 dims two rows share the 64 banks, so the
+    // row's upper bits select the slot and its parity the half.
+    __device__ static constexpr int k_swizzle(int row) { return kChunks == 8 ? (row >> 1) & 7 : row & 15; }
+    __device__ static constexpr int v_swizzle(int row) { return kChunks == 8 ? row & 6 : (2 * row) & 15; }
 };
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -125,7 +132,7 @@ struct PrefillArgs {
     int max_chunks;
     int chunk_choice;  // 1: a walk with more than one round of items may take a larger chunk
     int head_dim;
-    int part_dim;  // elements per partial row: the tile shape's padded head dim
+    int part_dim;  // elements per partial row: the tile shape's PfShape::kPart
     int64_t num_blocks;
     int block_size;
     int block_shift;  // log2(block_size) when a power of two, else -1
@@ -441,10 +448,10 @@ constexpr int kPagesPerWave = 3;
 //     are a scalar base plus precomputed per-lane offsets -- a few scalar
 //     instructions per tile, which matters because the scalar unit is shared
 //     by all waves of the CU.
-//   kPagesPerWave: block_size is 8, 16 or 32 (the 128 shape): the 8 key rows
-//     of a tile that one wave copies lie in one page, so a whole tile's copies
-//     are again a scalar base (each wave its own page's) plus the same
-//     per-lane offsets.
+//   kPagesPerWave: block_size is 8, 16 or 32 at the 128 shape, or a power of
+//     two of at least 8 at the 64 shape: the 8 key rows of a tile that one wave
+//     copies lie in one page, so a whole tile's copies are again a scalar base
+//     (each wave its own page's) plus the same per-lane offsets.
 //   kPagesPerRows: see below; the fallback for partial tiles as well.
 // SCALAR_PAGES: block_size is a multiple of 4, so the 4 key rows one copy
 // instruction covers sit in one page and the page id is wave-uniform (a
@@ -582,7 +589,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
     // The software-pipelined loop serves pages of the 128 shape that hold
     // each wave's copy rows of a tile.
     constexpr bool WAVE_PAGES = PAGES == kPagesPerWave;
-    constexpr bool PIPE = (PAGES == kPagesPerTile || WAVE_PAGES) && !NARROW && HD == 128;
+    constexpr bool PIPE = (PAGES == kPagesPerTile || WAVE_PAGES) && !NARROW && HD <= 128;
     // Queries scaled once by scale*log2(e) (one more rounding of q) instead
     // of every score in fp32.  The modes that joined the pipelined loop later
     // (small pages 127.9 -> 111.2 us for 16 sequences of 56..900 tokens with
@@ -692,12 +699,12 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
     // 2 adjacent chunks) hit 8 different 16-byte bank groups.
     int koff[SH::kDc];
 #pragma unroll
-    for (int dc = 0; dc < SH::kDc; ++dc) koff[dc] = li * SH::kRowBytes + 16 * ((4 * dc + lg) ^ li);
+    for (int dc = 0; dc < SH::kDc; ++dc) koff[dc] = li * SH::kRowBytes + 16 * ((4 * dc + lg) ^ SH::k_swizzle(li));
     const int vrow = 4 * lg + (li >> 2);
     int voff[SH::kDt];
 #pragma unroll
     for (int dt = 0; dt < SH::kDt; ++dt)
-        voff[dt] = vrow * SH::kRowBytes + 16 * ((2 * dt + ((li & 3) >> 1)) ^ ((2 * vrow) & 15)) + 8 * (li & 1);
+        voff[dt] = vrow * SH::kRowBytes + 16 * ((2 * dt + ((li & 3) >> 1)) ^ SH::v_swizzle(vrow)) + 8 * (li & 1);
 
     // Copy plan: a tile's K (and V) is 16 instructions of 1 KiB; wave w issues
     // instructions j = SH::kIpw*w + i, each covering key rows 4j..4j+3 (lane ->
@@ -718,7 +725,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
 #pragma unroll
     for (int i = 0; i < SH::kIpw; ++i) {
         const int row = SH::kRowsPerInst * (SH::kIpw * wave + i) + lrow;
-        const int kc = lslot ^ (row & 15), vc = lslot ^ ((2 * row) & 15);
+        const int kc = lslot ^ SH::k_swizzle(row), vc = lslot ^ SH::v_swizzle(row);
         kchunk_ok[i] = !NARROW || kc < dchunks;
         vchunk_ok[i] = !NARROW || vc < dchunks;
         tile_off[i] = (uint32_t)(row * row_bytes_g) + 16u * (uint32_t)(kchunk_ok[i] ? kc : 0);
@@ -799,8 +806,8 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
             const int j = SH::kIpw * wave + i;
             const int row = SH::kRowsPerInst * j + lrow;
             const int key = tile * SH::kKeys + row;
-            const int cidx = lslot ^ (row & 15);
-            const int cidx_v = lslot ^ ((2 * row) & 15);
+            const int cidx = lslot ^ SH::k_swizzle(row);
+            const int cidx_v = lslot ^ SH::v_swizzle(row);
             const int page = pg_next[i];
             // Rows past the chunk inside a valid first-row page are masked too.
             const bool ok = page >= 0 && key < chunk_end;
@@ -889,16 +896,19 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
             const int key0 = (base + lane) * SH::kKeys;
             bool whole = key0 + SH::kKeys <= chunk_end;
             int64_t mine = 0;
-            if (whole) {
-                const int per_tile = SH::kKeys >> bs_shift;
-                const int own = (kCopyRows * wave) >> bs_shift;
+            const int first = key0 + kCopyRows * wave;
+            if (ident) {
+                mine = seq;
+            } else if (whole) {
+                const int idx = key0 >> bs_shift, own = (first >> bs_shift) - idx;
+                const int per_tile = max(SH::kKeys >> bs_shift, 1);
                 for (int j = 0; j < per_tile; ++j) {
-                    const int64_t page = table[(key0 >> bs_shift) + j];
+                    const int64_t page = table[idx + j];
                     whole = whole && page >= 0 && page < a.num_blocks;
                     if (j == own) mine = page;
                 }
             }
-            const int in_page = (kCopyRows * wave) & (a.block_size - 1);
+            const int in_page = first & (a.block_size - 1);
             return whole ? mine * page_bytes_g + (int64_t)(in_page - kCopyRows * wave) * row_bytes_g + wave_bias
                          : (int64_t)-1;
         };
@@ -933,7 +943,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                 const int j = SH::kIpw * wave + i;
                 const int row = SH::kRowsPerInst * j + lrow;
                 const int key = key0 + row;
-                const int cidx = is_k ? lslot ^ (row & 15) : lslot ^ ((2 * row) & 15);
+                const int cidx = lslot ^ (is_k ? SH::k_swizzle(row) : SH::v_swizzle(row));
                 const bool ok = pg_ok && key < chunk_end;
                 const uint8_t* g = reinterpret_cast<const uint8_t*>(kZeroChunk);
                 if (ok) g = cache + base + (int64_t)(key & (a.block_size - 1)) * row_bytes_g + 16 * cidx;
@@ -1484,7 +1494,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
             const int64_t slot = (int64_t)chunk * a.ws_rows + rowid;
             const float inv = (row_ok[nb] && l_row > 0.f) ? __builtin_amdgcn_rcpf(l_row) : 0.f;
             using P = typename PartialOf<T>::type;
-            P* po = static_cast<P*>(a.ws_o) + slot * SH::kD;
+            P* po = static_cast<P*>(a.ws_o) + slot * SH::kPart;
 #pragma unroll
             for (int dt = 0; dt < SH::kDt; ++dt) {
                 if constexpr (sizeof(P) == 4) {
@@ -2007,7 +2017,8 @@ int check_prefill(int64_t num_seqs, int64_t total_tokens, int64_t q_heads, int64
 struct PrefillPlan {
     bool mfma;
     bool narrow;  // head_dim below the tile shape's, zero-padded in LDS
-    int hd;       // tile shape: padded head dim (128 or 256)
+    int hd;       // tile shape: padded head dim (64, 128 or 256)
+    int part;     // elements between partial rows (PfShape::kPart)
     int keys;     // keys per tile of that shape
     int qb;
     int chunk;
@@ -2032,7 +2043,15 @@ PrefillPlan make_prefill_plan(int64_t num_seqs, int64_t total_tokens, int64_t q_
     // with zeros in LDS (zero dims add nothing to the scores and give zero
     // outputs).
     const bool wide = head_dim > 128;
-    p.hd = wide ? 256 : 128;
+    // 64 dims have a shape of their own on pages that hold a wave's copy
+    // rows; padded to 128 they cost twice the products and ran the loop that
+    // is not pipelined (us: 16/8 heads, 8 ragged sequences of up to 900 tokens
+    // 63.8 -> 39.5; 14/2 heads, 16 of them 84.0 -> 47.3; dense 8192 258 ->
+    // 178).
+    const bool half = head_dim == 64 && block_size >= 8 && (block_size & (block_size - 1)) == 0 &&
+                      (double)kv_heads * 64.0 * 2.0 * PfShape<64>::kKeys < 2147483648.0;
+    p.hd = wide ? 256 : half ? 64 : 128;
+    p.part = wide ? PfShape<256>::kPart : PfShape<128>::kPart;
     p.narrow = head_dim < p.hd;
     p.keys = wide ? PfShape<256>::kKeys : PfShape<128>::kKeys;
     const int rows = wide ? PfShape<256>::kRows : PfShape<128>::kRows;
@@ -2088,7 +2107,7 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
         if (table_width * a.block_size > 2147483647)
             return fail(MVME_EINVAL, "paged prefill table capacity exceeds 2^31 tokens");
         a.qb = p.qb;
-        a.part_dim = p.hd;
+        a.part_dim = p.part;
         a.chunk = p.chunk;
         a.max_chunks = p.max_chunks;
         a.ws_rows = total_tokens * q_heads;
@@ -2096,7 +2115,7 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
         a.chunk_choice = chunk_tokens <= 0 ? 1 : 0;
         if (need > 0) {
             const PrefillWorkspace w = prefill_workspace_layout(total_tokens * q_heads, p.max_chunks, total_tokens,
-                                                                dtype, p.hd);
+                                                                dtype, p.part);
             a.ws_o = workspace;
             a.ws_ml = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + w.ml_offset);
             a.ws_tok = reinterpret_cast<int*>(static_cast<uint8_t*>(workspace) + w.tok_offset);
@@ -2126,8 +2145,9 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
         if (dense && !tile_pages) return fail(MVME_EINVAL, "prefill key/value token stride too large");
         // Pages per wave: a wave copies 8 consecutive key rows of a tile, so
         // power-of-two blocks of 8, 16 or 32 tokens keep them in one page.
-        const bool wave_pages = a.block_shift >= 3 && p.hd == 128 && !p.narrow &&
+        const bool wave_pages = a.block_shift >= 3 && p.hd <= 128 && !p.narrow &&
                                 a.kv_row_bytes * p.keys < (int64_t(1) << 31);
+        if (p.hd == 64 && !wave_pages) return fail(MVME_EINVAL, "prefill key/value token stride too large");
         int pages = tile_pages ? kPagesPerTile : wave_pages ? kPagesPerWave : (block_size % 4 == 0 ? kPagesPerRows : kPagesPerLane);
         if (p.narrow && pages == kPagesPerRows) pages = kPagesPerLane;  // no narrow instantiation of that mode
         const dim3 grid((unsigned)groups), block(kPfThreads);
@@ -2138,7 +2158,14 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
         };
         auto launch_type = [&](auto type_tag) {
             using T = decltype(type_tag);
-            if (dense) {
+            if (p.hd == 64) {
+                if (dense)
+                    launch_walk(paged_prefill_mfma_kernel<T, kPagesPerWave, false, false, 64, true>,
+                                paged_prefill_mfma_kernel<T, kPagesPerWave, true, false, 64, true>);
+                else
+                    launch_walk(paged_prefill_mfma_kernel<T, kPagesPerWave, false, false, 64, false>,
+                                paged_prefill_mfma_kernel<T, kPagesPerWave, true, false, 64, false>);
+            } else if (dense) {
                 // Dense mode: one power-of-two page per sequence, whole-tile copies.
                 if (p.hd == 256 && p.narrow)
                     launch_walk(paged_prefill_mfma_kernel<T, kPagesPerTile, false, true, 256, true>,
@@ -2230,7 +2257,7 @@ extern "C" size_t mvme_paged_prefill_workspace_size(int64_t num_seqs, int64_t to
     const PrefillPlan p = make_prefill_plan(num_seqs, total_tokens, q_heads, kv_heads, head_dim, block_size,
                                             table_width, chunk_tokens);
     if (!p.mfma || p.max_chunks <= 1) return 0;
-    return prefill_workspace_layout(total_tokens * q_heads, p.max_chunks, total_tokens, dtype, p.hd).bytes;
+    return prefill_workspace_layout(total_tokens * q_heads, p.max_chunks, total_tokens, dtype, p.part).bytes;
 }
 
 extern "C" int mvme_paged_prefill_attention(void* out, const void* q, const void* key_cache,
@@ -2354,7 +2381,7 @@ extern "C" size_t mvme_prefill_attention_workspace_size(int64_t batch, int64_t q
     const PrefillPlan p = make_prefill_plan(batch, rows, q_heads, kv_heads, head_dim,
                                             dense_block(query_start + q_tokens), 1, 0);
     if (!p.mfma || p.max_chunks <= 1) return 0;
-    return prefill_workspace_layout(rows * q_heads, p.max_chunks, rows, dtype, p.hd).bytes;
+    return prefill_workspace_layout(rows * q_heads, p.max_chunks, rows, dtype, p.part).bytes;
 }
 
 extern "C" int mvme_prefill_attention(void* out, const void* q, const void* key, const void* value, int64_t batch,

@@ -13,17 +13,17 @@ DEV = "cuda"
 GATE = {torch.float16: 2e-3, torch.bfloat16: 1.6e-2}
 
 
-def paged_case(new, prior, block, heads, kv_heads, dtype, seed):
+def paged_case(new, prior, block, heads, kv_heads, dtype, seed, dim=128):
     gen = torch.Generator().manual_seed(seed)
     cu = torch.tensor([0] + torch.tensor(new).cumsum(0).tolist())
     starts = torch.tensor(prior)
     lens = starts + torch.tensor(new)
     width = max(1, -(-int(lens.max()) // block))
     pages = len(new) * width + 3
-    kc = torch.randn(pages, block, kv_heads, 128, generator=gen).to(dtype)
-    vc = torch.randn(pages, block, kv_heads, 128, generator=gen).to(dtype)
+    kc = torch.randn(pages, block, kv_heads, dim, generator=gen).to(dtype)
+    vc = torch.randn(pages, block, kv_heads, dim, generator=gen).to(dtype)
     tables = torch.randperm(pages, generator=gen)[:len(new) * width].view(len(new), width)
-    q = torch.randn(int(cu[-1]), heads, 128, generator=gen).to(dtype)
+    q = torch.randn(int(cu[-1]), heads, dim, generator=gen).to(dtype)
     return [q, kc, vc, cu, starts, tables, lens]
 
 
@@ -91,4 +91,32 @@ def test_dense_tiles_and_windows(dtype, tokens, start):
     v = torch.randn(1, 4, start + tokens + 9, 128, generator=gen).to(dtype)
     actual = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), query_start=start).float().cpu()
     expected = paged_oracle.prefill_attention(q, k, v, query_start=start, cast=False)
+    assert (actual - expected).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block", [4, 8, 16, 64, 256])
+@pytest.mark.parametrize("new,prior,chunk,heads", [
+    ([64, 1, 130], [0, 63, 64], 0, 14), ([40], [4400], 8192, 8), ([300, 77], [1200, 41], 256, 4),
+])
+def test_head_dim_64_tiles(dtype, block, new, prior, chunk, heads):
+    """The 64-dim tile shape: whole and partial tiles, windows, key chunks,
+    pages smaller and larger than a tile (4-token pages keep the padded
+    shape), groups of 7, 4 and 2."""
+    args = paged_case(new, prior, block, heads, 2, dtype, seed=block + sum(new), dim=64)
+    actual = paged_prefill_attention(*[a.to(DEV) for a in args], block, chunk_tokens=chunk).float().cpu()
+    expected = paged_oracle.paged_prefill_attention(*args, block, cast=False)
+    assert (actual - expected).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("batch,tokens,start,view", [(1, 130, 0, True), (2, 65, 4300, True), (1, 700, 33, False)])
+def test_head_dim_64_dense(batch, tokens, start, view):
+    dtype, gen = torch.bfloat16, torch.Generator().manual_seed(tokens)
+    make = lambda n, h: torch.randn(batch, n, h, 64, generator=gen).to(dtype)  # noqa: E731
+    q, k, v = make(tokens, 14), make(start + tokens, 2), make(start + tokens, 2)
+    dev = [t.to(DEV).transpose(1, 2) for t in (q, k, v)]
+    if not view:
+        dev = [t.contiguous() for t in dev]
+    actual = prefill_attention(*dev, query_start=start).float().cpu()
+    expected = paged_oracle.prefill_attention(*[t.transpose(1, 2) for t in (q, k, v)], query_start=start, cast=False)
     assert (actual - expected).abs().max().item() <= GATE[dtype]
