@@ -390,13 +390,14 @@ void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim) {
 
 constexpr int64_t kEvenCapacity = 2048;
 
-// Partition length of a split over tiles of 2 to 4 heads of 128: the number of
+// Partition length of a split over tiles of 1 to 4 heads of 128: the number of
 // partitions n that minimises the iterations the busiest CU runs, half at full
 // tables and half at tables filled a little over half (ragged batches), plus
 // a share per partition for its start, its end and the merge.  A target of two
 // work-groups per CU alone leaves some CUs with three and others with two: 24
 // sequences of 2048, 8 kv heads (192 units): 3 partitions 42.9 us (26.7 for
 // U[1,2048]), 4 partitions -- three per CU -- 36.5 (22.1).
+// (8/8 heads: 42.8 -> 37.9 and 26.2 -> 21.3.)
 int64_t split_partition(int64_t cap, int64_t units, int64_t step) {
     const int64_t steps = (cap + step - 1) / step;
     int64_t best = 1;
@@ -463,7 +464,7 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
         p.waves = kSplitWaves;
         if (requested > 0) {
             part = requested;
-        } else if (group >= 2 && group <= 4 && head_dim == 128) {
+        } else if (group <= 4 && head_dim == 128) {
             part = split_partition(cap, units, split_step);
         } else {
             // Wide tiles of 64 dims gain from more and shorter partitions: 14/2 heads, 60 sequences
