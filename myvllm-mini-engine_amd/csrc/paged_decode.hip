@@ -511,12 +511,20 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
         p.max_parts = 1;
     }
     // Pairs of heads: the matrix cores' loop, which keeps loads in flight,
-    // where several work-groups share a CU (16/8 heads, pages of 16: 64 sequences U[1,4096] 94.5 -> 91.5 us, 16 of
-    // U[1,1024] 13.2 -> 12.5, 8 of 512 8.9 -> 8.6; one 8-wave work-group per CU
-    // or the walk has no use for it: 32 of 2048 44.6 -> 45.8, walk of 32 of
-    // U[1,4096] 51.7 -> 54.0.)
-    if (group == 2 && (head_dim == 64 || head_dim == 128) && !flat &&
-        (p.max_parts > 1 || (p.waves == kWholeWaves && units > kDeviceCUs))) {
+    // where two work-groups share a CU (16/8 heads of 128, pages of 16: 64
+    // sequences U[1,4096] 94.5 -> 91.5 us, 16 of U[1,1024] 13.2 -> 12.5, 8 of
+    // 512 8.9 -> 8.6; one 8-wave work-group per CU, the walk and more units
+    // than two per CU have no use for it: 32 of 2048 44.6 -> 45.8, walk of 32
+    // of U[1,4096] 51.7 -> 54.0, 96 of U[1,2600] 93.7 -> 95.9, 200 of
+    // U[1,1500] 107.9 -> 112.5.)
+    // At 64 dims pairs take the matrix cores where pages hold runs of 16 tokens
+    // but not the dot products' iterations of 32, which then look up every
+    // token's page (16/8 heads, pages of 16: 64 of 1000 39.7 -> 29.1, 48 of
+    // U[1,2000] 35.2 -> 29.3, 1 of 128 5.2 -> 4.4; pages of 256, 128 of 1024
+    // 52.7 -> 57.0, of 24, 16 of 700 12.6 -> 17.2).
+    const bool runs_only = block_size % 32 == 16;
+    const bool shared_cu = p.max_parts > 1 || (p.waves == kWholeWaves && units > kDeviceCUs && units <= 2 * kDeviceCUs);
+    if (group == 2 && !flat && ((head_dim == 128 && shared_cu) || (head_dim == 64 && runs_only))) {
         p.gtile = 4;
         p.tile_heads = 2;
     }

@@ -76,6 +76,12 @@ struct DecodeShape {
     static constexpr bool kMatrix = D == 64 || D == 128;
     static constexpr int kParts = 16 / kTpl;
     static constexpr int kCols = 16 / kParts;  // query heads per score product
+    // Runs of 16 tokens that an iteration of the matrix-core path is made of.
+    // A run lies in one page, so pages of 16 keep scalar page lookups and
+    // loads without branches at 64 dims, where an iteration has 32 tokens
+    // (32/8 heads, pages of 16, us per call, a lookup per token -> per run: 48
+    // sequences U[1,2000] 54.0 -> 30.1, 40 of U[1,600] 23.5 -> 11.2).
+    static constexpr int kRuns = D == 64 ? 2 : 1;
 };
 
 // Largest query-head tile: 8 heads where the matrix-core path serves the
@@ -85,6 +91,9 @@ constexpr int max_gtile() { return DecodeShape<D>::kMatrix ? 8 : 4; }
 // The tile sizes computed on the matrix cores (the others use dot products).
 template <int D, int G>
 constexpr bool matrix_tile() { return DecodeShape<D>::kMatrix && G >= 4; }
+// Page lookups per iteration in the page-uniform loops.
+template <int D, int G>
+constexpr int page_runs() { return matrix_tile<D, G>() ? DecodeShape<D>::kRuns : 1; }
 
 // Balanced walk: the merge duty of share l, written by the attention
 // kernel's work-group for that share on every call and read by the merge
@@ -341,12 +350,18 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
     // on the lengths: looked up beside the length, not after it (entries past
     // the context are read but not used).
     typedef __attribute__((address_space(4))) const int64_t const_i64;
-    int64_t first_page = -1;
+    constexpr int H = page_runs<D, G>(), kRun = S::kTpi / H;
+    int64_t first_page[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) first_page[h] = -1;
     auto early_page = [&](int seq) __attribute__((always_inline)) {
-        const int t = __builtin_amdgcn_readfirstlane(part * a.partition + wave * S::kTpi);
-        if (PAGE_UNIFORM && t < a.capacity)
-            first_page = ((const const_i64*)(a.tables + (int64_t)seq * a.table_width))[a.block_shift >= 0 ? t >> a.block_shift
-                                                                                                     : t / a.block_size];
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const int t = __builtin_amdgcn_readfirstlane(part * a.partition + wave * S::kTpi) + h * kRun;
+            if (PAGE_UNIFORM && t < a.capacity)
+                first_page[h] = ((const const_i64*)(a.tables + (int64_t)seq * a.table_width))
+                    [a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size];
+        }
     };
     int64_t fl_wc = 0, fl_pos = 0, fl_stop = 0, fl_row = 0, fl_row_later = 0;
     if constexpr (FLAT) {
@@ -505,8 +520,13 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             return ctable[a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size];
         };
         int it = __builtin_amdgcn_readfirstlane(start + wave * S::kTpi);
-        int64_t page_next = 0;
-        if constexpr (PAGE_UNIFORM) page_next = !FLAT && a.lpt_batch == 0 && !(EVEN && a.even_slots > 0) ? first_page : page_of(it);
+        int64_t page_next[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            page_next[h] = 0;
+            if constexpr (PAGE_UNIFORM)
+                page_next[h] = !FLAT && a.lpt_batch == 0 && !(EVEN && a.even_slots > 0) ? first_page[h] : page_of(it + h * kRun);
+        }
         // The next iteration's rows are loaded into the registers as soon as
         // the products have read them: K right after the score products,
         // V load by load, so that their latency overlaps the softmax and
@@ -515,46 +535,77 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         // or without a page the loads read page 0's first rows, and `lim`
         // masks what they bring.
         u32x4 mk[MM ? L : 1], mv[MM ? L : 1];
-        int next_lim = 0;  // page-uniform: rows of the iteration at or past it are absent
-        int64_t next_base = 0;
-        bool next_ok[L];
-        auto row_of = [&](int t) __attribute__((always_inline)) -> int64_t {
-            int64_t page = -1;
-            if (t < end) page = table[t / a.block_size];
-            return page >= 0 && page < a.num_blocks ? page * page_elems + (int64_t)(t % a.block_size) * row_elems
-                                                    : (int64_t)-1;
-        };
-        auto fetch_page = [&](int t0) __attribute__((always_inline)) {
-            if constexpr (PAGE_UNIFORM) {
-                const int64_t page = page_next;
-                page_next = page_of(t0 + kStep);
-                const bool page_ok = page >= 0 && page < a.num_blocks;
-                const int in_page = a.block_shift >= 0 ? t0 & (a.block_size - 1) : t0 % a.block_size;
-                next_base = page_ok ? (page * a.block_size + in_page) * (int64_t)row_bytes : 0;
-                next_lim = page_ok ? end : 0;
+        constexpr int kRunLoads = L / H;  // loads per run
+        int next_lim[H];  // page-uniform: rows of the run at or past it are absent
+        int64_t next_base[H];
+        // Other pages: each lane's page ids of the iteration after the next,
+        // looked up before the K loads of the next one, and the next one's
+        // rows.  (Looked up when they are needed, every load waits for all
+        // loads before it: 32/8 heads of 64, pages of 8, 24 sequences
+        // U[1,2000] 35.4 us on dot products -> 25.7; of 128, U[1,3000] 85.4 ->
+        // 41.9.)
+        constexpr bool kLookup = MM && !PAGE_UNIFORM;
+        int64_t ahead_k[kLookup ? L : 1], ahead_v[kLookup ? L : 1];
+        int64_t next_krow[kLookup ? L : 1], next_vrow[kLookup ? L : 1];
+        auto lookup = [&](int t0) __attribute__((always_inline)) {
+            auto page_at = [&](int t) __attribute__((always_inline)) -> int64_t {
+                const int tc = min(t, end - 1);
+                return table[a.block_shift >= 0 ? tc >> a.block_shift : tc / a.block_size];
+            };
+#pragma unroll
+            for (int u = 0; u < L; ++u) {
+                ahead_k[kLookup ? u : 0] = page_at(t0 + u * S::kTpl + key_tok);
+                ahead_v[kLookup ? u : 0] = page_at(t0 + u * S::kTpl + tl);
             }
         };
-        auto fetch_k = [&](int t0) __attribute__((always_inline)) {
+        auto row_of = [&](int64_t page, int t) __attribute__((always_inline)) -> int64_t {
+            const int in_page = a.block_shift >= 0 ? t & (a.block_size - 1) : t % a.block_size;
+            return t < end && page >= 0 && page < a.num_blocks ? page * page_elems + (int64_t)in_page * row_elems
+                                                               : (int64_t)-1;
+        };
+        // Where the rows of the iteration at t0 are, for fetch_k and fetch_v.
+        auto fetch_page = [&](int t0) __attribute__((always_inline)) {
             if constexpr (PAGE_UNIFORM) {
-                const uint8_t* kp = static_cast<const uint8_t*>(a.key_cache) + next_base;
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const int t = t0 + h * kRun;
+                    const int64_t page = page_next[h];
+                    page_next[h] = page_of(t + kStep);
+                    const bool page_ok = page >= 0 && page < a.num_blocks;
+                    const int in_page = a.block_shift >= 0 ? t & (a.block_size - 1) : t % a.block_size;
+                    next_base[h] = page_ok ? (page * a.block_size + in_page) * (int64_t)row_bytes : 0;
+                    next_lim[h] = page_ok ? end : 0;
+                }
+            } else if constexpr (kLookup) {
+#pragma unroll
+                for (int u = 0; u < L; ++u) {
+                    next_krow[u] = row_of(ahead_k[u], t0 + u * S::kTpl + key_tok);
+                    next_vrow[u] = row_of(ahead_v[u], t0 + u * S::kTpl + tl);
+                }
+                lookup(t0 + kStep);
+            }
+        };
+        auto fetch_k = [&]() __attribute__((always_inline)) {
+            if constexpr (PAGE_UNIFORM) {
 #pragma unroll
                 for (int u = 0; u < L; ++u)
-                    mk[MM ? u : 0] = kv_load<STREAM>(kp + (key_off + (uint32_t)(u * S::kTpl * row_bytes)));
+                    mk[MM ? u : 0] = kv_load<STREAM>(static_cast<const uint8_t*>(a.key_cache) + next_base[u / kRunLoads] +
+                                                     (key_off + (uint32_t)(u % kRunLoads * S::kTpl * row_bytes)));
             } else {
 #pragma unroll
                 for (int u = 0; u < L; ++u) {
-                    const int64_t row = row_of(t0 + u * S::kTpl + key_tok);
+                    const int64_t row = next_krow[kLookup ? u : 0];
                     mk[MM ? u : 0] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
                         static_cast<const uint16_t*>(a.key_cache) + (row >= 0 ? row : 0) + kvh * D + key_dim));
                 }
             }
         };
-        auto fetch_v = [&](int t0, int u) __attribute__((always_inline)) {
+        auto fetch_v = [&](int u) __attribute__((always_inline)) {
             if constexpr (PAGE_UNIFORM) {
-                mv[MM ? u : 0] = kv_load<STREAM>(static_cast<const uint8_t*>(a.value_cache) + next_base + lane_off[u]);
+                mv[MM ? u : 0] = kv_load<STREAM>(static_cast<const uint8_t*>(a.value_cache) + next_base[u / kRunLoads] +
+                                                 lane_off[u % kRunLoads]);
             } else {
-                const int64_t row = row_of(t0 + u * S::kTpl + tl);
-                next_ok[u] = row >= 0;
+                const int64_t row = next_vrow[kLookup ? u : 0];
                 mv[MM ? u : 0] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(
                     static_cast<const uint16_t*>(a.value_cache) + (row >= 0 ? row : 0) + kvh * D + 8 * c));
             }
@@ -565,10 +616,11 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         // of 512 10.1 -> 9.6).
         if constexpr (MM)
             if (it < end) {
+                if constexpr (kLookup) lookup(it);
                 fetch_page(it);
-                fetch_k(it);
+                fetch_k();
 #pragma unroll
-                for (int u = 0; u < L; ++u) fetch_v(it, u);
+                for (int u = 0; u < L; ++u) fetch_v(u);
             }
 
         static_assert(!PRO || (S::kLpt == S::kChunks && S::kLpt >= 2), "prologue needs head_dim 16/32/64/128/256");
@@ -640,9 +692,9 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         if constexpr (PRO && MM)
             if (owner && it <= pos && pos < it + S::kTpi) {
                 __builtin_amdgcn_s_waitcnt(0);
-                fetch_k(it);
+                fetch_k();
 #pragma unroll
-                for (int u = 0; u < L; ++u) fetch_v(it, u);
+                for (int u = 0; u < L; ++u) fetch_v(u);
             }
 
         // Query operands.  Matrix tiles: column li of the score product.
@@ -700,10 +752,12 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
 
         if constexpr (MM) {
             for (; it < end; it += kStep) {
-                const int lim = next_lim;  // page-uniform: rows of the iteration at or past it are absent
-                bool ok[L];
+                bool ok[L], all = PAGE_UNIFORM;
 #pragma unroll
-                for (int u = 0; u < L; ++u) ok[u] = PAGE_UNIFORM ? it + u * S::kTpl + tl < lim : next_ok[u];
+                for (int u = 0; u < L; ++u)
+                    ok[u] = PAGE_UNIFORM ? it + u * S::kTpl + tl < next_lim[u / kRunLoads] : next_vrow[kLookup ? u : 0] >= 0;
+#pragma unroll
+                for (int h = 0; h < H; ++h) all = all && it + S::kTpi <= next_lim[h];
                 f32x4 sc[kStates][L];
 #pragma unroll
                 for (int u = 0; u < L; ++u)
@@ -714,7 +768,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 if constexpr (PRO)
                     if (owner && it + kStep <= pos && pos < it + kStep + S::kTpi) __builtin_amdgcn_s_waitcnt(0);
                 fetch_page(it + kStep);
-                fetch_k(it + kStep);
+                fetch_k();
                 float p[kStates][L];
 #pragma unroll
                 for (int t = 0; t < kStates; ++t) {
@@ -765,7 +819,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                     l[t] += (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
                 }
                 // 0 * (stale NaN) must not reach the sums.
-                if (!PAGE_UNIFORM || it + S::kTpi > lim) {
+                if (!all) {
 #pragma unroll
                     for (int u = 0; u < L; ++u)
                         if (!ok[u]) mv[u] = u32x4{0u, 0u, 0u, 0u};
@@ -785,7 +839,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                                 __builtin_amdgcn_mfma_f32_4x4x1f32(v1, pu[t], macc[t][2 * i + 1], 0, 0, 0);
                         }
                     }
-                    fetch_v(it + kStep, u);
+                    fetch_v(u);
                 }
             }
         } else {
@@ -796,8 +850,8 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             if constexpr (PRO)
                 if (owner && it <= pos && pos < it + S::kTpi) __builtin_amdgcn_s_waitcnt(0);
             if constexpr (PAGE_UNIFORM) {
-                const int64_t page = page_next;
-                page_next = page_of(it + kStep);
+                const int64_t page = page_next[0];
+                page_next[0] = page_of(it + kStep);
                 const bool page_ok = page >= 0 && page < a.num_blocks;
                 const int in_page = a.block_shift >= 0 ? it & (a.block_size - 1) : it % a.block_size;
 #pragma unroll
@@ -1031,6 +1085,8 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
 
 template <typename T, int D, int G, int NW, bool STREAM, bool PRO>
 void launch_decode_kernel(const DecodeArgs& a, dim3 grid, bool page_uniform, hipStream_t s) {
+    // page_uniform: pages hold whole iterations; here whole runs are enough.
+    if (page_runs<D, G>() > 1) page_uniform = a.block_size % (DecodeShape<D>::kTpi / page_runs<D, G>()) == 0;
     if constexpr (NW == kFlatWaves && STREAM) {
         if (a.flat_groups > 0) {
             if (page_uniform)

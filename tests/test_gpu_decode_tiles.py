@@ -125,3 +125,29 @@ def test_partitions_decided_by_the_lengths(lengths, kv_heads, group):
     write_kv_cache_batch(k2, v2, table, lens - 1, new_k, new_v, block, validate=False)
     assert torch.equal(key, k2) and torch.equal(value, v2)
     assert torch.equal(fused, paged_attention(q, k2, v2, table, lens, block, validate=False))
+
+
+@pytest.mark.parametrize("block", [8, 16, 24, 32, 48, 17])
+@pytest.mark.parametrize("dim,group", [(64, 2), (64, 4), (64, 8), (128, 4)])
+def test_runs_of_pages(block, dim, group):
+    """Iterations of 32 tokens at 64 dims cover two runs of 16, each in a page
+    of its own; contexts end inside the first and the second run, and absent
+    pages lie under either."""
+    dtype = torch.float16
+    args = list(decode_inputs(dtype, head_dim=dim, block_size=block, lengths=(1, 16, 17, 31, 32, 33, 49, 300, 530),
+                              heads=2 * group, kv_heads=2, seed=block + dim))
+    for partition in (0, 128, -1):
+        check(args, dtype, partition)
+    q, k, v, table, lens, _ = [a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args]
+    for bad, hole in ((-1, 0), (k.shape[0], 1), (1 << 33, 2)):
+        holed = table.clone()
+        holed[7, hole] = bad
+        out = paged_attention(q, k, v, holed, lens, block, validate=False).float().cpu()
+        rows = torch.arange(300).div(block, rounding_mode="floor") != hole
+        pages = args[3][7].repeat_interleave(block)[:300][rows]
+        offsets = (torch.arange(300) % block)[rows]
+        keys, values = args[1][pages, offsets].float(), args[2][pages, offsets].float()
+        query = args[0][7].float().view(2, group, dim)
+        scores = torch.einsum("hgd,thd->hgt", query, keys) / dim ** 0.5
+        want = torch.einsum("hgt,thd->hgd", scores.softmax(-1), values).reshape(2 * group, dim)
+        assert (out[7] - want).abs().max().item() <= GATE[dtype]
