@@ -390,6 +390,35 @@ void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim) {
 
 constexpr int64_t kEvenCapacity = 2048;
 
+// Smallest K+V capacity of a 128-dim unit from which the balanced walk takes a plan of
+// `units` units, in bytes; 0: none.  us per call, other plan -> walk (16/8
+// heads, bf16, pages of 16; first ragged U[1,ctx], then all ctx):
+// * fewer units than CUs (split-K): 2048 tokens (1 MiB) 24 sequences 23.0 ->
+//   28.0, 39.2 -> 39.6; 2600 tokens 24.4 -> 23.7, 34.6 -> 32.9 (16 sequences),
+//   32.2 -> 28.5, 49.6 -> 46.1 (24); 4000 tokens 50.2 -> 39.9, 70.3 -> 67.4.
+// * one unit per CU: 1400 tokens, 32 sequences 23.7 -> 24.3, 32.0 -> 33.2; 2048
+//   tokens 34.9 -> 30.2, 46.3 -> 45.2; 4000 tokens 60.0 -> 52.3.
+// * up to 1.25 per CU, some CUs with two units and others with one: 34
+//   sequences of 1000 25.2 -> 22.3, 35.7 -> 29.3, of 4000 81.1 -> 55.0, 131.4 ->
+//   90.9; 40 of 1000 25.1 -> 25.5, 38.6 -> 33.6.
+// * up to 1.5: 48 of 1000 25.8 -> 27.8, 41.3 -> 39.2; of 2000 44.5 -> 42.9, 76.1
+//   -> 66.6.
+// * up to 1.9: 56 of 2000 46.8 -> 48.2, 81.3 -> 77.5; of 4000 86.3 -> 82.4,
+//   157.0 -> 146.7; two per CU (64 of 4000) 90.8 -> 92.3: none.
+// The walk's pieces of 8-head tiles end more slowly: up to one unit per CU 62
+// sequences of 3000 (28/4 heads) 53.8 -> 51.8, 64 of 2048 (32/4) 40.5 -> 50.2;
+// above, 48 of 4000 (40/8) 84.3 -> 81.9, 40 of 2000 38.7 -> 47.0.
+int64_t walk_unit_bytes(int64_t units, int gtile) {
+    const int64_t mib = int64_t(1) << 20;
+    const bool one_per_cu = units >= kDeviceCUs - kDeviceCUs / 16 && units <= kDeviceCUs;
+    if (gtile == 8) return one_per_cu ? mib * 3 / 2 : units <= kDeviceCUs * 3 / 2 ? 2 * mib : 0;
+    if (units < kDeviceCUs * 3 / 8) return 2 * mib;
+    if (units <= kDeviceCUs) return mib * 5 / 4;
+    if (units <= kDeviceCUs * 5 / 4) return mib / 2;
+    if (units <= kDeviceCUs * 3 / 2) return mib;
+    return units <= kDeviceCUs * 15 / 8 ? mib * 3 / 2 : 0;
+}
+
 // Partition length of a split over tiles of 1 to 4 heads of 128: the number of
 // partitions n that minimises the iterations the busiest CU runs, half at full
 // tables and half at tables filled a little over half (ragged batches), plus
@@ -414,8 +443,9 @@ int64_t split_partition(int64_t cap, int64_t units, int64_t step) {
 }
 
 // Host-side plan (lengths stay on the device, so it depends on the table
-// capacity only).  Long units (kLongUnitBytes of K+V capacity) numbering at
-// most one per CU take the balanced walk.  Otherwise, enough (sequence, kv
+// capacity only).  Long units (walk_unit_bytes) take the balanced walk, unless
+// `walk` is off, where only units of kLongUnitBytes numbering at most one per
+// CU do (what a call without room for the walk's partials had).  Otherwise, enough (sequence, kv
 // head) units to occupy every CU, a capacity of one 16-wave step, or two
 // steps with more than a quarter of the CUs' worth of units: one work-group
 // per unit over the whole context, merged in LDS (8 waves; with two
@@ -439,7 +469,7 @@ int64_t split_partition(int64_t cap, int64_t units, int64_t step) {
 //   x 64: 11.61 -> 9.93 at 128; 2048 x 32: 11.56 -> 10.48 at 128); the
 //   earlier plan took at least 256 keys for a target of 1024 work-groups.
 DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
-                            int64_t block_size, int64_t table_width, int64_t requested) {
+                            int64_t block_size, int64_t table_width, int64_t requested, bool walk = true) {
     DecodePlan p{};
     const int64_t group = q_heads / kv_heads;
     plan_tiles(p, group, head_dim);
@@ -478,23 +508,16 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
     }
     p.partition = (int)part;
     p.max_parts = (int)((cap + part - 1) / part);
-    // Long units (kLongUnitBytes of K+V capacity or more) numbering at most
-    // one per CU, or a request (requested == -1), take the balanced walk.
-    // With one work-group per unit the CUs holding the shortest units idle
-    // while the longest stream alone, whatever the order: 32 sequences of
-    // contexts U[1,4096] (fp16, block 256) 70.5 -> 62.5 µs per call, all 4096
-    // tokens 84.3 -> 84.6.  Fewer units, which split-K cuts into partitions
-    // sized by capacity, leave ragged batches with empty partitions and
-    // uneven CUs (bf16, block 16 unless noted, µs per call, split-K ->
-    // walk): 24 sequences U[1,4096] 60.8 -> 47.3, 16 U[1,8192] 58.1 -> 46.4,
-    // 8 U[1,8192] fp16 block 256 30.1 -> 27.4, 4 U[1,32768] block 256 61.5
-    // -> 56.9; equal lengths cost the walk 2-6 % (8 x 4096 26.2 -> 27.7, 1 x
-    // 32768 block 256 28.5 -> 29.7) and short capacities more (8 x 512 8.4
-    // -> 9.6), so those keep split-K.  With two or more units per CU the
-    // longest-first order already balances the CUs, and the walk was slower
-    // (64 sequences U[1,4096] sharing a 1024-token prefix, bf16, block 16:
-    // 88.1 -> 90.5 µs; 128 sequences U[1,4096]: 166.4 -> 169.2).
-    const bool long_units = (double)cap * (double)head_dim * 4.0 >= (double)kLongUnitBytes;
+    // Long units (walk_unit_bytes) or a request (requested == -1) take the
+    // balanced walk.  With one work-group per unit the CUs holding the shortest
+    // units, or one unit where others hold two, idle while the rest stream
+    // alone, whatever the order; split-K partitions sized by capacity leave
+    // ragged batches with empty partitions and uneven CUs.  With two units per
+    // CU the longest-first order already balances them.
+    const int64_t long_bytes = walk && head_dim == 128 ? walk_unit_bytes(units, p.gtile)
+                               : units <= kDeviceCUs   ? kLongUnitBytes
+                                                       : 0;
+    const bool long_units = long_bytes > 0 && (double)cap * (double)head_dim * 4.0 >= (double)long_bytes;
     // Even parts: 8-head tiles over tables of 2048 tokens and more.
     const bool even = requested <= 0 && requested != -1 && !whole && p.gtile == 8 && head_dim == 128 && batch <= kWave &&
                       cap >= kEvenCapacity;
@@ -504,7 +527,7 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
         p.max_parts = 1;
     }
     const bool flat = !even && batch <= kLptMax &&
-                      (requested == -1 || (requested <= 0 && long_units && units <= kDeviceCUs));
+                      (requested == -1 || (requested <= 0 && long_units));
     if (flat) {
         p.flat_groups = kFlatGroups;
         p.waves = kFlatWaves;
@@ -629,9 +652,11 @@ int check_decode_shapes(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_
 
 using namespace mvme;
 
-extern "C" size_t mvme_paged_attention_workspace_size(int64_t batch, int64_t q_heads, int64_t kv_heads,
-                                                      int64_t head_dim, int64_t block_size,
-                                                      int64_t table_width, int64_t partition_tokens) {
+namespace mvme {
+namespace {
+
+size_t decode_workspace(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t block_size,
+                        int64_t table_width, int64_t partition_tokens, bool walk) {
     if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || block_size <= 0 ||
         table_width <= 0 || decode_tile_tokens(head_dim) == 0)
         return 0;
@@ -641,7 +666,7 @@ extern "C" size_t mvme_paged_attention_workspace_size(int64_t batch, int64_t q_h
         batch > kMaxBatchHeads || q_heads > kMaxBatchHeads || batch * q_heads > kMaxBatchHeads)
         return 0;
     const DecodePlan p = make_decode_plan(batch, q_heads, kv_heads, head_dim, block_size, table_width,
-                                          partition_tokens);
+                                          partition_tokens, walk);
     if (p.flat_groups > 0)
         return (size_t)p.flat_groups * 2 * p.gtile * (head_dim + 2) * sizeof(float) +
                (size_t)p.flat_groups * sizeof(FlatMergeDesc);
@@ -649,6 +674,30 @@ extern "C" size_t mvme_paged_attention_workspace_size(int64_t batch, int64_t q_h
         return (size_t)p.even_slots * kv_heads * p.gtiles * p.gtile * (head_dim + 2) * sizeof(float);
     if (p.max_parts <= 1) return 0;
     return (size_t)batch * q_heads * p.max_parts * (head_dim + 2) * sizeof(float);
+}
+
+// A caller's workspace too small (or misaligned) for a plan that the walk's
+// longer reach gave it: `walk` off, the plan without it, which needs less or
+// none.  Returns what the chosen plan needs.
+size_t fit_workspace(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t block_size,
+                     int64_t table_width, int64_t partition_tokens, const void* workspace, size_t bytes,
+                     bool& walk) {
+    walk = true;
+    const size_t need = decode_workspace(batch, q_heads, kv_heads, head_dim, block_size, table_width,
+                                         partition_tokens, true);
+    if (need == 0 || (workspace != nullptr && bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0))
+        return need;
+    walk = false;
+    return decode_workspace(batch, q_heads, kv_heads, head_dim, block_size, table_width, partition_tokens, false);
+}
+
+}  // namespace
+}  // namespace mvme
+
+extern "C" size_t mvme_paged_attention_workspace_size(int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                                      int64_t head_dim, int64_t block_size,
+                                                      int64_t table_width, int64_t partition_tokens) {
+    return decode_workspace(batch, q_heads, kv_heads, head_dim, block_size, table_width, partition_tokens, true);
 }
 
 namespace mvme {
@@ -673,9 +722,10 @@ int launch_paged_attention(void* out, const void* query, const void* key_cache, 
                            const int64_t* block_tables, const int64_t* context_lens, int64_t batch,
                            int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t num_blocks,
                            int64_t block_size, int64_t table_width, int64_t partition_tokens, int dtype,
-                           size_t need, void* workspace, void* stream, const DecodePrologue* pro = nullptr) {
+                           size_t need, bool walk, void* workspace, void* stream,
+                           const DecodePrologue* pro = nullptr) {
     const DecodePlan p = make_decode_plan(batch, q_heads, kv_heads, head_dim, block_size, table_width,
-                                          partition_tokens);
+                                          partition_tokens, walk);
     const int64_t group = q_heads / kv_heads;
     const int64_t units = batch * kv_heads * p.gtiles;
     if (units > 2147483647) return fail(MVME_EINVAL, "batch/head product too large");
@@ -786,14 +836,15 @@ extern "C" int mvme_paged_attention(void* out, const void* query, const void* ke
         return rc;
     if (!out || !query || !key_cache || !value_cache || !block_tables || !context_lens)
         return fail(MVME_EINVAL, "paged attention received a null pointer");
-    const size_t need = mvme_paged_attention_workspace_size(batch, q_heads, kv_heads, head_dim, block_size,
-                                                            table_width, partition_tokens);
+    bool walk;
+    const size_t need = fit_workspace(batch, q_heads, kv_heads, head_dim, block_size, table_width,
+                                      partition_tokens, workspace, workspace_bytes, walk);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need))
         return fail(MVME_EWORKSPACE, "paged attention workspace too small: need " + std::to_string(need) +
                                          " bytes, got " + std::to_string(workspace_bytes));
     return launch_paged_attention(out, query, key_cache, value_cache, block_tables, context_lens, batch,
                                   q_heads, kv_heads, head_dim, num_blocks, block_size, table_width,
-                                  partition_tokens, dtype, need, workspace, stream);
+                                  partition_tokens, dtype, need, walk, workspace, stream);
 }
 
 namespace {
@@ -841,8 +892,9 @@ extern "C" int mvme_paged_attention_decode_write(
         if (o_lo < q_hi && q_lo < o_hi)
             return fail(MVME_EINVAL, "q_out must not overlap the raw query rows");
     }
-    const size_t need = mvme_paged_attention_workspace_size(batch, q_heads, kv_heads, head_dim, block_size,
-                                                            table_width, partition_tokens);
+    bool walk;
+    const size_t need = fit_workspace(batch, q_heads, kv_heads, head_dim, block_size, table_width,
+                                      partition_tokens, workspace, workspace_bytes, walk);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need))
         return fail(MVME_EWORKSPACE, "paged attention workspace too small: need " + std::to_string(need) +
                                          " bytes, got " + std::to_string(workspace_bytes));
@@ -861,7 +913,7 @@ extern "C" int mvme_paged_attention_decode_write(
     pro.eps = eps;
     return launch_paged_attention(out, query, key_cache, value_cache, block_tables, context_lens, batch,
                                   q_heads, kv_heads, head_dim, num_blocks, block_size, table_width,
-                                  partition_tokens, dtype, need, workspace, stream, &pro);
+                                  partition_tokens, dtype, need, walk, workspace, stream, &pro);
 }
 
 extern "C" int mvme_paged_attention_noalloc(void* out, const void* query, const void* key_cache,
@@ -875,6 +927,7 @@ extern "C" int mvme_paged_attention_noalloc(void* out, const void* query, const 
         return rc;
     if (!out || !query || !key_cache || !value_cache || !block_tables || !context_lens)
         return fail(MVME_EINVAL, "paged attention received a null pointer");
+    const bool walk = true;
     const size_t need = mvme_paged_attention_workspace_size(batch, q_heads, kv_heads, head_dim, block_size,
                                                             table_width, partition_tokens);
     if (need > kScratchBytes)
@@ -886,5 +939,5 @@ extern "C" int mvme_paged_attention_noalloc(void* out, const void* query, const 
         if (int rc = device_scratch(&workspace)) return rc;
     return launch_paged_attention(out, query, key_cache, value_cache, block_tables, context_lens, batch,
                                   q_heads, kv_heads, head_dim, num_blocks, block_size, table_width,
-                                  partition_tokens, dtype, need, workspace, stream);
+                                  partition_tokens, dtype, need, walk, workspace, stream);
 }
