@@ -61,7 +61,7 @@ constexpr int kLptMax = 256;     // largest batch whose units go longest context
 static_assert(kSplitWaves * kWave >= kLptMax, "one thread per sequence key");
 constexpr int kDecodeLoads = 4;  // K (and V) loads per lane per iteration
 // Balanced walk: waves per work-group (its own kernel instances, with
-// non-temporal loads: the plan takes the walk for calls of 480 MiB or more).
+// non-temporal loads, as long units are read once).
 constexpr int kFlatWaves = kWholeWaves;
 
 template <int D>
