@@ -591,10 +591,10 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
     constexpr bool WAVE_PAGES = PAGES == kPagesPerWave;
     constexpr bool PIPE = (PAGES == kPagesPerTile || WAVE_PAGES) && !NARROW && HD <= 128;
     // Queries scaled once by scale*log2(e) (one more rounding of q) instead
-    // of every score in fp32.  The modes that joined the pipelined loop later
-    // (small pages 127.9 -> 111.2 us for 16 sequences of 56..900 tokens with
-    // their norm, rotation and write; a dense 8192-token prompt 255.3 -> 239.4)
-    // scale in fp32, which they did before: their error stays what it was.
+    // of every score in fp32, and row sums of the 16-bit probabilities from
+    // the matrix core.  The modes that joined the pipelined loop later scale
+    // and sum in fp32, which they did before: rounded to fp16, the many tiny
+    // probabilities of a long row with a few large ones are all 0.
     constexpr bool PRESCALE = PAGES == kPagesPerTile && !DENSE;
     const int hd = NARROW ? a.head_dim : SH::kD;  // elements per K/V/Q/output row in memory
     const int dchunks = hd / 8;                 // 16-byte chunks per row
@@ -998,7 +998,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
             }
             __builtin_amdgcn_s_setprio(0);
         };
-        // O^T += V^T P^T of a tile (V stage st), and the row sums.
+        // O^T += V^T P^T of a tile (V stage st), and with PRESCALE the row sums.
         auto pv_product = [&](int st) __attribute__((always_inline)) {
             typedef __attribute__((address_space(3))) uint8_t lds_u8;
             lds_u8* vbase = (lds_u8*)&sm_v[st][0];
@@ -1030,7 +1030,7 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                 for (int h = 0; h < SH::kHalves; ++h) vcur[h] = vnext[h];
             }
 #pragma unroll
-            for (int nb = 0; nb < SH::kNb; ++nb) {
+            for (int nb = 0; nb < (PRESCALE ? SH::kNb : 0); ++nb) {
 #pragma unroll
                 for (int h = 0; h < SH::kHalves; ++h) osum[nb] = T::mfma16x16x32(ones, pops[h][nb], osum[nb]);
                 __builtin_amdgcn_sched_barrier(0);
@@ -1041,10 +1041,11 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
         // biased first unless every key is present and visible to every row
         // of the wave.  p = 2^sc; the exact step (row maxima, rescale of what
         // is accumulated, new probabilities) runs when a row sees its first
-        // key or some probability, rounded to the operand type, exceeds 2^8
-        // (inf and NaN included: as 16-bit patterns of non-negative values
-        // they order above 256, so an unsigned maximum of the packed halves
-        // decides).  `first`:
+        // key or its probabilities grow too large: with PRESCALE when one,
+        // rounded to the operand type, exceeds 2^8 (inf and NaN included: as
+        // 16-bit patterns of non-negative values they order above 256, so an
+        // unsigned maximum of the packed halves decides), otherwise when the
+        // fp32 sum of 8 does, which the row sums need anyway.  `first`:
         // the item's first tile, where nothing is accumulated yet (every
         // rescale factor is 1, so the rescale is skipped).
         auto softmax_tile = [&](int tile, int st, bool first) __attribute__((always_inline)) {
@@ -1069,8 +1070,15 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                     }
             }
             bool need = false;
+            float dl[SH::kNb];  // the lane's share of the tile's row sums (without PRESCALE)
+            auto sum8 = [](const float (&p)[8]) __attribute__((always_inline)) -> float {
+                return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+            };
 #pragma unroll
-            for (int nb = 0; nb < SH::kNb; ++nb) need = need | ((m_run[nb] == kNegInf) & (pos[nb] >= tile0));
+            for (int nb = 0; nb < SH::kNb; ++nb) {
+                need = need | ((m_run[nb] == kNegInf) & (pos[nb] >= tile0));
+                dl[nb] = 0.f;
+            }
 #pragma unroll
             for (int h = 0; h < SH::kHalves; ++h)
 #pragma unroll
@@ -1083,7 +1091,11 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                             p[4 * kk + j] = fast_exp2(PRESCALE ? sc[h][nb][kk][j]
                                                                : fmaf(sc[h][nb][kk][j], a.scale_log2, nref[nb]));
                     pops[h][nb] = u32x4{T::pack(p[0], p[1]), T::pack(p[2], p[3]), T::pack(p[4], p[5]), T::pack(p[6], p[7])};
-                    {
+                    if constexpr (!PRESCALE) {
+                        const float d = sum8(p);
+                        need = need | !(d <= kPSumLimit);
+                        dl[nb] += d;
+                    } else {
                         typedef unsigned short us2 __attribute__((ext_vector_type(2)));
                         us2 m = __builtin_elementwise_max(__builtin_bit_cast(us2, pops[h][nb][0]),
                                                           __builtin_bit_cast(us2, pops[h][nb][1]));
@@ -1110,10 +1122,12 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                     m_run[nb] = mn;
                     nref[nb] = mn == kNegInf ? 0.f : -mn;
                     if (!first) {
-                        osum[nb] *= alpha;
+                        if constexpr (PRESCALE) osum[nb] *= alpha;
+                        else l_part[nb] *= alpha;
 #pragma unroll
                         for (int dt = 0; dt < SH::kDt; ++dt) o[nb][dt] *= alpha;
                     }
+                    dl[nb] = 0.f;
 #pragma unroll
                     for (int h = 0; h < SH::kHalves; ++h) {
                         float p[8];
@@ -1125,9 +1139,13 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
                                                                    : fmaf(sc[h][nb][kk][j], a.scale_log2, nref[nb]));
                         pops[h][nb] =
                             u32x4{T::pack(p[0], p[1]), T::pack(p[2], p[3]), T::pack(p[4], p[5]), T::pack(p[6], p[7])};
+                        if constexpr (!PRESCALE) dl[nb] += sum8(p);
                     }
                 }
             }
+            if constexpr (!PRESCALE)
+#pragma unroll
+                for (int nb = 0; nb < SH::kNb; ++nb) l_part[nb] += dl[nb];
         };
 
         // Split barrier of the loop.  A wave arrives (one LDS count) once its
@@ -1477,8 +1495,8 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
 
 #pragma unroll
     for (int nb = 0; nb < SH::kNb; ++nb) {
-        // The pipelined loop's sums come from the matrix core, whole per lane.
-        const float l_row = PIPE ? osum[nb][0] : row4_sum(l_part[nb]);
+        // Sums from the matrix core are whole per lane.
+        const float l_row = PIPE && PRESCALE ? osum[nb][0] : row4_sum(l_part[nb]);
         if (qi[nb] >= qlen) continue;
         const int64_t rowid = (row0 + qi[nb]) * a.q_heads + head[nb];
         if (nchunks == 1) {

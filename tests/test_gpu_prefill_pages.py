@@ -2,6 +2,8 @@
 tile (8, 16 and 32 tokens) and in dense mode, and of the order of query
 blocks across sequences."""
 
+import math
+
 import pytest
 import torch
 
@@ -120,3 +122,34 @@ def test_head_dim_64_dense(batch, tokens, start, view):
     actual = prefill_attention(*dev, query_start=start).float().cpu()
     expected = paged_oracle.prefill_attention(*[t.transpose(1, 2) for t in (q, k, v)], query_start=start, cast=False)
     assert (actual - expected).abs().max().item() <= GATE[dtype]
+
+
+def peaked_row(keys, dim):
+    """One query whose first key has probability ~1 and the others 2^-25.2 each, below
+    half of fp16's smallest number; V is 1 at the first key and 0 elsewhere.  Returns
+    q [dim], K, V [keys, dim] and the exact output."""
+    q, k, v = torch.zeros(dim), torch.zeros(keys, dim), torch.zeros(keys, dim)
+    q[0], k[0, 0], v[0] = 16.0, 25.2 * math.log(2) * dim ** 0.5 / 16, 1.0
+    q, k, v = q.half(), k.half(), v.half()
+    exact = 1 / (1 + (keys - 1) * math.exp(-float(q[0]) * float(k[0, 0]) / dim ** 0.5))
+    return q, k, v, exact
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("mode", [8, 32, "dense"])
+def test_row_sums_hold_tiny_probabilities(mode, dim):
+    """65535 keys of probability 2^-25.2 are 0.17 % of the row's sum, 3.5 spacings of
+    fp16 below 1: sums of probabilities rounded to fp16 lose all of it.  The bound is
+    half a spacing of the output and 1e-5 for the sum's own fp32 roundings."""
+    keys = 65536
+    q, k, v, exact = peaked_row(keys, dim)
+    if mode == "dense":
+        # 384 rows of work, so that keys are not split; every row reads the same keys.
+        wide = [t.to(DEV)[None, None].expand(48, 8, keys, dim) for t in (k, v)]
+        out = prefill_attention(q.to(DEV).expand(48, 8, 1, dim).contiguous(), *wide, query_start=keys - 1)
+    else:
+        pages = [t.to(DEV).view(keys // mode, mode, 1, dim) for t in (k, v)]
+        meta = [[0, 1], [keys - 1], [list(range(keys // mode))], [keys]]
+        out = paged_prefill_attention(q.to(DEV)[None, None], *pages, *[torch.tensor(m).to(DEV) for m in meta], mode,
+                                      chunk_tokens=keys)
+    assert (out.double() - exact).abs().max().item() <= 2.0 ** -12 + 1e-5
