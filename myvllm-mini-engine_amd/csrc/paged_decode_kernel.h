@@ -781,10 +781,12 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                         if constexpr (S::kParts == 4) {
                             // Lane li has the partial of part li / 4; its
                             // token's other parts are in lanes li +- 4, 8.
+                            // The pairs 8 apart first: then all four lanes add
+                            // the same two sums, and get the same bits.
                             const float lo = (li & 4) ? sc[t][u][1] : sc[t][u][0], hi = (li & 4) ? sc[t][u][3] : sc[t][u][2];
                             d = (li & 8) ? hi : lo;
-                            d += dpp<kDppRowRor4>(d);
                             d += dpp<kDppRowRor8>(d);
+                            d += dpp<kDppRowRor4>(d);
                         } else {
                             // Rows 4 lg + 0, 1: token 2 lg's parts; + 2, 3:
                             // token 2 lg + 1's.  Lanes 0..7 keep the first

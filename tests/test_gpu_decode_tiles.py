@@ -77,6 +77,27 @@ def test_scores_that_keep_rising_and_stale_rows(dim, group):
         assert (actual - oracle(clean)).abs().max().item() <= GATE[dtype]
 
 
+@pytest.mark.parametrize("dim,group", [(64, 4), (64, 8), (128, 2), (128, 4), (128, 7)])
+def test_one_score_for_all_of_a_tokens_lanes(dim, group):
+    """Scores near 2^13 binary orders that differ by a few: a lane that rounded its
+    token's score otherwise than its neighbours gives the dims it holds other weights
+    than the sum has, 2^-10 apart.  With V all 1 every output is the weights' sum over
+    itself, 1 to the few fp32 roundings by which the two sums' orders differ."""
+    gen = torch.Generator().manual_seed(dim + group)
+    args = list(decode_inputs(torch.float16, head_dim=dim, lengths=(5, 11, 20, 30, 48, 100, 200, 300) * 4,
+                              heads=8 * group, kv_heads=8))
+    q, key, value = args[:3]
+    sign = torch.randint(0, 2, (8, dim), generator=gen) * 2.0 - 1
+    scale = 40 * (128 / dim) ** 0.5
+    q.copy_((sign * scale).repeat_interleave(group, 0) * (1 + 0.01 * torch.randn(q.shape, generator=gen)))
+    key.copy_(20 * sign + 0.03 * key.float())
+    value.fill_(1.0)
+    dev = [a.to(DEV) if isinstance(a, torch.Tensor) else a for a in args]
+    for partition in (0, 64, -1):
+        out = paged_attention(*dev, partition_tokens=partition)
+        assert torch.equal(out, torch.ones_like(out))
+
+
 def test_absent_pages_and_lengths_count_as_nothing():
     """Trusted calls with pages and lengths out of range: those tokens are
     absent, a sequence without any gives zeros."""
