@@ -123,7 +123,7 @@ def write_kv_cache_slots(key_cache, value_cache, slot_mapping, key, value,
     may be strided views whose per-token [kv_heads, head_dim] rows are dense.
     """
     _backend(backend)
-    if not validate and ext.native_calls().write_slots(key_cache, value_cache, slot_mapping, key, value):
+    if not validate and ext.native.write_slots(key_cache, value_cache, slot_mapping, key, value):
         return
     if (key_cache.ndim != 4 or value_cache.shape != key_cache.shape
             or any(size <= 0 for size in key_cache.shape)

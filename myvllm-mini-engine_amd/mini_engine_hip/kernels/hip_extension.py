@@ -109,12 +109,28 @@ def check_build_digest(digest_file, expected: str) -> None:
                            f"python -m mini_engine_hip.build")
 
 
+class NoNativeCalls:
+    """Stands for the native call path until the library is loaded: declines every call."""
+
+    def _decline(self, *args):
+        return None
+
+    decode = decode_write = prefill = dense = linear = rope_slots = write_slots = _decline
+
+
+# What the entry points ask first; `load_hip_extension` puts the native call
+# path here.  The first call of a process therefore runs the Python code, and a
+# call that is refused, or that needs no library, never loads one.
+native = NoNativeCalls()
+
+
 @functools.lru_cache(maxsize=1)
 def load_hip_extension() -> HipLibrary:
     """Load the prebuilt library; build it first only if no build exists.
 
     An existing library must carry the digest of the current sources.
     """
+    global native
     path = _build.library_path()
     if not path.exists():
         _build.build_library()
@@ -123,7 +139,9 @@ def load_hip_extension() -> HipLibrary:
         lib = ctypes.CDLL(str(path))
     except OSError as error:
         raise RuntimeError(f"cannot load the HIP paged-attention library {path}: {error}") from error
-    return HipLibrary(lib, path)
+    library = HipLibrary(lib, path)
+    native = _bind_native(library)
+    return library
 
 
 # Entry points of the native call path (csrc/host_calls.cpp), in its order.
@@ -135,14 +153,7 @@ _HOST_ENTRY_POINTS = ("mvme_last_error", "mvme_paged_attention_workspace_size", 
 
 
 @functools.lru_cache(maxsize=1)
-def native_calls():
-    """The entry points' native call path: functions that run a plain call
-    (dense CUDA tensors of the current device, no caller-supplied buffers, no
-    host-synchronising validation) and return None for any other, which the
-    Python code then checks and runs.  Measured, us per call: a decode call of
-    one 128-token sequence 14.6 -> 4.6, a decode step of 8 sequences 29.0 ->
-    9.8, which is then the GPU's time."""
-    lib = load_hip_extension()
+def _host_module():
     path = _build.host_path()
     loader = importlib.machinery.ExtensionFileLoader("mvme_host", str(path))
     spec = importlib.util.spec_from_file_location("mvme_host", str(path), loader=loader)
@@ -151,9 +162,25 @@ def native_calls():
         loader.exec_module(module)
     except (ImportError, OSError) as error:
         raise RuntimeError(f"cannot load the native call path {path}: {error}") from error
-    module.bind(torch._C._cuda_getCurrentRawStream,
-                tuple(ctypes.cast(getattr(lib._lib, name), _vp).value for name in _HOST_ENTRY_POINTS))
     return module
+
+
+def _bind_native(library):
+    module = _host_module()
+    module.bind(torch._C._cuda_getCurrentRawStream,
+                tuple(ctypes.cast(getattr(library._lib, name), _vp).value for name in _HOST_ENTRY_POINTS))
+    return module
+
+
+def native_calls():
+    """The entry points' native call path: functions that run a plain call
+    (dense CUDA tensors of the current device, no caller-supplied buffers, no
+    host-synchronising validation) and return None for any other, which the
+    Python code then checks and runs.  Measured, us per call: a decode call of
+    one 128-token sequence 14.6 -> 4.6, a decode step of 8 sequences 29.0 ->
+    9.8, which is then the GPU's time."""
+    load_hip_extension()
+    return native
 
 
 def dtype_code(dtype: torch.dtype) -> int:

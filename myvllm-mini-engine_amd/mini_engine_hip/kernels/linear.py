@@ -21,7 +21,7 @@ MAX_ROWS = 64
 def linear_rows(x, weight, bias=None, *, out=None):
     """out[m] = x[m] @ weight.T (+ bias) for a 2-D ``x`` of at most 64 rows."""
     if out is None:
-        result = ext.native_calls().linear(x, weight, bias)
+        result = ext.native.linear(x, weight, bias)
         if result is not None:
             return result
     if not x.is_cuda or not weight.is_cuda:
@@ -65,7 +65,7 @@ class HipLinear(nn.Linear):
     backend = "hip"
 
     def forward(self, x):
-        result = ext.native_calls().linear(x, self.weight, self.bias)
+        result = ext.native.linear(x, self.weight, self.bias)
         if result is not None:
             return result
         if not x.is_cuda or not self.weight.is_cuda:

@@ -82,8 +82,8 @@ def paged_attention(query, key_cache, value_cache, block_tables, context_lens, b
     if backend != "hip":
         raise ValueError("decode backend must be hip")
     if not validate and out is None and workspace is None:
-        result = ext.native_calls().decode(query, key_cache, value_cache, block_tables, context_lens, block_size,
-                                           partition_tokens)
+        result = ext.native.decode(query, key_cache, value_cache, block_tables, context_lens, block_size,
+                                   partition_tokens)
         if result is not None:
             return result
     if query.dtype not in (torch.float16, torch.bfloat16):
@@ -142,9 +142,9 @@ def paged_attention_decode_write(query, key_cache, value_cache, block_tables, co
     if backend != "hip":
         raise ValueError("decode backend must be hip")
     if not validate and out is None and workspace is None and q_out is None:
-        result = ext.native_calls().decode_write(query, key_cache, value_cache, block_tables, context_lens, block_size,
-                                                 new_key, new_value, q_weight, k_weight, cos, sin, eps,
-                                                 partition_tokens)
+        result = ext.native.decode_write(query, key_cache, value_cache, block_tables, context_lens, block_size,
+                                         new_key, new_value, q_weight, k_weight, cos, sin, eps,
+                                         partition_tokens)
         if result is not None:
             return result
     from .data import _row_stride, write_kv_cache_batch

@@ -47,8 +47,8 @@ def paged_prefill_attention(q, key_cache, value_cache, cu_seqlens_q, query_start
     if backend != "hip":
         raise ValueError("paged prefill backend must be hip")
     if not validate and workspace is None:
-        result = ext.native_calls().prefill(q, key_cache, value_cache, cu_seqlens_q, query_starts, block_tables,
-                                            context_lens, block_size, chunk_tokens)
+        result = ext.native.prefill(q, key_cache, value_cache, cu_seqlens_q, query_starts, block_tables,
+                                    context_lens, block_size, chunk_tokens)
         if result is not None:
             return result
     if (type(block_size) is not int or block_size <= 0 or key_cache.ndim != 4
@@ -174,7 +174,7 @@ def prefill_attention(q, k, v, backend="hip", *, query_start=0, out=None, worksp
     if backend != "hip":
         raise ValueError("unknown prefill backend")
     if out is None and workspace is None:
-        result = ext.native_calls().dense(q, k, v, query_start)
+        result = ext.native.dense(q, k, v, query_start)
         if result is not None:
             return result
     if (q.ndim != 4 or k.ndim != 4 or k.shape != v.shape or k.shape[1] == 0

@@ -49,8 +49,8 @@ def qk_norm_rope_write_kv(q, k, v, q_weight, k_weight, cos, sin, key_cache, valu
     if (slot_mapping is None) == (positions is None):
         raise ValueError("pass either slot_mapping or block_tables with positions")
     if slot_mapping is not None and not validate and out is None:
-        result = ext.native_calls().rope_slots(q, k, v, q_weight, k_weight, cos, sin, key_cache, value_cache,
-                                               slot_mapping, eps)
+        result = ext.native.rope_slots(q, k, v, q_weight, k_weight, cos, sin, key_cache, value_cache,
+                                       slot_mapping, eps)
         if result is not None:
             return result
     if q.ndim != 3 or k.ndim != 3 or q.shape[0] != k.shape[0] or q.shape[2] != k.shape[2]:

@@ -2,9 +2,13 @@
 takes gives the same bits as the same call with caller-supplied buffers (which
 it leaves to the Python code), and it declines everything else."""
 
+import subprocess
+import sys
+
 import pytest
 import torch
 
+from mini_engine_hip.build import PACKAGE_DIR as PACKAGE
 from mini_engine_hip.kernels import hip_extension as ext
 from mini_engine_hip.kernels.data import write_kv_cache_slots
 from mini_engine_hip.kernels.linear import linear_rows
@@ -13,6 +17,7 @@ from mini_engine_hip.kernels.prefill import paged_prefill_attention, prefill_att
 from mini_engine_hip.kernels.rope import qk_norm_rope_write_kv
 
 DEV = "cuda"
+PACKAGE_DIR = PACKAGE.parent
 
 
 class Subclass(torch.Tensor):
@@ -47,6 +52,46 @@ def test_declines_what_is_not_plain():
 def test_bind_refuses_a_wrong_library():
     with pytest.raises(ValueError):
         ext.native_calls().bind(len, (1, 2))
+
+
+REFUSED = """
+import torch
+from mini_engine_hip import HipLinear, build, linear_rows, paged_attention, paged_prefill_attention, prefill_attention
+from mini_engine_hip import qk_norm_rope_write_kv, write_kv_cache_slots
+from mini_engine_hip.kernels.paged import paged_attention_decode_write
+
+def no_build(**_):
+    raise SystemExit("a refused call went to the library")
+
+build.library_path = lambda: build.PACKAGE_DIR / "absent.so"
+build.build_library = no_build
+half, i64 = lambda *s: torch.zeros(*s).half(), lambda *s: torch.zeros(*s, dtype=torch.int64)
+cache, rows, row = half(2, 16, 2, 64), half(1, 4, 64), half(1, 2, 64)
+calls = [
+    (ValueError, lambda: HipLinear(64, 32)(torch.zeros(2, 64))),
+    (ValueError, lambda: linear_rows(half(2, 64), half(32, 64))),
+    (ValueError, lambda: prefill_attention(half(1, 4, 3, 64), half(1, 2, 3, 64), half(1, 2, 3, 64))),
+    (ValueError, lambda: paged_prefill_attention(rows, cache, cache, i64(2), i64(1), i64(1, 2), i64(1), 16, validate=False)),
+    (RuntimeError, lambda: paged_attention(rows, cache, cache, i64(1, 2), i64(1), 16, validate=False)),
+    (RuntimeError, lambda: paged_attention_decode_write(rows, cache, cache, i64(1, 2), i64(1), 16, row, row, validate=False)),
+    (ValueError, lambda: write_kv_cache_slots(cache, cache, i64(1), row, row, validate=False)),
+    (RuntimeError, lambda: qk_norm_rope_write_kv(rows, row, row, half(64), half(64), half(1, 32), half(1, 32), cache, cache,
+                                                 slot_mapping=i64(1), validate=False)),
+]
+for kind, call in calls:
+    try:
+        call()
+    except kind as error:
+        assert "library" not in str(error), error
+    else:
+        raise SystemExit("not refused")
+"""
+
+
+def test_refused_calls_need_no_library():
+    """What the entry points refuse is refused before any library is looked for."""
+    done = subprocess.run([sys.executable, "-c", REFUSED], cwd=PACKAGE_DIR, capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr[-2000:]
 
 
 @pytest.mark.gpu
