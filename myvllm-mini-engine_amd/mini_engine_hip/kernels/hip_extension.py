@@ -2,7 +2,8 @@
 
 Plays the role of the reference's ``load_cuda_extension``
 (mini_engine/kernels/cuda_extension.py:14-66): one cached handle per
-process.  There is no fallback: a missing or unloadable library raises.
+process.  There is no fallback: a missing or unloadable library raises.  (The
+native call path beside it is only a faster way into the same library.)
 """
 
 from __future__ import annotations
@@ -11,6 +12,7 @@ import ctypes
 import functools
 import importlib.machinery
 import importlib.util
+import warnings
 
 import torch
 
@@ -110,7 +112,7 @@ def check_build_digest(digest_file, expected: str) -> None:
 
 
 class NoNativeCalls:
-    """Stands for the native call path until the library is loaded: declines every call."""
+    """Stands for the native call path where it is not loaded: declines every call."""
 
     def _decline(self, *args):
         return None
@@ -166,7 +168,15 @@ def _host_module():
 
 
 def _bind_native(library):
-    module = _host_module()
+    """The native call path on ``library``, or what declines every call: the
+    Python code serves them all, so a host module that cannot be loaded costs
+    time, not calls."""
+    try:
+        module = _host_module()
+    except RuntimeError as error:
+        warnings.warn(f"{error}; calls take the Python path (rebuild with python -m mini_engine_hip.build)",
+                      RuntimeWarning, stacklevel=3)
+        return NoNativeCalls()
     module.bind(torch._C._cuda_getCurrentRawStream,
                 tuple(ctypes.cast(getattr(library._lib, name), _vp).value for name in _HOST_ENTRY_POINTS))
     return module

@@ -8,7 +8,7 @@ import sys
 import pytest
 import torch
 
-from mini_engine_hip.build import PACKAGE_DIR as PACKAGE
+from mini_engine_hip import build
 from mini_engine_hip.kernels import hip_extension as ext
 from mini_engine_hip.kernels.data import write_kv_cache_slots
 from mini_engine_hip.kernels.linear import linear_rows
@@ -17,7 +17,6 @@ from mini_engine_hip.kernels.prefill import paged_prefill_attention, prefill_att
 from mini_engine_hip.kernels.rope import qk_norm_rope_write_kv
 
 DEV = "cuda"
-PACKAGE_DIR = PACKAGE.parent
 
 
 class Subclass(torch.Tensor):
@@ -90,8 +89,34 @@ for kind, call in calls:
 
 def test_refused_calls_need_no_library():
     """What the entry points refuse is refused before any library is looked for."""
-    done = subprocess.run([sys.executable, "-c", REFUSED], cwd=PACKAGE_DIR, capture_output=True, text=True, timeout=300)
+    done = subprocess.run([sys.executable, "-c", REFUSED], cwd=build.PACKAGE_DIR.parent, capture_output=True, text=True, timeout=300)
     assert done.returncode == 0, done.stderr[-2000:]
+
+
+@pytest.fixture
+def fresh_loader(monkeypatch):
+    """The loader as in a new process; the process's own state comes back afterwards."""
+    monkeypatch.setattr(ext, "native", ext.NoNativeCalls())
+    caches = (ext.load_hip_extension, ext._host_module)
+    for cached in caches:
+        cached.cache_clear()
+    yield monkeypatch
+    for cached in caches:
+        cached.cache_clear()
+
+
+@pytest.mark.parametrize("content", [None, b"no shared object"])
+def test_python_path_serves_without_the_native_one(fresh_loader, tmp_path, content):
+    """A host module that is missing or cannot be loaded: a warning, and every
+    call is left to the Python code."""
+    planted = tmp_path / "mvme_host.so"
+    if content is not None:
+        planted.write_bytes(content)
+    fresh_loader.setattr(build, "host_path", lambda: planted)
+    with pytest.warns(RuntimeWarning, match="Python path"):
+        lib = ext.load_hip_extension()
+    assert lib.workspace_size(4, 16, 8, 128, 16, 64, 64) > 0
+    assert ext.native.decode(*decode_args("cpu"), 0) is None
 
 
 @pytest.mark.gpu
