@@ -63,16 +63,36 @@ def digest_path() -> Path:
     return LIB_DIR / "SOURCE_DIGEST"
 
 
+def host_digest_path() -> Path:
+    return LIB_DIR / "HOST_DIGEST"
+
+
 def sources() -> list[Path]:
     return sorted(SOURCE_DIR.glob("*.hip"))
 
 
 def source_digest() -> str:
     digest = hashlib.sha256()
-    for path in sorted([*SOURCE_DIR.glob("*.hip"), *SOURCE_DIR.glob("*.cpp"), *SOURCE_DIR.glob("*.h"),
-                        *INCLUDE_DIR.glob("*.h")]):
+    for path in sorted([*SOURCE_DIR.glob("*.hip"), *SOURCE_DIR.glob("*.h"), *INCLUDE_DIR.glob("*.h")]):
         digest.update(path.name.encode())
         digest.update(path.read_bytes())
+    return digest.hexdigest()
+
+
+def host_digest() -> str:
+    """What the native call path is built from: its source and the library's
+    header, and the torch and the Python whose headers it inlines (it reads
+    tensors through them, so another build of either needs another module)."""
+    import sysconfig
+
+    import torch
+
+    digest = hashlib.sha256()
+    for path in (SOURCE_DIR / "host_calls.cpp", INCLUDE_DIR / "mvme_paged.h"):
+        digest.update(path.read_bytes())
+    for part in (torch.__version__, torch.version.git_version, torch._C._GLIBCXX_USE_CXX11_ABI,
+                 sysconfig.get_config_var("EXT_SUFFIX")):
+        digest.update(f"|{part}".encode())
     return digest.hexdigest()
 
 
@@ -96,9 +116,9 @@ def _run(cmd: list[str]) -> None:
 def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
     """Compile every csrc/*.hip for gfx950 and link libmvme_paged.so; build mvme_host.so beside it.
 
-    Always recompiles (the build check must exercise the compiler).  The
-    source digest is written next to the library; the loader refuses a
-    library whose digest differs from the current sources.
+    Always recompiles (the build check must exercise the compiler).  A digest
+    is written next to each; the loader refuses a library whose digest differs
+    from the current sources, and leaves out such a call path.
     """
     hipcc = _hipcc()
     build_dir = PACKAGE_DIR / "_build"
@@ -123,6 +143,7 @@ def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
     os.replace(tmp, target)
     os.replace(host_tmp, host_path())
     digest_path().write_text(source_digest() + "\n")
+    host_digest_path().write_text(host_digest() + "\n")
     return target
 
 

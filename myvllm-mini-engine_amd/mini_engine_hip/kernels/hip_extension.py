@@ -157,6 +157,12 @@ _HOST_ENTRY_POINTS = ("mvme_last_error", "mvme_paged_attention_workspace_size", 
 @functools.lru_cache(maxsize=1)
 def _host_module():
     path = _build.host_path()
+    try:
+        recorded = _build.host_digest_path().read_text().strip()
+    except OSError as error:
+        raise RuntimeError(f"no build digest of the native call path: {error}") from error
+    if recorded != _build.host_digest():
+        raise RuntimeError("the native call path was built from other sources or for another torch or Python")
     loader = importlib.machinery.ExtensionFileLoader("mvme_host", str(path))
     spec = importlib.util.spec_from_file_location("mvme_host", str(path), loader=loader)
     try:

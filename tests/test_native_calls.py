@@ -119,6 +119,22 @@ def test_python_path_serves_without_the_native_one(fresh_loader, tmp_path, conte
     assert ext.native.decode(*decode_args("cpu"), 0) is None
 
 
+@pytest.mark.parametrize("name,value", [("__version__", "0.0"), ("version.git_version", "f" * 40)])
+def test_another_torch_needs_another_native_path(fresh_loader, name, value):
+    """The module inlines torch's headers: one built for another torch is not loaded."""
+    fresh_loader.setattr(f"torch.{name}", value)
+    with pytest.warns(RuntimeWarning, match="another torch"):
+        ext.load_hip_extension()
+    assert isinstance(ext.native, ext.NoNativeCalls)
+
+
+def test_native_path_without_a_digest_is_left_out(fresh_loader, tmp_path):
+    fresh_loader.setattr(build, "host_digest_path", lambda: tmp_path / "absent")
+    with pytest.warns(RuntimeWarning, match="no build digest"):
+        ext.load_hip_extension()
+    assert isinstance(ext.native, ext.NoNativeCalls)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("dim", [64, 80, 128])
