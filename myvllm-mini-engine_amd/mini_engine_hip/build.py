@@ -118,7 +118,8 @@ def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
 
     Always recompiles (the build check must exercise the compiler).  A digest
     is written next to each; the loader refuses a library whose digest differs
-    from the current sources, and leaves out such a call path.
+    from the current sources, and leaves out such a call path.  Where only the
+    call path cannot be compiled, the library is complete when this raises.
     """
     hipcc = _hipcc()
     build_dir = PACKAGE_DIR / "_build"
@@ -130,10 +131,9 @@ def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
         obj = build_dir / (src.stem + ".o")
         objects.append(obj)
         commands.append([hipcc, *HIP_FLAGS, f"-I{INCLUDE_DIR}", "-c", str(src), "-o", str(obj)])
-    host_tmp = host_path().with_suffix(".so.tmp")
-    commands.append(host_command(host_tmp))
-    workers = jobs or min(len(commands), max(1, min(8, os.cpu_count() or 1)))
+    workers = jobs or min(len(commands) + 1, max(1, min(8, os.cpu_count() or 1)))
     with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as pool:
+        host = pool.submit(_build_host)
         for cmd, _ in zip(commands, pool.map(_run, commands)):
             if verbose:
                 print(" ".join(cmd), flush=True)
@@ -141,10 +141,16 @@ def build_library(*, jobs: int | None = None, verbose: bool = False) -> Path:
     tmp = target.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objects)])
     os.replace(tmp, target)
-    os.replace(host_tmp, host_path())
     digest_path().write_text(source_digest() + "\n")
-    host_digest_path().write_text(host_digest() + "\n")
+    host.result()
     return target
+
+
+def _build_host() -> None:
+    tmp = host_path().with_suffix(".so.tmp")
+    _run(host_command(tmp))
+    os.replace(tmp, host_path())
+    host_digest_path().write_text(host_digest() + "\n")
 
 
 if __name__ == "__main__":

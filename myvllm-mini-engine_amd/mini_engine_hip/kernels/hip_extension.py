@@ -135,7 +135,11 @@ def load_hip_extension() -> HipLibrary:
     global native
     path = _build.library_path()
     if not path.exists():
-        _build.build_library()
+        try:
+            _build.build_library()
+        except RuntimeError:
+            if not path.exists():  # else only the native call path is missing
+                raise
     check_build_digest(_build.digest_path(), _build.source_digest())
     try:
         lib = ctypes.CDLL(str(path))

@@ -2,6 +2,7 @@
 takes gives the same bits as the same call with caller-supplied buffers (which
 it leaves to the Python code), and it declines everything else."""
 
+from pathlib import Path
 import subprocess
 import sys
 
@@ -133,6 +134,26 @@ def test_native_path_without_a_digest_is_left_out(fresh_loader, tmp_path):
     with pytest.warns(RuntimeWarning, match="no build digest"):
         ext.load_hip_extension()
     assert isinstance(ext.native, ext.NoNativeCalls)
+
+
+def test_library_is_built_where_the_native_path_cannot_be(fresh_loader, tmp_path):
+    """No host compiler or torch headers: the library needs neither."""
+    built = build.library_path()
+    fresh_loader.setattr(build, "LIB_DIR", tmp_path)
+    fresh_loader.setattr(build, "PACKAGE_DIR", tmp_path)
+
+    def run(cmd):
+        if "host_calls.cpp" in " ".join(cmd):
+            raise RuntimeError("no host compiler")
+        target = Path(cmd[cmd.index("-o") + 1])
+        target.write_bytes(built.read_bytes() if ".so" in target.name else b"")
+
+    fresh_loader.setattr(build, "_run", run)
+    with pytest.warns(RuntimeWarning, match="Python path"):
+        lib = ext.load_hip_extension()
+    assert lib.path == tmp_path / build.LIB_NAME
+    with pytest.raises(RuntimeError, match="no host compiler"):
+        build.build_library()
 
 
 @pytest.mark.gpu
