@@ -126,6 +126,8 @@ struct DecodeArgs {
     int64_t num_blocks;
     int block_size;
     int block_shift;  // log2(block_size) when it is a power of two, else -1
+    uint32_t block_magic;  // other sizes: t / block_size = (t * block_magic) >> (32 + block_rest)
+    int block_rest;
     int table_width;
     int capacity;   // table_width * block_size
     int partition;  // tokens per partition (multiple of the wave tile)
@@ -160,6 +162,16 @@ struct DecodeArgs {
     uint16_t* q_out;  // [batch, q_heads, D] rotated queries, or nullptr
     float eps;
 };
+
+// Page of token t in a table, and the token's row in that page.  Sizes that are
+// no power of two divide by a product (magic_divisor): a loop that looks up
+// every token's page has dozens of these, 20 instructions each as a division.
+__device__ inline int page_index(const DecodeArgs& a, int t) {
+    return a.block_shift >= 0 ? t >> a.block_shift : (int)(__umulhi((uint32_t)t, a.block_magic) >> a.block_rest);
+}
+__device__ inline int page_row(const DecodeArgs& a, int t) {
+    return a.block_shift >= 0 ? t & (a.block_size - 1) : t - page_index(a, t) * a.block_size;
+}
 
 // K/V rows are read once per call, by one work-group.  When a call's rows
 // can exceed the caches (more than 64 MiB of K/V within the tables'
@@ -360,7 +372,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             const int t = __builtin_amdgcn_readfirstlane(part * a.partition + wave * S::kTpi) + h * kRun;
             if (PAGE_UNIFORM && t < a.capacity)
                 first_page[h] = ((const const_i64*)(a.tables + (int64_t)seq * a.table_width))
-                    [a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size];
+                    [page_index(a, t)];
         }
     };
     int64_t fl_wc = 0, fl_pos = 0, fl_stop = 0, fl_row = 0, fl_row_later = 0;
@@ -517,7 +529,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         const uint32_t key_off = (uint32_t)(key_tok * row_bytes + (kvh * D + key_dim) * 2);
         auto page_of = [&](int t) __attribute__((always_inline)) -> int64_t {
             if (t >= end) return -1;
-            return ctable[a.block_shift >= 0 ? t >> a.block_shift : t / a.block_size];
+            return ctable[page_index(a, t)];
         };
         int it = __builtin_amdgcn_readfirstlane(start + wave * S::kTpi);
         int64_t page_next[H];
@@ -549,8 +561,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         int64_t next_krow[kLookup ? L : 1], next_vrow[kLookup ? L : 1];
         auto lookup = [&](int t0) __attribute__((always_inline)) {
             auto page_at = [&](int t) __attribute__((always_inline)) -> int64_t {
-                const int tc = min(t, end - 1);
-                return table[a.block_shift >= 0 ? tc >> a.block_shift : tc / a.block_size];
+                return table[page_index(a, min(t, end - 1))];
             };
 #pragma unroll
             for (int u = 0; u < L; ++u) {
@@ -559,8 +570,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             }
         };
         auto row_of = [&](int64_t page, int t) __attribute__((always_inline)) -> int64_t {
-            const int in_page = a.block_shift >= 0 ? t & (a.block_size - 1) : t % a.block_size;
-            return t < end && page >= 0 && page < a.num_blocks ? page * page_elems + (int64_t)in_page * row_elems
+            return t < end && page >= 0 && page < a.num_blocks ? page * page_elems + page_row(a, t) * row_elems
                                                                : (int64_t)-1;
         };
         // Where the rows of the iteration at t0 are, for fetch_k and fetch_v.
@@ -572,8 +582,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                     const int64_t page = page_next[h];
                     page_next[h] = page_of(t + kStep);
                     const bool page_ok = page >= 0 && page < a.num_blocks;
-                    const int in_page = a.block_shift >= 0 ? t & (a.block_size - 1) : t % a.block_size;
-                    next_base[h] = page_ok ? (page * a.block_size + in_page) * (int64_t)row_bytes : 0;
+                    next_base[h] = page_ok ? (page * a.block_size + page_row(a, t)) * (int64_t)row_bytes : 0;
                     next_lim[h] = page_ok ? end : 0;
                 }
             } else if constexpr (kLookup) {
@@ -635,10 +644,8 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         if constexpr (PRO) {
             int64_t slot = -1;
             if (owner) {
-                const int64_t page = a.tables[(int64_t)b * a.table_width +
-                                              (a.block_shift >= 0 ? pos >> a.block_shift : pos / a.block_size)];
-                if (page >= 0 && page < a.num_blocks)
-                    slot = page * a.block_size + (a.block_shift >= 0 ? pos & (a.block_size - 1) : pos % a.block_size);
+                const int64_t page = a.tables[(int64_t)b * a.table_width + page_index(a, pos)];
+                if (page >= 0 && page < a.num_blocks) slot = page * a.block_size + page_row(a, pos);
             }
             const int64_t cache_row = slot * a.kv_heads * D + (int64_t)kvh * D + 8 * c;
             const uint16_t* kv_src = a.new_k + (int64_t)b * a.k_stride + kvh * D + 8 * c;
@@ -855,14 +862,13 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 const int64_t page = page_next[0];
                 page_next[0] = page_of(it + kStep);
                 const bool page_ok = page >= 0 && page < a.num_blocks;
-                const int in_page = a.block_shift >= 0 ? it & (a.block_size - 1) : it % a.block_size;
 #pragma unroll
                 for (int u = 0; u < L; ++u) {
                     ok[u] = page_ok && it + u * S::kTpl + tl < end;
                     kk[u] = vv[u] = u32x4{0u, 0u, 0u, 0u};
                 }
                 if (page_ok) {  // wave-uniform
-                    const int64_t base = (page * a.block_size + in_page) * (int64_t)row_bytes;
+                    const int64_t base = (page * a.block_size + page_row(a, it)) * (int64_t)row_bytes;
                     const uint8_t* kp = static_cast<const uint8_t*>(a.key_cache) + base;
                     const uint8_t* vp = static_cast<const uint8_t*>(a.value_cache) + base;
 #pragma unroll
@@ -885,9 +891,9 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 for (int u = 0; u < L; ++u) {
                     const int t = it + u * S::kTpl + tl;
                     int64_t page = -1;
-                    if (t < end) page = table[t / a.block_size];
+                    if (t < end) page = table[page_index(a, t)];
                     ok[u] = page >= 0 && page < a.num_blocks;
-                    const int64_t off = page * page_elems + (int64_t)(t % a.block_size) * row_elems;
+                    const int64_t off = page * page_elems + page_row(a, t) * row_elems;
                     kk[u] = vv[u] = u32x4{0u, 0u, 0u, 0u};
                     if (ok[u] && chunk_ok) {
                         kk[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(kbase + off));

@@ -172,3 +172,32 @@ def test_runs_of_pages(block, dim, group):
         scores = torch.einsum("hgd,thd->hgt", query, keys) / dim ** 0.5
         want = torch.einsum("hgt,thd->hgd", scores.softmax(-1), values).reshape(2 * group, dim)
         assert (out[7] - want).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("dim", [16, 64])
+@pytest.mark.parametrize("block,length", [(3, 1048575), (5, 1048575), (1000, 1048000), (524287, 1048574), (174763, 174764)])
+def test_pages_of_no_power_of_two(block, length, dim):
+    """Page lookups up to the largest capacity, 2^20 tokens, by a product instead of
+    a division: every key's row holds the key's position, spread over the pages by a
+    permutation, and the query picks out single positions, the last one and those
+    around page ends among them."""
+    width = -(-length // block)
+    gen = torch.Generator(device=DEV).manual_seed(block)
+    table = torch.randperm(width, generator=gen, device=DEV)
+    spots = [t for t in {length - 1, length - length % block, block - 1, block, 2 * block - 1, length // 2, 0} if 0 <= t < length][:8]
+    key = torch.zeros(width, block, 1, dim, dtype=torch.float16, device=DEV)
+    value = torch.zeros_like(key)
+    q = torch.zeros(1, 4, dim, dtype=torch.float16, device=DEV)
+    q[0, :, 0] = 240.0
+    for heads in (spots[:4], spots[4:]):
+        key.zero_()
+        for h, t in enumerate(heads):
+            q[0, h] = 0
+            q[0, h, h] = 240.0
+            key[table[t // block], t % block, 0, h] = 240.0
+            value[table[t // block], t % block, 0] = 1.0 + h
+        lens = torch.tensor([length], device=DEV)
+        out = paged_attention(q, key, value, table[None], lens, block)
+        want = torch.tensor([1.0 + h for h in range(len(heads))], device=DEV).half()
+        assert torch.equal(out[0, :len(heads)], want[:, None].expand(-1, dim))
+        value.zero_()
