@@ -374,8 +374,27 @@ constexpr int64_t kDeviceCUs = 256;  // MI355X compute units
 // most 8 heads, of equal size (a tile reads all K/V rows of its kv head, so
 // one tile of 7 beats seven of 1, and 9 heads are 5 + 4); otherwise tiles that
 // divide the group.
-void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim) {
-    if ((head_dim == 64 || head_dim == 128) && group >= kMatrixGroup) {
+// Small calls take the latter too: a wide tile rotates, merges and stores all
+// of its heads in one work-group, 1 to 3 us that nothing overlaps, while the
+// many narrow ones' repeated reads come from L2.  The lines are in tokens that
+// all narrow tiles together may read, each at half a page below the tables'
+// capacity.  us per call, wide -> narrow, bf16: 9/1 heads, 3 x 38 step 8.1 ->
+// 5.0; 7/1, 1 x 2720 step 14.2 -> 11.7; 28/4, 8 x 496 8.0 -> 6.0; 12/1, 8 x 2400
+// (43 k tokens) 15.0 -> 14.1; 54/6 of 64, 8 x 256 (55 k) 7.2 -> 5.9; 5/1 of 64,
+// 40 x 304 (61 k) 7.1 -> 7.2; 6/1 of 64, 16 x 1344 (65 k) 8.5 -> 10.5; 6/1,
+// 96 x 128 (74 k) 7.3 -> 8.5.
+// Groups of 4, 8, ... in tiles of 4 on the matrix cores or of 2 on dot
+// products: 12/1, 39 x 24 step (5 k) 9.4 -> 6.6, 8/1, 18 x 168 step (12 k) 10.8
+// -> 7.6, both on odd pages; 12/1, 72 x 48 (17 k) 4.7 -> 4.9; 8/4, 4 x 512 (25 k)
+// 7.0 -> 7.9; 12/4, 12 x 144 (39 k) 7.6 -> 10.5.
+constexpr int64_t kNarrowTokens = 56 << 10;
+constexpr int64_t kPairTokens = 20 << 10;
+void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim, int64_t kv_units, int64_t cap, int64_t block_size) {
+    const bool matrix = head_dim == 64 || head_dim == 128;
+    const double tokens = (double)kv_units * (double)(cap - block_size / 2);
+    const bool fours = group % 4 == 0 && !(matrix && tokens * (double)(group / 2) <= (double)kPairTokens);
+    const int64_t narrow = fours ? 4 : group % 2 == 0 ? 2 : 1;
+    if (matrix && group >= kMatrixGroup && tokens * (double)(group / narrow) > (double)kNarrowTokens) {
         const int64_t tiles = (group + 7) / 8;
         const int64_t heads = (group + tiles - 1) / tiles;
         p.gtiles = (int)((group + heads - 1) / heads);
@@ -383,8 +402,8 @@ void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim) {
         p.gtile = heads <= 4 ? 4 : 8;
         return;
     }
-    p.gtile = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-    p.gtiles = (int)(group / p.gtile);
+    p.gtile = (int)narrow;
+    p.gtiles = (int)(group / narrow);
     p.tile_heads = p.gtile;
 }
 
@@ -472,9 +491,9 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
                             int64_t block_size, int64_t table_width, int64_t requested, bool walk = true) {
     DecodePlan p{};
     const int64_t group = q_heads / kv_heads;
-    plan_tiles(p, group, head_dim);
-    const int64_t tile = decode_tile_tokens(head_dim);
     const int64_t cap = table_width * block_size;
+    plan_tiles(p, group, head_dim, batch * kv_heads, cap, block_size);
+    const int64_t tile = decode_tile_tokens(head_dim);
     const int64_t units = batch * kv_heads * p.gtiles;
     const int64_t split_step = tile * kSplitWaves;
     const int64_t whole_step = tile * 16;  // the capacity unit the thresholds below were measured in

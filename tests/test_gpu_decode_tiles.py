@@ -40,6 +40,19 @@ def test_group_sizes_around_the_tiles(dtype, dim, group):
         check(args, dtype, partition)
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("group", [3, 5, 6, 8, 12, 17])
+@pytest.mark.parametrize("block,lengths", [(16, (33, 1, 18)), (24, (70, 24)), (256, (5,)), (16, (2500,))])
+def test_groups_of_small_calls(block, lengths, group, dim):
+    """Calls of few tokens split groups into tiles of 1, 2 or 4 heads: whole
+    sequences, split-K and the walk."""
+    dtype = torch.float16
+    args = decode_inputs(dtype, head_dim=dim, block_size=block, lengths=lengths, heads=group, kv_heads=1,
+                         seed=block + group)
+    for partition in (0, 64, -1):
+        check(args, dtype, partition)
+
+
 @pytest.mark.parametrize("block,lengths,partition", [
     (7, (50, 13, 1), 0), (24, (500, 24, 25), 128), (5, (333, 40), -1),     # per-token page lookups
     (16, (4097,), 0), (256, (2048, 1, 700), 0), (256, (5000, 4100), 0),    # plan's walk and split-K
