@@ -792,6 +792,7 @@ int launch_paged_attention(void* out, const void* query, const void* key_cache, 
     a.max_parts = p.max_parts;
     a.even_slots = p.even_slots;
     a.even_min = p.even_min;
+    a.even_few = (int)(kEvenFew / (kv_heads * p.gtiles));
     a.lpt_batch = p.flat_groups == 0 && p.even_slots == 0 && p.max_parts == 1 && batch >= 2 && batch <= kLptMax ? (int)batch : 0;
     // Two 8-wave work-groups per CU hold every unit at once (units in
     // (CUs, 2 CUs]): pair long sequences with short ones.  Longest first

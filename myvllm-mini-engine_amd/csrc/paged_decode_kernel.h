@@ -144,9 +144,10 @@ struct DecodeArgs {
     int batch;
     // Even parts (even_slots > 0, batch <= 64): split-K whose partition length
     // the lengths decide; even_slots work-groups per column, even_min tokens
-    // at least.
+    // at least, half of that for up to even_few tokens per column.
     int even_slots;
     int even_min;
+    int even_few;
     float scale_log2;
     // Fused prologue: 0 none; 1 write new_k / new_v rows at position len - 1;
     // 2 RMSNorm + RoPE of the query heads (query = raw rows, q_stride apart)
@@ -272,6 +273,11 @@ __device__ inline int64_t flat_share_start(int64_t l, int64_t total) { return (l
 // 16/8, 16 of U[1,1024] 12.6 against 13.8).
 template <int D, int G>
 constexpr bool even_tile() { return D == 128 && G == 8; }
+// Tokens over all columns up to which parts may be half as long: 128 parts of
+// 256 leave half of the CUs idle, and shorter ones end sooner than the longer
+// merge costs (7/1 heads, 5 of U[1,2240] 12.0 -> 10.7 us; 28/4, 3 of 5456 18.4
+// -> 17.0; beyond, 7/1, 14 of 3936 14.8 -> 16.0 and 32/4, 2 of 5680 15.2 -> 16.4).
+constexpr int kEvenFew = 128 * 256;
 constexpr int kEvenGroups = 512;  // work-groups: two of 4 waves per CU, what the 8-head tile's registers hold
 struct EvenParts {
     int len, count, incl, part;  // lane b: its sequence's tokens, partitions, inclusive prefix; uniform length
@@ -283,7 +289,8 @@ __device__ inline EvenParts even_parts(const DecodeArgs& a, int step) {
     // At most 64 sequences of 2^20 tokens: the sum fits 32 bits.
     const int total = lane_value(wave_incl_scan(e.len), kWave - 1);
     const int room = a.even_slots - a.batch;
-    const int want = max((total + room - 1) / room, a.even_min);
+    const int least = total <= a.even_few ? a.even_min / 2 : a.even_min;
+    const int want = max((total + room - 1) / room, least);
     e.part = (want + step - 1) / step * step;
     e.count = lane < a.batch ? max((e.len + e.part - 1) / e.part, 1) : 0;
     e.incl = wave_incl_scan(e.count);

@@ -133,6 +133,7 @@ def test_absent_pages_and_lengths_count_as_nothing():
 
 @pytest.mark.parametrize("lengths,kv_heads", [
     ((2048,), 1), ((3000,), 4), ((1, 2500, 64, 65, 129, 2), 4), (tuple([2300] * 20), 4),
+    ((2730,) * 12, 1), ((2730,) * 11 + (2739,), 1),  # 32760 and 32769 tokens: parts of 128 and of 256
     (tuple(1 + 37 * i for i in range(64)), 3), (tuple(2600 - 40 * i for i in range(59)), 4),
 ])
 @pytest.mark.parametrize("group", [7, 8, 12])
