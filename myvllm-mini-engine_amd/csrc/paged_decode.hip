@@ -552,21 +552,30 @@ DecodePlan make_decode_plan(int64_t batch, int64_t q_heads, int64_t kv_heads, in
         p.waves = kFlatWaves;
         p.max_parts = 1;
     }
-    // Pairs of heads: the matrix cores' loop, which keeps loads in flight,
-    // where two work-groups share a CU (16/8 heads of 128, pages of 16: 64
-    // sequences U[1,4096] 94.5 -> 91.5 us, 16 of U[1,1024] 13.2 -> 12.5, 8 of
-    // 512 8.9 -> 8.6; one 8-wave work-group per CU, the walk and more units
-    // than two per CU have no use for it: 32 of 2048 44.6 -> 45.8, walk of 32
-    // of U[1,4096] 51.7 -> 54.0, 96 of U[1,2600] 93.7 -> 95.9, 200 of
-    // U[1,1500] 107.9 -> 112.5.)
-    // At 64 dims pairs take the matrix cores where pages hold runs of 16 tokens
-    // but not the dot products' iterations of 32, which then look up every
-    // token's page (16/8 heads, pages of 16: 64 of 1000 39.7 -> 29.1, 48 of
-    // U[1,2000] 35.2 -> 29.3, 1 of 128 5.2 -> 4.4; pages of 256, 128 of 1024
-    // 52.7 -> 57.0, of 24, 16 of 700 12.6 -> 17.2).
-    const bool runs_only = block_size % 32 == 16;
-    const bool shared_cu = p.max_parts > 1 || (p.waves == kWholeWaves && units > kDeviceCUs && units <= 2 * kDeviceCUs);
-    if (group == 2 && !flat && ((head_dim == 128 && shared_cu) || (head_dim == 64 && runs_only))) {
+    // Pairs of heads on the matrix cores, whose loop keeps loads in flight but
+    // starts and ends more slowly (dot products / matrix cores, us per call,
+    // 16/8 heads unless noted).
+    // At 128 dims, on pages that hold whole iterations (2/1 heads, 3 x 2928 on
+    // pages of 8 10.5 / 12.8; 8/4, 39 x 840 on pages of 24 21.1 / 24.2):
+    // * splits of up to 160 units: 8 of 512 step 10.0 / 9.7, 16 of U[1,1024]
+    //   13.2 / 12.5; 26 of 720 18.6 / 21.0, 26 of 1088 24.0 / 25.5, 23 of 2816 step
+    //   44.8 / 47.1;
+    // * two long units on most CUs: 64 of U[1,4096] 95.0 / 92.5, 420 units of
+    //   U[1,1792] 41.0 / 38.8; 400 of U[1,928] 23.4 / 25.9, 344 of U[1,2304] 62.0 /
+    //   64.8, 376 of 1536 step 53.8 / 56.6, one per CU (32 of 2048) 44.6 / 45.8.
+    // At 64 dims where pages hold runs of 16 tokens but not the dot products'
+    // iterations of 32, which then look up every token's page: 64 of 1000 39.7 /
+    // 29.1, 48 of U[1,2000] 35.2 / 29.3 (pages of 256, 128 of 1024 52.7 / 57.0, of
+    // 24, 16 of 700 12.6 / 17.2); but not for many short units: 800 of 96 step 10.6
+    // / 11.3, 1376 of 192 18.0 / 21.5, 3312 of 480 step 52.9 / 58.0 (768 of 464 step
+    // 24.5 / 22.3, 1552 of 864 step 86.1 / 72.0).
+    const bool matrix_pairs =
+        head_dim == 128 ? block_size % tile == 0 &&
+                              (p.max_parts > 1 ? units <= kDeviceCUs * 5 / 8
+                                               : p.waves == kWholeWaves && units >= kDeviceCUs * 3 / 2 &&
+                                                     units <= 2 * kDeviceCUs && cap >= 1536)
+                        : head_dim == 64 && block_size % 32 == 16 && 2 * units <= 5 * cap;
+    if (group == 2 && !flat && matrix_pairs) {
         p.gtile = 4;
         p.tile_heads = 2;
     }
