@@ -1046,8 +1046,9 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
         // 16-bit patterns of non-negative values they order above 256, so an
         // unsigned maximum of the packed halves decides), otherwise when the
         // fp32 sum of 8 does, which the row sums need anyway.  `first`:
-        // the item's first tile, where nothing is accumulated yet (every
-        // rescale factor is 1, so the rescale is skipped).
+        // the item's first tile, where every row needs the exact step and
+        // nothing is accumulated yet (every rescale factor is 1, so the
+        // rescale is skipped).
         auto softmax_tile = [&](int tile, int st, bool first) __attribute__((always_inline)) {
             const int tile0 = tile * SH::kKeys;
             const bool full = ((full_stages >> st) & 1u) != 0;
@@ -1074,37 +1075,41 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
             auto sum8 = [](const float (&p)[8]) __attribute__((always_inline)) -> float {
                 return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
             };
-#pragma unroll
-            for (int nb = 0; nb < SH::kNb; ++nb) {
-                need = need | ((m_run[nb] == kNegInf) & (pos[nb] >= tile0));
-                dl[nb] = 0.f;
-            }
-#pragma unroll
-            for (int h = 0; h < SH::kHalves; ++h)
+            if (first) {
+                need = true;
+            } else {
 #pragma unroll
                 for (int nb = 0; nb < SH::kNb; ++nb) {
-                    float p[8];
-#pragma unroll
-                    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            p[4 * kk + j] = fast_exp2(PRESCALE ? sc[h][nb][kk][j]
-                                                               : fmaf(sc[h][nb][kk][j], a.scale_log2, nref[nb]));
-                    pops[h][nb] = u32x4{T::pack(p[0], p[1]), T::pack(p[2], p[3]), T::pack(p[4], p[5]), T::pack(p[6], p[7])};
-                    if constexpr (!PRESCALE) {
-                        const float d = sum8(p);
-                        need = need | !(d <= kPSumLimit);
-                        dl[nb] += d;
-                    } else {
-                        typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-                        us2 m = __builtin_elementwise_max(__builtin_bit_cast(us2, pops[h][nb][0]),
-                                                          __builtin_bit_cast(us2, pops[h][nb][1]));
-                        m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, pops[h][nb][2]));
-                        m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, pops[h][nb][3]));
-                        const uint32_t lim = T::pack(kPSumLimit, 0.f) & 0xffffu;
-                        need = need | ((uint32_t)max(m.x, m.y) > lim);
-                    }
+                    need = need | ((m_run[nb] == kNegInf) & (pos[nb] >= tile0));
+                    dl[nb] = 0.f;
                 }
+#pragma unroll
+                for (int h = 0; h < SH::kHalves; ++h)
+#pragma unroll
+                    for (int nb = 0; nb < SH::kNb; ++nb) {
+                        float p[8];
+#pragma unroll
+                        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                p[4 * kk + j] = fast_exp2(PRESCALE ? sc[h][nb][kk][j]
+                                                                   : fmaf(sc[h][nb][kk][j], a.scale_log2, nref[nb]));
+                        pops[h][nb] = u32x4{T::pack(p[0], p[1]), T::pack(p[2], p[3]), T::pack(p[4], p[5]), T::pack(p[6], p[7])};
+                        if constexpr (!PRESCALE) {
+                            const float d = sum8(p);
+                            need = need | !(d <= kPSumLimit);
+                            dl[nb] += d;
+                        } else {
+                            typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+                            us2 m = __builtin_elementwise_max(__builtin_bit_cast(us2, pops[h][nb][0]),
+                                                              __builtin_bit_cast(us2, pops[h][nb][1]));
+                            m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, pops[h][nb][2]));
+                            m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, pops[h][nb][3]));
+                            const uint32_t lim = T::pack(kPSumLimit, 0.f) & 0xffffu;
+                            need = need | ((uint32_t)max(m.x, m.y) > lim);
+                        }
+                    }
+            }
             if (__builtin_amdgcn_ballot_w64(need)) {
 #pragma unroll
                 for (int nb = 0; nb < SH::kNb; ++nb) {
