@@ -108,6 +108,11 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // context): loading zeros keeps every LDS slot finite without predication.
 __device__ __attribute__((aligned(16))) const uint32_t kZeroChunk[4] = {0u, 0u, 0u, 0u};
 
+// Order in which a call without a key split hands out its query blocks.
+constexpr int kInTurn = 0;         // sequence by sequence
+constexpr int kLongestFirst = 1;   // see find_item_longest
+constexpr int kLongestIfAlike = 2; // longest first when all sequences are alike, else in turn
+
 struct PrefillArgs {
     void* out;
     const void* q;
@@ -130,6 +135,7 @@ struct PrefillArgs {
     int qb;        // query tokens per item (rows of the tile shape / group, rounded down)
     int chunk;     // keys per item (multiple of the tile's keys)
     int max_chunks;
+    int order;  // query blocks without a key split: kInTurn, kLongestFirst or kLongestIfAlike
     int chunk_choice;  // 1: a walk with more than one round of items may take a larger chunk
     int head_dim;
     int part_dim;  // elements per partial row: the tile shape's PfShape::kPart
@@ -334,11 +340,19 @@ __device__ inline int blocks_above(const PrefillArgs& a, const SeqMeta& m, int b
 // 265.1.  Buckets, not single lengths, so that the blocks of one sequence
 // stay together and share its K/V in L2.  Lane s holds sequence s; the bucket
 // is found by bisection on the number of blocks above a key count.
+// Not where all work-groups run at once (the lookup is 0.2 us of a call of 10),
+// and over tables of two buckets only for sequences that are alike, whose
+// blocks of one length in turn would meet on the same XCDs: 41 x 277 tokens at
+// 256 dims, 14/2 heads, 115 -> 95 us in this order, but 17 of up to 416, 32/8
+// heads, 79 -> 84, and 33 of up to 307 at 128 dims, 56/8, 83 -> 86.
 constexpr int kOrderKeys = 256;
 template <bool DENSE>
 __device__ inline bool find_item_longest(const PrefillArgs& a, int item, PrefillItem& it) {
     const int lane = __lane_id();
     const SeqMeta m = load_meta<DENSE>(a, lane);
+    if (a.order == kLongestIfAlike &&
+        __ballot(lane < a.num_seqs && (m.n != lane_value(m.n, 0) || m.start != lane_value(m.start, 0))) != 0)
+        return find_item<DENSE>(a, a.chunk, item, it, nullptr, &m);
     const int blocks = query_blocks(a, m.n);
     auto count_above = [&](int64_t t) __attribute__((always_inline)) -> int {
         return lane_value(wave_incl_scan(blocks_above(a, m, blocks, t)), kWave - 1);
@@ -1721,8 +1735,8 @@ __global__ __launch_bounds__(kPfThreads, 1) void paged_prefill_mfma_kernel(Prefi
     if constexpr (!WALK) {
         PrefillItem item;
         const int index = blockIdx.x / a.kv_heads;
-        const bool found = a.max_chunks == 1 && a.num_seqs <= kWave ? find_item_longest<DENSE>(a, index, item)
-                                                                    : find_item<DENSE>(a, a.chunk, index, item);
+        const bool found = a.order != kInTurn ? find_item_longest<DENSE>(a, index, item)
+                                              : find_item<DENSE>(a, a.chunk, index, item);
         if (!found) return;
         prefill_item<T, PAGES, NARROW, HD, DENSE>(a, item, lds);
     } else {
@@ -2159,6 +2173,9 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
         }
         const int64_t groups = item_slots * kv_heads;
         if (groups > 2147483647) return fail(MVME_EINVAL, "paged prefill grid too large");
+        a.order = p.max_chunks > 1 || a.num_seqs > kWave || groups <= kPrefillCUs ? kInTurn
+                  : table_width * a.block_size <= 2 * kOrderKeys                  ? kLongestIfAlike
+                                                                                  : kLongestFirst;
         // Whole-tile pages: a tile lies in one page (power-of-two blocks of at
         // least a tile's keys) and per-lane offsets inside a tile fit 32 bits.
         const bool tile_pages = a.block_shift >= 0 && a.block_size >= p.keys &&

@@ -7,7 +7,8 @@ import math
 import pytest
 import torch
 
-from mini_engine_hip.kernels.prefill import paged_prefill_attention, prefill_attention
+from mini_engine_hip.kernels.prefill import (paged_prefill_attention, paged_prefill_workspace_bytes,
+                                              prefill_attention)
 from oracle import paged_oracle
 
 pytestmark = pytest.mark.gpu
@@ -78,6 +79,26 @@ def test_query_blocks_of_many_sequences(seqs, heads, kv_heads):
     prior[5] = 0
     args = paged_case(new, prior, block, heads, kv_heads, dtype, seed=seqs)
     dev = [a.to(DEV) for a in args]
+    torch.full_like(dev[0], float("nan"))  # freed at once: the output's storage
+    actual = paged_prefill_attention(*dev, block, validate=False).float().cpu()
+    expected = paged_oracle.paged_prefill_attention(*args, block, cast=False)
+    assert (actual - expected).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("lengths", ["alike", "ragged"])
+def test_query_blocks_over_short_tables(lengths, dim):
+    """Tables of at most 512 tokens: longest blocks first where the sequences are
+    alike, in turn otherwise, an empty one among them."""
+    dtype, block, seqs = torch.bfloat16, 16, 40
+    gen = torch.Generator().manual_seed(dim)
+    new = [290] * seqs if lengths == "alike" else torch.randint(60, 450, (seqs,), generator=gen).tolist()
+    prior = [0] * seqs if lengths == "alike" else torch.randint(0, 60, (seqs,), generator=gen).tolist()
+    if lengths == "ragged":
+        new[7] = 0
+    args = paged_case(new, prior, block, 8, 4, dtype, seed=seqs, dim=dim)
+    dev = [a.to(DEV) for a in args]
+    assert paged_prefill_workspace_bytes(seqs, sum(new), 8, 4, dim, block, args[5].shape[1], dtype) == 0
     torch.full_like(dev[0], float("nan"))  # freed at once: the output's storage
     actual = paged_prefill_attention(*dev, block, validate=False).float().cpu()
     expected = paged_oracle.paged_prefill_attention(*args, block, cast=False)
