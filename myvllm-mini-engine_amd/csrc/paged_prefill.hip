@@ -2188,7 +2188,12 @@ int launch_prefill(PrefillArgs a, const PrefillPlan& p, int64_t total_tokens, in
         const bool wave_pages = a.block_shift >= 3 && p.hd <= 128 && !p.narrow &&
                                 a.kv_row_bytes * p.keys < (int64_t(1) << 31);
         if (p.hd == 64 && !wave_pages) return fail(MVME_EINVAL, "prefill key/value token stride too large");
-        int pages = tile_pages ? kPagesPerTile : wave_pages ? kPagesPerWave : (block_size % 4 == 0 ? kPagesPerRows : kPagesPerLane);
+        // Over a tile or two the loop that is not pipelined starts sooner (us per
+        // call, pipelined / not, 8/4 heads of 128): 4 x 64 tokens on pages of 8 9.5 /
+        // 8.6, of 16 9.0 / 8.6, 4 x 192 on pages of 8 12.8 / 12.6; 4 x 128 on pages
+        // of 16 11.9 / 12.2, 4 x 256 on pages of 8 15.3 / 16.4.
+        const bool few_keys = p.hd == 128 && table_width * block_size < (block_size == 8 ? 256 : 128);
+        int pages = tile_pages ? kPagesPerTile : wave_pages && !few_keys ? kPagesPerWave : (block_size % 4 == 0 ? kPagesPerRows : kPagesPerLane);
         if (p.narrow && pages == kPagesPerRows) pages = kPagesPerLane;  // no narrow instantiation of that mode
         const dim3 grid((unsigned)groups), block(kPfThreads);
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
