@@ -27,6 +27,7 @@
 // x loads removed; with 8 features per work-group, as the staged kernel
 // has, it took 7.7 us).
 #include <mutex>
+#include <type_traits>
 
 #include "mvme_common.h"
 
@@ -172,42 +173,42 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_quads_kernel(LinearAr
     f32x4 acc[MB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int kInFlight = MB <= 2 ? 2 : 1;
-    for (int s0 = wave; s0 < slices; s0 += kLinWaves * kInFlight) {
-        u32x4 wv[kInFlight][4], xv[kInFlight][MB][4];
+    // F slices from s on, 16 apart, all loaded before the first product.
+    auto run = [&](auto count, int s) __attribute__((always_inline)) {
+        constexpr int F = decltype(count)::value;
+        u32x4 wv[F][4], xv[F][MB][4];
 #pragma unroll
-        for (int f = 0; f < kInFlight; ++f) {
-            const int s = min(s0 + f * kLinWaves, slices - 1);  // past the end: re-read the last, unused
+        for (int f = 0; f < F; ++f) {
+            const int k = 128 * (s + f * kLinWaves);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                wv[f][j] = *reinterpret_cast<const u32x4*>(wrow + (int64_t)j * a.in_features + 128 * s);
+                wv[f][j] = *reinterpret_cast<const u32x4*>(wrow + (int64_t)j * a.in_features + k);
             // Rows of x past M read row 0 (in bounds); their products are dropped.
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int r = 16 * mb + quad + j;
-                    xv[f][mb][j] = *reinterpret_cast<const u32x4*>(xbase + (int64_t)(r < a.rows ? r : 0) * a.x_stride + 128 * s);
+                    xv[f][mb][j] = *reinterpret_cast<const u32x4*>(xbase + (int64_t)(r < a.rows ? r : 0) * a.x_stride + k);
                 }
         }
 #pragma unroll
-        for (int f = 0; f < kInFlight; ++f) {
-            const bool live = s0 + f * kLinWaves < slices;
+        for (int f = 0; f < F; ++f) {
             quad_transpose(wv[f]);
-            if (!live)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) wv[f][j] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) {
                 quad_transpose(xv[f][mb]);
-                if (!live)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) xv[f][mb][j] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[mb] = T::mfma16x16x32(wv[f][j], xv[f][mb][j], acc[mb]);
             }
         }
-    }
+    };
+    // (Loading a slice that is not there, to keep one loop, cost depths up to
+    // 2048 twice the loads.)
+    constexpr int kInFlight = MB <= 2 ? 2 : 1;
+    int s = wave;
+    for (; s + (kInFlight - 1) * kLinWaves < slices; s += kInFlight * kLinWaves) run(std::integral_constant<int, kInFlight>{}, s);
+    if (s < slices) run(std::integral_constant<int, 1>{}, s);
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) sm_part[wave][mb][lane] = acc[mb];
     __syncthreads();
