@@ -467,7 +467,13 @@ template <typename T>
 void launch_linear_rows(const LinearArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)(a.out_features / 16)), block(kLinThreads);
     const int mb = (a.rows + 15) / 16;
-    if (a.in_features % 128 == 0) {
+    // One to three rows into wide layers keep operand-order loads, whose x is then one
+    // to three lines and whose 16 waves all work at any depth.  us per call, operand
+    // order / quads: 1 row, K = 4096, N = 8192 14.6 / 16.0, K = 1920, N = 16384 14.2 /
+    // 15.9; 3 rows 15.3 / 16.1, 14.8 / 16.0; 6 rows 16.7 / 16.1; 1 row, K = 4096, N =
+    // 6144 14.4 / 14.5, K = 1408, N = 16384 14.1 / 14.0, K = 5120, N = 8192 19.0 / 17.5.
+    const bool few_rows = a.rows <= 3 && a.out_features >= 8192 && a.in_features > 1536 && a.in_features <= 4096;
+    if (a.in_features % 128 == 0 && !few_rows) {
         if (mb == 1) hipLaunchKernelGGL((linear_rows_quads_kernel<T, 1>), grid, block, 0, s, a);
         else if (mb == 2) hipLaunchKernelGGL((linear_rows_quads_kernel<T, 2>), grid, block, 0, s, a);
         else if (mb == 3) hipLaunchKernelGGL((linear_rows_quads_kernel<T, 3>), grid, block, 0, s, a);

@@ -55,10 +55,12 @@ def test_linear_rows_wide_layers(dtype, rows, k, n, bias):
     (1, 128, 16, False), (16, 640, 48, True), (32, 896, 2048, False), (33, 3584, 80, False),
     (64, 4096, 2048, True), (48, 384, 32, False), (17, 2176, 64, False),
     (16, 4224, 48, False), (32, 6272, 32, True), (5, 8320, 16, False),
+    (3, 1920, 8192, False), (4, 1920, 8192, False), (1, 4096, 8208, True),
 ])
 def test_linear_rows_quad_slices(dtype, rows, k, n, bias):
     """K a multiple of 128 outside the staged and the streaming kernel: fewer
-    slices than waves, one round of them, a remainder of a second and third."""
+    slices than waves, one round of them, a remainder of a second and third;
+    one to three rows into wide layers, which load in operand order."""
     test_linear_rows_matches_fp32_product(dtype, rows, k, n, bias)
 
 
