@@ -386,7 +386,8 @@ constexpr int64_t kDeviceCUs = 256;  // MI355X compute units
 // Groups of 4, 8, ... in tiles of 4 on the matrix cores or of 2 on dot
 // products: 12/1, 39 x 24 step (5 k) 9.4 -> 6.6, 8/1, 18 x 168 step (12 k) 10.8
 // -> 7.6, both on odd pages; 12/1, 72 x 48 (17 k) 4.7 -> 4.9; 8/4, 4 x 512 (25 k)
-// 7.0 -> 7.9; 12/4, 12 x 144 (39 k) 7.6 -> 10.5.
+// 7.0 -> 7.9; 12/4, 12 x 144 (39 k) 7.6 -> 10.5.  Tiles of 4 that outnumber the
+// CUs lose to one wide tile per CU: 64/4, 18 x 141 8.9 against 7.6.
 constexpr int64_t kNarrowTokens = 56 << 10;
 constexpr int64_t kPairTokens = 20 << 10;
 void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim, int64_t kv_units, int64_t cap, int64_t block_size) {
@@ -394,7 +395,9 @@ void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim, int64_t kv_units
     const double tokens = (double)kv_units * (double)(cap - block_size / 2);
     const bool fours = group % 4 == 0 && !(matrix && tokens * (double)(group / 2) <= (double)kPairTokens);
     const int64_t narrow = fours ? 4 : group % 2 == 0 ? 2 : 1;
-    if (matrix && group >= kMatrixGroup && tokens * (double)(group / narrow) > (double)kNarrowTokens) {
+    const bool small = tokens * (double)(group / narrow) <= (double)kNarrowTokens &&
+                       (!fours || kv_units * (group / narrow) <= kDeviceCUs);
+    if (matrix && group >= kMatrixGroup && !small) {
         const int64_t tiles = (group + 7) / 8;
         const int64_t heads = (group + tiles - 1) / tiles;
         p.gtiles = (int)((group + heads - 1) / heads);
