@@ -748,12 +748,16 @@ struct DecodePrologue {
     float eps;
 };
 
-// Division of t < 2^31 by a block size b that is no power of two as a product:
-// with s = floor(log2 b) and m = ceil(2^(32+s) / b) < 2^32, t * m / 2^(32+s)
-// exceeds t / b by t * e / (b * 2^(32+s)) with e = m * b - 2^(32+s) < b < 2^(s+1),
-// less than 1 / b, so the integer part is the quotient.
+// Division of t < 2^31 by a block size b as a product: with s = floor(log2(b - 1))
+// and m = ceil(2^(32+s) / b) < 2^32, t * m / 2^(32+s) exceeds t / b by t * e / (b *
+// 2^(32+s)) with e = m * b - 2^(32+s) < b <= 2^(s+1), less than 1 / b, so the
+// integer part is the quotient.  (b = 1, whose factor would be 2^32, adds t itself.)
 void magic_divisor(DecodeArgs& a, int64_t block_size) {
-    a.block_rest = 63 - __builtin_clzll((unsigned long long)block_size);
+    if (block_size == 1) {
+        a.block_one = ~0u;
+        return;
+    }
+    a.block_rest = 63 - __builtin_clzll((unsigned long long)(block_size - 1));
     a.block_magic = (uint32_t)(((1ull << (32 + a.block_rest)) + block_size - 1) / block_size);
 }
 
@@ -797,7 +801,7 @@ int launch_paged_attention(void* out, const void* query, const void* key_cache, 
     a.num_blocks = num_blocks;
     a.block_size = (int)block_size;
     a.block_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctzll((unsigned long long)block_size) : -1;
-    if (a.block_shift < 0) magic_divisor(a, block_size);
+    magic_divisor(a, block_size);
     a.table_width = (int)table_width;
     a.capacity = (int)(table_width * block_size);
     a.partition = p.partition;

@@ -126,7 +126,8 @@ struct DecodeArgs {
     int64_t num_blocks;
     int block_size;
     int block_shift;  // log2(block_size) when it is a power of two, else -1
-    uint32_t block_magic;  // other sizes: t / block_size = (t * block_magic) >> (32 + block_rest)
+    // t / block_size = ((t * block_magic >> 32) + (t & block_one)) >> block_rest
+    uint32_t block_magic, block_one;
     int block_rest;
     int table_width;
     int capacity;   // table_width * block_size
@@ -164,15 +165,22 @@ struct DecodeArgs {
     float eps;
 };
 
-// Page of token t in a table, and the token's row in that page.  Sizes that are
-// no power of two divide by a product (magic_divisor): a loop that looks up
-// every token's page has dozens of these, 20 instructions each as a division.
+// Page of token t in a table, and the token's row in that page, for a token of
+// the whole wave.
 __device__ inline int page_index(const DecodeArgs& a, int t) {
     return a.block_shift >= 0 ? t >> a.block_shift : (int)(__umulhi((uint32_t)t, a.block_magic) >> a.block_rest);
 }
 __device__ inline int page_row(const DecodeArgs& a, int t) {
     return a.block_shift >= 0 ? t & (a.block_size - 1) : t - page_index(a, t) * a.block_size;
 }
+// The same for a token per lane: a product (magic_divisor) instead of a division of
+// 20 instructions, of which a loop that looks up every token's page has dozens,
+// and no branch on the size, which would keep the lookups apart (32 dims on
+// pages of 32, 31 sequences of 6347: 70 us with divisions, 76 with the branch).
+__device__ inline int lane_page(const DecodeArgs& a, int t) {
+    return (int)((__umulhi((uint32_t)t, a.block_magic) + ((uint32_t)t & a.block_one)) >> a.block_rest);
+}
+__device__ inline int lane_row(const DecodeArgs& a, int t, int page_of_t) { return t - page_of_t * a.block_size; }
 
 // K/V rows are read once per call, by one work-group.  When a call's rows
 // can exceed the caches (more than 64 MiB of K/V within the tables'
@@ -568,7 +576,7 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
         int64_t next_krow[kLookup ? L : 1], next_vrow[kLookup ? L : 1];
         auto lookup = [&](int t0) __attribute__((always_inline)) {
             auto page_at = [&](int t) __attribute__((always_inline)) -> int64_t {
-                return table[page_index(a, min(t, end - 1))];
+                return table[lane_page(a, min(t, end - 1))];
             };
 #pragma unroll
             for (int u = 0; u < L; ++u) {
@@ -577,8 +585,9 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             }
         };
         auto row_of = [&](int64_t page, int t) __attribute__((always_inline)) -> int64_t {
-            return t < end && page >= 0 && page < a.num_blocks ? page * page_elems + page_row(a, t) * row_elems
-                                                               : (int64_t)-1;
+            return t < end && page >= 0 && page < a.num_blocks
+                       ? page * page_elems + lane_row(a, t, lane_page(a, t)) * row_elems
+                       : (int64_t)-1;
         };
         // Where the rows of the iteration at t0 are, for fetch_k and fetch_v.
         auto fetch_page = [&](int t0) __attribute__((always_inline)) {
@@ -898,9 +907,10 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 for (int u = 0; u < L; ++u) {
                     const int t = it + u * S::kTpl + tl;
                     int64_t page = -1;
-                    if (t < end) page = table[page_index(a, t)];
+                    const int idx = lane_page(a, t);
+                    if (t < end) page = table[idx];
                     ok[u] = page >= 0 && page < a.num_blocks;
-                    const int64_t off = page * page_elems + page_row(a, t) * row_elems;
+                    const int64_t off = page * page_elems + lane_row(a, t, idx) * row_elems;
                     kk[u] = vv[u] = u32x4{0u, 0u, 0u, 0u};
                     if (ok[u] && chunk_ok) {
                         kk[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(kbase + off));
