@@ -370,6 +370,9 @@ int decode_tile_tokens(int64_t head_dim) {
 
 constexpr int64_t kDeviceCUs = 256;  // MI355X compute units
 
+// Smallest tables, in tokens, over which 8-head tiles take even parts.
+constexpr int64_t kEvenCapacity = 2048;
+
 // Query-head tiles of a group: on the matrix cores the fewest tiles of at
 // most 8 heads, of equal size (a tile reads all K/V rows of its kv head, so
 // one tile of 7 beats seven of 1, and 9 heads are 5 + 4); otherwise tiles that
@@ -378,25 +381,28 @@ constexpr int64_t kDeviceCUs = 256;  // MI355X compute units
 // of its heads in one work-group, 1 to 3 us that nothing overlaps, while the
 // many narrow ones' repeated reads come from L2.  The lines are in tokens that
 // all narrow tiles together may read, each at half a page below the tables'
-// capacity.  us per call, wide -> narrow, bf16: 9/1 heads, 3 x 38 step 8.1 ->
-// 5.0; 7/1, 1 x 2720 step 14.2 -> 11.7; 28/4, 8 x 496 8.0 -> 6.0; 12/1, 8 x 2400
-// (43 k tokens) 15.0 -> 14.1; 54/6 of 64, 8 x 256 (55 k) 7.2 -> 5.9; 5/1 of 64,
-// 40 x 304 (61 k) 7.1 -> 7.2; 6/1 of 64, 16 x 1344 (65 k) 8.5 -> 10.5; 6/1,
-// 96 x 128 (74 k) 7.3 -> 8.5.
-// Groups of 4, 8, ... in tiles of 4 on the matrix cores or of 2 on dot
-// products: 12/1, 39 x 24 step (5 k) 9.4 -> 6.6, 8/1, 18 x 168 step (12 k) 10.8
-// -> 7.6, both on odd pages; 12/1, 72 x 48 (17 k) 4.7 -> 4.9; 8/4, 4 x 512 (25 k)
-// 7.0 -> 7.9; 12/4, 12 x 144 (39 k) 7.6 -> 10.5.  Tiles of 4 that outnumber the
-// CUs lose to one wide tile per CU: 64/4, 18 x 141 8.9 against 7.6.
-constexpr int64_t kNarrowTokens = 56 << 10;
-constexpr int64_t kPairTokens = 20 << 10;
+// capacity.  us per call, wide / narrow, bf16:
+// * tiles of 1 or 2 heads: 9/1 heads, 3 x 38 step 8.1 / 5.0; 28/4, 8 x 496 8.0 /
+//   6.0; 7/1, 1 x 3440 (24 k tokens; 2 of them 48 k) 12.0 / 11.5 (12.7 / 13.2); 5/1,
+//   16 x 608 (48 k) 8.2 / 9.7; 5/1 of 64, 40 x 304 (61 k) 7.1 / 7.2; 6/1, 96 x 128
+//   (74 k) 7.3 / 8.5;
+// * three heads, which one tile of 4 holds: 8 x 32 step 5.9 / 4.9; 16 x 576 (26 k)
+//   8.2 / 8.5; 19 x 832 (47 k) 8.5 / 10.8; 6 x 3072 (53 k) 8.3 / 11.2;
+// * tiles of 4: 12/4, 24 x 144 step 9.9 / 7.6; 8/1, 2 x 1536 11.9 / 11.2; 48/8, 4 x
+//   592 9.9 / 9.2; over tables that take even parts 8/1, 2 x 4096 (16 k) 12.3 / 15.0,
+//   12/1, 3 x 4624 (42 k) 12.2 / 15.4; and more of them than CUs, 64/4, 18 x 141
+//   7.6 / 8.9;
+// * groups of 4, 8, ... in tiles of 2 (tiles of 4 / of 2): 12/1, 39 x 24 step (5 k)
+//   9.4 / 6.6, 8/1, 18 x 168 step (12 k) 10.8 / 7.6, both on odd pages; 12/1, 72 x 48
+//   (17 k) 4.7 / 4.9; 8/4, 4 x 512 (25 k) 7.0 / 7.9.
+constexpr int64_t kNarrowTokens = 48 << 10, kNarrowThree = 28 << 10, kPairTokens = 20 << 10;
 void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim, int64_t kv_units, int64_t cap, int64_t block_size) {
     const bool matrix = head_dim == 64 || head_dim == 128;
     const double tokens = (double)kv_units * (double)(cap - block_size / 2);
     const bool fours = group % 4 == 0 && !(matrix && tokens * (double)(group / 2) <= (double)kPairTokens);
     const int64_t narrow = fours ? 4 : group % 2 == 0 ? 2 : 1;
-    const bool small = tokens * (double)(group / narrow) <= (double)kNarrowTokens &&
-                       (!fours || kv_units * (group / narrow) <= kDeviceCUs);
+    bool small = tokens * (double)(group / narrow) <= (double)(group == 3 ? kNarrowThree : kNarrowTokens);
+    if (fours) small = small && kv_units * (group / 4) <= kDeviceCUs && (head_dim != 128 || cap < kEvenCapacity);
     if (matrix && group >= kMatrixGroup && !small) {
         const int64_t tiles = (group + 7) / 8;
         const int64_t heads = (group + tiles - 1) / tiles;
@@ -409,8 +415,6 @@ void plan_tiles(DecodePlan& p, int64_t group, int64_t head_dim, int64_t kv_units
     p.gtiles = (int)(group / narrow);
     p.tile_heads = p.gtile;
 }
-
-constexpr int64_t kEvenCapacity = 2048;
 
 // Smallest K+V capacity of a 128-dim unit from which the balanced walk takes a plan of
 // `units` units, in bytes; 0: none.  us per call, other plan -> walk (16/8
