@@ -219,10 +219,19 @@ def test_prefill_write_and_rope_equal_the_python_path(new):
     rope = lambda c, **kw: qk_norm_rope_write_kv(q, k, v, weight, weight, cos, sin, *c, slot_mapping=slots,  # noqa: E731
                                                  validate=False, **kw)
     assert torch.equal(rope(caches[0]), rope(caches[1], out=out))
-    write_kv_cache_slots(*caches[0], slots, k, v, validate=False)
-    write_kv_cache_slots(*caches[1], slots, k, v)
-    assert all(torch.equal(a, b) for a, b in zip(*caches))
+    assert all(torch.equal(a, b) and not torch.equal(a, c) for a, b, c in zip(*caches, (key, value)))
+    native = ext.native_calls()
+    again = [key.clone(), value.clone()]
+    assert native.rope_slots(q, k, v, weight, weight, cos, sin, *again, slots, 1e-6) is not None
+    assert all(torch.equal(a, b) for a, b in zip(again, caches[1]))
+    rows = torch.randn(2, tokens, kv, dim, generator=gen).to(dtype).to(DEV)
+    write_kv_cache_slots(*caches[0], slots, *rows, validate=False)
+    write_kv_cache_slots(*caches[1], slots, *rows)
+    assert all(torch.equal(a, b) and not torch.equal(a, c) for a, b, c in zip(*caches, again))
+    assert native.write_slots(*again, slots, *rows) is True
+    assert all(torch.equal(a, b) for a, b in zip(again, caches[1]))
     args = (out, *caches[0], cu, starts, table, lens, block)
+    assert native.prefill(*args, 0) is not None
     workspace = torch.empty(1 << 24, dtype=torch.uint8, device=DEV)
     assert torch.equal(paged_prefill_attention(*args, validate=False),
                        paged_prefill_attention(*args, validate=False, workspace=workspace))
@@ -240,9 +249,48 @@ def test_dense_and_linear_equal_the_python_path(dim, view):
     result = prefill_attention(q, k, v, query_start=20)
     assert torch.equal(result, prefill_attention(q, k, v, query_start=20, out=out))
     assert result.stride() == (70 * 4 * dim, dim, 4 * dim, 1)
+    assert (ext.native_calls().dense(q, k, v, 20) is not None) == (dim % 8 == 0)
     x, weight = torch.randn(7, 512, generator=gen).bfloat16().to(DEV), torch.randn(64, 512, generator=gen).bfloat16().to(DEV)
     bias = torch.randn(64, generator=gen).bfloat16().to(DEV)
     for b in (None, bias):
         buffer = torch.empty(7, 64, dtype=x.dtype, device=DEV)
         assert torch.equal(linear_rows(x, weight, b), linear_rows(x, weight, b, out=buffer))
+        assert ext.native_calls().linear(x, weight, b) is not None
     assert torch.equal(linear_rows(x[:, ::1][:3], weight), linear_rows(x, weight)[:3])
+
+
+@pytest.mark.gpu
+def test_declines_layouts_of_the_python_path():
+    """Layouts that the kernels cannot read in place, and types they do not take, are
+    left to the Python code: misaligned and oddly strided rows, FP32, other devices'
+    and other types' metadata."""
+    native = ext.native_calls()
+    flat = torch.randn(1 + 70 * 4 * 64, device=DEV).bfloat16()
+    plain, shifted = (flat[i:i + 70 * 4 * 64].view(1, 4, 70, 64) for i in (0, 1))
+    assert native.dense(plain, plain, plain, 0) is not None
+    for q, k, v in ((shifted, plain, plain), (plain, shifted, shifted), (plain, plain, plain.transpose(1, 2).contiguous().transpose(1, 2)),
+                    (plain[..., ::2], plain[..., ::2], plain[..., ::2]), (plain.float(),) * 3):
+        assert native.dense(q, k, v, 0) is None
+    assert native.dense(plain, plain, plain, True) is None and native.dense(plain, plain, plain, 1) is None
+    x, weight = torch.randn(4, 68, device=DEV).bfloat16()[:, :64], torch.randn(32, 64, device=DEV).bfloat16()
+    assert native.linear(x.contiguous(), weight, None) is not None
+    for a, w, b in ((x, weight, None), (x.contiguous().float(), weight.float(), None), (x.contiguous(), weight.t().contiguous().t(), None),
+                    (x.contiguous(), weight, torch.zeros(31, device=DEV).bfloat16()), (x.contiguous()[None], weight, None)):
+        assert native.linear(a, w, b) is None
+    q, key, value, table, lens, block = decode_args(DEV)
+    rows = torch.randn(3, 2, 64, device=DEV).bfloat16()
+    slots = torch.tensor([3, 20, 40], device=DEV)
+    assert native.write_slots(key, value, slots, rows, rows) is True
+    for args in ((key, value, slots.int(), rows, rows), (key, value, slots.cpu(), rows, rows), (key.float(), value.float(), slots, rows.float(), rows.float()),
+                 (key, value, slots, rows.transpose(1, 2).contiguous().transpose(1, 2), rows), (key, value, slots[:2], rows, rows)):
+        assert native.write_slots(*args) is None
+    weight, trig = torch.rand(64, device=DEV).bfloat16(), torch.rand(3, 32, device=DEV).bfloat16()
+    rope = (q, rows, rows, weight, weight, trig, trig, key, value, slots)
+    assert native.rope_slots(*rope, 1e-6) is not None
+    assert native.rope_slots(*rope, 0.0) is None and native.rope_slots(*rope, 1) is None
+    assert native.rope_slots(*rope[:5], trig.float(), trig.float(), *rope[7:], 1e-6) is None
+    cu, starts = torch.tensor([0, 1, 2, 3], device=DEV), lens - 1
+    assert native.prefill(q, key, value, cu, starts, table, lens, block, 0) is not None
+    for args in ((q.float(), key.float(), value.float(), cu, starts, table, lens), (q, key, value, cu.int(), starts, table, lens),
+                 (q, key, value, cu, starts, table.t().contiguous().t(), lens), (q[:, :, ::2], key, value, cu, starts, table, lens)):
+        assert native.prefill(*args, block, 0) is None
