@@ -64,7 +64,7 @@ def test_absent_pages_inside_a_tile(block):
             assert (out[row, h] - p @ value[seen, h // 2]).abs().max().item() <= GATE[dtype]
 
 
-@pytest.mark.parametrize("seqs,heads,kv_heads", [(40, 16, 8), (64, 8, 8), (65, 8, 8)])
+@pytest.mark.parametrize("seqs,heads,kv_heads", [(40, 16, 8), (64, 8, 8), (65, 16, 8)])
 def test_query_blocks_of_many_sequences(seqs, heads, kv_heads):
     """Enough ragged sequences that keys are not split: the work-groups take
     the query blocks by falling key end across sequences (up to 64 of them;
@@ -79,6 +79,8 @@ def test_query_blocks_of_many_sequences(seqs, heads, kv_heads):
     prior[5] = 0
     args = paged_case(new, prior, block, heads, kv_heads, dtype, seed=seqs)
     dev = [a.to(DEV) for a in args]
+    # Keys are not split: nothing to merge.
+    assert paged_prefill_workspace_bytes(seqs, sum(new), heads, kv_heads, 128, block, args[5].shape[1], dtype) == 0
     torch.full_like(dev[0], float("nan"))  # freed at once: the output's storage
     actual = paged_prefill_attention(*dev, block, validate=False).float().cpu()
     expected = paged_oracle.paged_prefill_attention(*args, block, cast=False)
@@ -142,6 +144,32 @@ def test_head_dim_64_dense(batch, tokens, start, view):
         dev = [t.contiguous() for t in dev]
     actual = prefill_attention(*dev, query_start=start).float().cpu()
     expected = paged_oracle.prefill_attention(*[t.transpose(1, 2) for t in (q, k, v)], query_start=start, cast=False)
+    assert (actual - expected).abs().max().item() <= GATE[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("mode", [8, 16, 32, 64, "dense"])
+def test_scores_that_keep_rising(mode, dim, dtype):
+    """Scores rise by 12 binary orders per tile of 64 keys, so that every tile exceeds
+    the reference by more than 2^8: the sums and the output so far are rescaled again
+    and again, and the last keys carry nearly all of the weight."""
+    new, prior, heads, kv_heads, block = 200, 437, 4, 2, mode if mode != "dense" else 16
+    q, kc, vc, cu, starts, tables, lens = paged_case([new], [prior], block, heads, kv_heads, dtype, seed=dim, dim=dim)
+    q.copy_(0.5 + 0.02 * q.float())
+    slope = 12 / 64 / (0.5 * dim ** 0.5 * math.log2(math.e))
+    for i, page in enumerate(tables[0].tolist()):
+        rows = (i * block + torch.arange(block)).float()[:, None, None]
+        kc[page] = (0.02 * kc[page].float() + slope * rows).to(dtype)
+    if mode == "dense":
+        k, v = (c[tables[0]].flatten(0, 1)[:new + prior].transpose(0, 1).unsqueeze(0) for c in (kc, vc))
+        views = (q.transpose(0, 1).unsqueeze(0), k, v)
+        actual = prefill_attention(*[t.to(DEV) for t in views], query_start=prior).float().cpu()
+        expected = paged_oracle.prefill_attention(*views, query_start=prior, cast=False)
+    else:
+        args = [q, kc, vc, cu, starts, tables, lens]
+        actual = paged_prefill_attention(*[a.to(DEV) for a in args], block, chunk_tokens=1024).float().cpu()
+        expected = paged_oracle.paged_prefill_attention(*args, block, cast=False)
     assert (actual - expected).abs().max().item() <= GATE[dtype]
 
 
