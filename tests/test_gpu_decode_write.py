@@ -146,11 +146,26 @@ def test_balanced_walk(rope, head_dim):
 
 @pytest.mark.parametrize("q_heads,kv_heads", [(8, 8), (32, 8), (64, 8), (28, 4)])
 def test_gqa_tiles(q_heads, kv_heads):
-    """Group 1, 4, 8 (two 4-head tiles, both writing the same rows) and 7."""
+    """Group 1, 4, 8 and 7: one tile each."""
     step = make_step(6, q_heads, kv_heads, 128, 32, [5, 300, 64, 1, 129, 700], torch.float16, seed=q_heads)
     print(f"decode write GQA {q_heads}/{kv_heads}", flush=True)
     check_equal(step, 32, True)
     check_equal(step, 32, False)
+
+
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("head_dim,q_heads,kv_heads", [
+    (64, 14, 2), (64, 36, 4), (64, 48, 4), (64, 68, 4), (128, 36, 4), (128, 48, 4), (128, 68, 4),
+])
+def test_several_matrix_tiles(rope, head_dim, q_heads, kv_heads):
+    """Groups of 7, 9, 12 and 17 in tiles of 7, 5 + 4, 6 + 6 and 6 + 6 + 5 heads: every
+    tile's work-group writes the same row, and the last tile rotates fewer heads.
+    Over 2112 tokens: partitions by the lengths (128 dims) or by the capacity, the
+    walk, and forced partitions."""
+    step = make_step(6, q_heads, kv_heads, head_dim, 16, [5, 300, 64, 1, 129, 2100], torch.bfloat16, seed=q_heads)
+    for partition in (0, -1, 320):
+        print(f"decode write tiles {q_heads}/{kv_heads} D={head_dim} rope={rope} partition {partition}", flush=True)
+        check_equal(step, 16, rope, partition_tokens=partition)
 
 
 def test_strided_fused_qkv_rows():
