@@ -347,10 +347,11 @@ struct DecodePlan {
 };
 
 
-// Query heads per kv head from which tiles run on the matrix cores.  A tile of
-// up to 4 heads costs them the same whatever the number; with 2 heads the
-// dot-product kernel is ahead (32 sequences of 2048, fp16: 44.6 us against
-// 46.3), with 4 the matrix cores are (48.4 -> 46.3).
+// Query heads per kv head from which tiles run on the matrix cores (small calls
+// apart, see plan_tiles).  A tile of up to 4 heads costs them the same whatever
+// the number; with 2 heads the dot-product kernel is ahead at one unit per CU (32
+// sequences of 2048, fp16: 44.6 us against 46.3) and make_decode_plan says where it
+// is not, with 4 the matrix cores are (48.4 -> 46.3).
 constexpr int64_t kMatrixGroup = 3;
 constexpr int64_t kStreamBytes = int64_t(64) << 20;  // K+V bytes within capacity above which loads stream
 
@@ -490,6 +491,8 @@ int64_t split_partition(int64_t cap, int64_t units, int64_t step) {
 // * ctx 256: level up to 64 units; whole ahead from 128 units.
 // * ctx 512: split at 64 ahead up to 64 units (1 unit 7.96 -> 6.87, 64 units
 //   8.18 -> 7.82); whole ahead from 128 units (128 units 9.01 vs 9.98).
+// (All of these on the dot-product loop.  Splits of pairs and of wider groups at 64
+// and 128 dims have since run the matrix cores' loop, with the same lines.)
 // * ctx 1024-4096 with 8-64 units: the best partition gives about 512
 //   work-groups (1024 keys x 8 units: 256-key parts 9.69, 64-key 7.30; 1024
 //   x 64: 11.61 -> 9.93 at 128; 2048 x 32: 11.56 -> 10.48 at 128); the

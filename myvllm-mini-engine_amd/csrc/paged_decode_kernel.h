@@ -29,8 +29,9 @@
 // that later reads that position (in every work-group whose token range
 // holds it: identical bytes from each G-tile), so no barrier is needed.
 //
-// Query groups of three or more heads at head_dim 64 and 128 run on the
-// matrix cores (see matrix_states); what follows describes the others.
+// At head_dim 64 and 128 query groups of three or more heads run on the matrix
+// cores (see matrix_states) except in small calls (plan_tiles), and pairs of heads
+// where the plan finds them ahead there; what follows describes the others.
 //
 // Scores: packed dot2 (fp16/bf16 products, fp32 accumulation) on the lane's
 // 8 elements, then a DPP reduction across the LPT lanes of the token.
@@ -741,16 +742,16 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
             }
         } else {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            u32x4 w = {0u, 0u, 0u, 0u};
-            if (PRO && a.prologue == 2) {
-                if (chunk_ok) w = *reinterpret_cast<const u32x4*>(&sm_q[PRO ? wave : 0][PRO ? g : 0][PRO ? 8 * c : 0]);
-            } else if (chunk_ok)
-                w = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.query) +
-                                                    ((int64_t)b * a.q_heads + h0 + g) * D + 8 * c);
+            for (int g = 0; g < G; ++g) {
+                u32x4 w = {0u, 0u, 0u, 0u};
+                if (PRO && a.prologue == 2) {
+                    if (chunk_ok) w = *reinterpret_cast<const u32x4*>(&sm_q[PRO ? wave : 0][PRO ? g : 0][PRO ? 8 * c : 0]);
+                } else if (chunk_ok)
+                    w = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.query) +
+                                                        ((int64_t)b * a.q_heads + h0 + g) * D + 8 * c);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) q[g][i] = w[i];
-        }
+                for (int i = 0; i < 4; ++i) q[g][i] = w[i];
+            }
         }
 
         // Running softmax state.  Matrix tiles: macc[t][e][i] is the sum of
@@ -868,96 +869,95 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                 }
             }
         } else {
-        for (; it < end; it += kStep) {
-            u32x4 kk[L], vv[L];
-            bool ok[L];
-            // The owner's store of the new row completes before the row is read.
-            if constexpr (PRO)
-                if (owner && it <= pos && pos < it + S::kTpi) __builtin_amdgcn_s_waitcnt(0);
-            if constexpr (PAGE_UNIFORM) {
-                const int64_t page = page_next[0];
-                page_next[0] = page_of(it + kStep);
-                const bool page_ok = page >= 0 && page < a.num_blocks;
-#pragma unroll
-                for (int u = 0; u < L; ++u) {
-                    ok[u] = page_ok && it + u * S::kTpl + tl < end;
-                    kk[u] = vv[u] = u32x4{0u, 0u, 0u, 0u};
-                }
-                if (page_ok) {  // wave-uniform
-                    const int64_t base = (page * a.block_size + page_row(a, it)) * (int64_t)row_bytes;
-                    const uint8_t* kp = static_cast<const uint8_t*>(a.key_cache) + base;
-                    const uint8_t* vp = static_cast<const uint8_t*>(a.value_cache) + base;
+            for (; it < end; it += kStep) {
+                u32x4 kk[L], vv[L];
+                bool ok[L];
+                // The owner's store of the new row completes before the row is read.
+                if constexpr (PRO)
+                    if (owner && it <= pos && pos < it + S::kTpi) __builtin_amdgcn_s_waitcnt(0);
+                if constexpr (PAGE_UNIFORM) {
+                    const int64_t page = page_next[0];
+                    page_next[0] = page_of(it + kStep);
+                    const bool page_ok = page >= 0 && page < a.num_blocks;
 #pragma unroll
                     for (int u = 0; u < L; ++u) {
-                        // In-page rows past the context are loaded (in bounds) and zeroed below.
-                        if constexpr (S::kChunks == S::kLpt) {
-                            kk[u] = kv_load<STREAM>(kp + lane_off[u]);
-                            vv[u] = kv_load<STREAM>(vp + lane_off[u]);
-                        } else if (chunk_ok) {
-                            kk[u] = kv_load<STREAM>(kp + lane_off[u]);
-                            vv[u] = kv_load<STREAM>(vp + lane_off[u]);
+                        ok[u] = page_ok && it + u * S::kTpl + tl < end;
+                        kk[u] = vv[u] = u32x4{0u, 0u, 0u, 0u};
+                    }
+                    if (page_ok) {  // wave-uniform
+                        const int64_t base = (page * a.block_size + page_row(a, it)) * (int64_t)row_bytes;
+                        const uint8_t* kp = static_cast<const uint8_t*>(a.key_cache) + base;
+                        const uint8_t* vp = static_cast<const uint8_t*>(a.value_cache) + base;
+#pragma unroll
+                        for (int u = 0; u < L; ++u) {
+                            // In-page rows past the context are loaded (in bounds) and zeroed below.
+                            if constexpr (S::kChunks == S::kLpt) {
+                                kk[u] = kv_load<STREAM>(kp + lane_off[u]);
+                                vv[u] = kv_load<STREAM>(vp + lane_off[u]);
+                            } else if (chunk_ok) {
+                                kk[u] = kv_load<STREAM>(kp + lane_off[u]);
+                                vv[u] = kv_load<STREAM>(vp + lane_off[u]);
+                            }
+                        }
+#pragma unroll
+                        for (int u = 0; u < L; ++u)
+                            if (!ok[u]) vv[u] = u32x4{0u, 0u, 0u, 0u};  // 0 * (stale NaN) must not reach acc
+                    }
+                } else {
+#pragma unroll
+                    for (int u = 0; u < L; ++u) {
+                        const int t = it + u * S::kTpl + tl;
+                        int64_t page = -1;
+                        const int idx = lane_page(a, t);
+                        if (t < end) page = table[idx];
+                        ok[u] = page >= 0 && page < a.num_blocks;
+                        const int64_t off = page * page_elems + lane_row(a, t, idx) * row_elems;
+                        kk[u] = vv[u] = u32x4{0u, 0u, 0u, 0u};
+                        if (ok[u] && chunk_ok) {
+                            kk[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(kbase + off));
+                            vv[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(vbase + off));
                         }
                     }
-#pragma unroll
-                    for (int u = 0; u < L; ++u)
-                        if (!ok[u]) vv[u] = u32x4{0u, 0u, 0u, 0u};  // 0 * (stale NaN) must not reach acc
                 }
-            } else {
+
 #pragma unroll
-                for (int u = 0; u < L; ++u) {
-                    const int t = it + u * S::kTpl + tl;
-                    int64_t page = -1;
-                    const int idx = lane_page(a, t);
-                    if (t < end) page = table[idx];
-                    ok[u] = page >= 0 && page < a.num_blocks;
-                    const int64_t off = page * page_elems + lane_row(a, t, idx) * row_elems;
-                    kk[u] = vv[u] = u32x4{0u, 0u, 0u, 0u};
-                    if (ok[u] && chunk_ok) {
-                        kk[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(kbase + off));
-                        vv[u] = kv_load<STREAM>(reinterpret_cast<const uint8_t*>(vbase + off));
+                for (int g = 0; g < G; ++g) {
+                    float s[L];
+#pragma unroll
+                    for (int u = 0; u < L; ++u) {
+                        float d = 0.f;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) d = T::dot2(kk[u][i], q[g][i], d);
+                        d = group_sum<S::kLpt>(d) * a.scale_log2;
+                        s[u] = ok[u] ? d : kNegInf;
+                    }
+                    float mx = s[0];
+#pragma unroll
+                    for (int u = 1; u < L; ++u) mx = fmaxf(mx, s[u]);
+                    const float mn = fmaxf(m[g], mx);
+                    const float ref = mn == kNegInf ? 0.f : mn;
+                    const float alpha = fast_exp2(m[g] - ref);
+                    float p[L];
+                    float psum = 0.f;
+#pragma unroll
+                    for (int u = 0; u < L; ++u) {
+                        p[u] = fast_exp2(s[u] - ref);
+                        psum += p[u];
+                    }
+                    l[g] = l[g] * alpha + psum;
+                    m[g] = mn;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) acc[g][i] *= alpha;
+#pragma unroll
+                    for (int u = 0; u < L; ++u) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            acc[g][2 * i] = fmaf(p[u], T::lo(vv[u][i]), acc[g][2 * i]);
+                            acc[g][2 * i + 1] = fmaf(p[u], T::hi(vv[u][i]), acc[g][2 * i + 1]);
+                        }
                     }
                 }
             }
-
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float s[L];
-#pragma unroll
-                for (int u = 0; u < L; ++u) {
-                    float d = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) d = T::dot2(kk[u][i], q[g][i], d);
-                    d = group_sum<S::kLpt>(d) * a.scale_log2;
-                    s[u] = ok[u] ? d : kNegInf;
-                }
-                float mx = s[0];
-#pragma unroll
-                for (int u = 1; u < L; ++u) mx = fmaxf(mx, s[u]);
-                const float mn = fmaxf(m[g], mx);
-                const float ref = mn == kNegInf ? 0.f : mn;
-                const float alpha = fast_exp2(m[g] - ref);
-                float p[L];
-                float psum = 0.f;
-#pragma unroll
-                for (int u = 0; u < L; ++u) {
-                    p[u] = fast_exp2(s[u] - ref);
-                    psum += p[u];
-                }
-                l[g] = l[g] * alpha + psum;
-                m[g] = mn;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc[g][i] *= alpha;
-#pragma unroll
-                for (int u = 0; u < L; ++u) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        acc[g][2 * i] = fmaf(p[u], T::lo(vv[u][i]), acc[g][2 * i]);
-                        acc[g][2 * i + 1] = fmaf(p[u], T::hi(vv[u][i]), acc[g][2 * i + 1]);
-                    }
-                }
-            }
-        }
-
         }
 
         // (Exchanging every sum with every partner lane through ds_bpermute,
@@ -997,37 +997,37 @@ __global__ __launch_bounds__(NW * kWave, (min_waves<D, G, FLAT>())) void paged_d
                     }
             }
         } else {
-        // The same for the dot-product tiles: token slots 2, 4 and 8 lanes
-        // apart are added in place, those 16 and 32 apart by exchanges, after
-        // which a lane keeps kKeep of its chunk's 8 dims, from keep0 on.
+            // The same for the dot-product tiles: token slots 2, 4 and 8 lanes
+            // apart are added in place, those 16 and 32 apart by exchanges, after
+            // which a lane keeps kKeep of its chunk's 8 dims, from keep0 on.
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float mn = m[g];
-            if constexpr (S::kLpt <= 2) mn = fmaxf(mn, dpp<kDppQuadSwap2>(mn));
-            if constexpr (S::kLpt <= 4) mn = fmaxf(mn, lane_xor4(mn));
-            if constexpr (S::kLpt <= 8) mn = fmaxf(mn, dpp<kDppRowRor8>(mn));
-            if constexpr (S::kLpt <= 16) mn = row4_max(mn);
-            else if constexpr (S::kLpt == 32) mn = pair32_max(mn);
-            const float f = fast_exp2(m[g] - (mn == kNegInf ? 0.f : mn));
-            m[g] = mn;
-            auto within = [](float v) __attribute__((always_inline)) -> float {
-                if constexpr (S::kLpt <= 2) v += dpp<kDppQuadSwap2>(v);
-                if constexpr (S::kLpt <= 4) v += lane_xor4(v);
-                if constexpr (S::kLpt <= 8) v += dpp<kDppRowRor8>(v);
-                return v;
-            };
-            l[g] = within(l[g] * f);
-            if constexpr (S::kLpt <= 16) l[g] = row4_sum(l[g]);
-            else if constexpr (S::kLpt == 32) l[g] = swap32_add(l[g], l[g]);
+            for (int g = 0; g < G; ++g) {
+                float mn = m[g];
+                if constexpr (S::kLpt <= 2) mn = fmaxf(mn, dpp<kDppQuadSwap2>(mn));
+                if constexpr (S::kLpt <= 4) mn = fmaxf(mn, lane_xor4(mn));
+                if constexpr (S::kLpt <= 8) mn = fmaxf(mn, dpp<kDppRowRor8>(mn));
+                if constexpr (S::kLpt <= 16) mn = row4_max(mn);
+                else if constexpr (S::kLpt == 32) mn = pair32_max(mn);
+                const float f = fast_exp2(m[g] - (mn == kNegInf ? 0.f : mn));
+                m[g] = mn;
+                auto within = [](float v) __attribute__((always_inline)) -> float {
+                    if constexpr (S::kLpt <= 2) v += dpp<kDppQuadSwap2>(v);
+                    if constexpr (S::kLpt <= 4) v += lane_xor4(v);
+                    if constexpr (S::kLpt <= 8) v += dpp<kDppRowRor8>(v);
+                    return v;
+                };
+                l[g] = within(l[g] * f);
+                if constexpr (S::kLpt <= 16) l[g] = row4_sum(l[g]);
+                else if constexpr (S::kLpt == 32) l[g] = swap32_add(l[g], l[g]);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[g][i] = within(acc[g][i] * f);
-            if constexpr (S::kLpt <= 32)
+                for (int i = 0; i < 8; ++i) acc[g][i] = within(acc[g][i] * f);
+                if constexpr (S::kLpt <= 32)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[g][i] = swap32_add(acc[g][i], acc[g][i + 4]);
-            if constexpr (S::kLpt <= 16)
+                    for (int i = 0; i < 4; ++i) acc[g][i] = swap32_add(acc[g][i], acc[g][i + 4]);
+                if constexpr (S::kLpt <= 16)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) acc[g][i] = swap16_add(acc[g][i], acc[g][i + 2]);
-        }
+                    for (int i = 0; i < 2; ++i) acc[g][i] = swap16_add(acc[g][i], acc[g][i + 2]);
+            }
         }
         constexpr int kKeep = S::kLpt <= 16 ? 2 : S::kLpt == 32 ? 4 : 8;
         const int keep0 = S::kLpt <= 16 ? 4 * (lane >> 5) + 2 * (lg & 1) : S::kLpt == 32 ? 4 * (lane >> 5) : 0;

@@ -43,13 +43,15 @@
 //   The online softmax keeps a per-row reference m and computes
 //   p = 2^(s*scale - m) without a row maximum; the sum of a lane's 8
 //   probabilities of a half tile (which any probability above 2^8, inf or
-//   NaN pushes past 256) triggers the exact step: the row maximum across the
+//   NaN pushes past 256; on pages of at least a tile at 128 dims the largest
+//   of them, rounded to 16 bits) triggers the exact step: the row maximum across the
 //   four lanes (permlane swaps), a rescale of the accumulators, and new
 //   probabilities.  It runs when a row sees its first key and when a row's
 //   scores grow by several binary orders, so the accumulators are rescaled
 //   rarely and probabilities stay below 2^8.  Tiles that are complete and
 //   entirely below the causal diagonal skip masking.  Accumulation, softmax
-//   and normalisation are fp32.
+//   and normalisation are fp32; the row sums are of fp32 probabilities, except on
+//   pages of at least a tile at 128 dims (of the 16-bit ones, on the matrix core).
 //
 // Generic path (any D <= 1024, any G): one wave per (query row, head),
 // online softmax over 64-key tiles, fp32 throughout.
@@ -74,8 +76,8 @@ constexpr int kTileBytes = 16384;         // one K (or V) tile in LDS, every til
 constexpr int kPfMaxKeys = 64;            // keys per tile, largest tile shape
 
 // Tile shape of the MFMA kernel by padded head dim: 64 (head_dim 64 on
-// power-of-two pages), 128 (head_dim 128 and other narrower multiples of 8)
-// or 256.  A tile is 16 KiB of K (and of V) in LDS, 8 at 64; at 256 a wave
+// power-of-two pages of at least 8 tokens and in dense mode), 128 (head_dim 128
+// and other narrower multiples of 8) or 256.  A tile is 16 KiB of K (and of V) in LDS, 8 at 64; at 256 a wave
 // holds one 16-row block (the accumulators of 256 dims fill the registers two
 // blocks used) and a tile has 32 keys.
 template <int HD>
@@ -708,9 +710,10 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
     // Swizzled LDS offsets this lane reads (independent of the tile):
     // K chunk 4*dc + lg of row 16*kt + li, and the transposing V reads of
     // rows 32*c + 4*lg + li/4 (+16), dims 16*dt + 4*(li%4) .. +4.  K rows
-    // store global chunk c in slot c ^ (row & 15); V rows in slot
-    // c ^ (2*row & 15), so that the 16 lanes of a transposing read (4 rows x
-    // 2 adjacent chunks) hit 8 different 16-byte bank groups.
+    // store global chunk c in slot c ^ k_swizzle(row); V rows in slot c ^
+    // v_swizzle(row) (row & 15 and 2*row & 15 at 128 and 256 dims), so that the
+    // 16 lanes of a transposing read (4 rows x 2 adjacent chunks) hit 8
+    // different 16-byte bank groups.
     int koff[SH::kDc];
 #pragma unroll
     for (int dc = 0; dc < SH::kDc; ++dc) koff[dc] = li * SH::kRowBytes + 16 * ((4 * dc + lg) ^ SH::k_swizzle(li));
@@ -720,10 +723,12 @@ __device__ __attribute__((always_inline)) void prefill_item(const PrefillArgs& a
     for (int dt = 0; dt < SH::kDt; ++dt)
         voff[dt] = vrow * SH::kRowBytes + 16 * ((2 * dt + ((li & 3) >> 1)) ^ SH::v_swizzle(vrow)) + 8 * (li & 1);
 
-    // Copy plan: a tile's K (and V) is 16 instructions of 1 KiB; wave w issues
-    // instructions j = SH::kIpw*w + i, each covering key rows 4j..4j+3 (lane ->
-    // row 4j + lane/16, LDS slot lane%16 = global chunk (lane%16)^(row&15) for
-    // K, (lane%16)^(2*row&15) for V).
+    // Copy plan: a tile's K (and V) is SH::kIpw instructions of 1 KiB per wave
+    // (16 in all; 8 at the 64 shape); wave w issues instructions j = SH::kIpw*w +
+    // i, each covering SH::kRowsPerInst key rows from kRowsPerInst*j on (4 at the
+    // 128 shape, 8 at 64, 2 at 256): lane -> row kRowsPerInst*j + lane/kChunks, LDS
+    // slot lane%kChunks = global chunk slot ^ k_swizzle(row) for K, slot ^
+    // v_swizzle(row) for V.
     // Paged mode: the cache layout [pages, block_size, kv_heads, hd] (the
     // strides follow from the shapes, nothing more is held in registers).
     const int64_t row_bytes_g = DENSE ? a.kv_row_bytes : (int64_t)a.kv_heads * hd * 2;
